@@ -82,7 +82,7 @@ STEP_TASK = np.dtype([
 MUON_TASK = np.dtype([
     ("grad", np.uint64), ("m_codebook", np.uint64), ("m_magnitude", np.uint64), ("out", np.uint64),
     ("numel", np.int64), ("block", np.int64), ("grad_dtype", np.int32), ("state_dtype", np.int32),
-    ("momentum", np.float64), ("nesterov", np.int32), ("pad", np.int32),
+    ("momentum", np.float64), ("nesterov", np.int32), ("out_bf16", np.int32),
 ])
 MUON_APPLY_TASK = np.dtype([
     ("p", np.uint64), ("update", np.uint64), ("numel", np.int64), ("param_dtype", np.int32),

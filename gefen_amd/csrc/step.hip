@@ -1148,7 +1148,8 @@ int make_muon_task(const gefen_muon_task& in, PendingMuon& out) {
         return fail_inval("Expected beta1 to be in [0, 1), got %g", in.momentum);
     if (n > 0 && (!in.grad || !in.m_codebook || !in.m_magnitude || !in.out)) return fail_inval("null tensor pointer");
     const int dsz = dtype_size(in.grad_dtype);
-    const int W = pick_width(dsz, rowlen, {in.grad, in.out}, 1, in.m_codebook, 0, nullptr);
+    int W = pick_width(dsz, rowlen, {in.grad, in.out_bf16 ? in.grad : in.out}, 1, in.m_codebook, 0, nullptr);
+    if (in.out_bf16 && !aligned(in.out, 2 * W)) W = 1;
     const int64_t nvec = rowlen / W;
     // rows of at most 32 vectors take half the lanes with twice the vectors per
     // lane (measured 6% faster on the Qwen3-1.7B momentum, mostly period-one rows)
@@ -1195,6 +1196,7 @@ int make_muon_task(const gefen_muon_task& in, PendingMuon& out) {
     t.alpha = round_host(alpha, in.grad_dtype);
     t.tiny = round_host(tiny, in.state_dtype);
     t.nesterov = in.nesterov ? 1 : 0;
+    t.out_bf16 = in.out_bf16 && in.grad_dtype != GEFEN_BF16 ? 1 : 0;
     t.nwg = task_wgs(k, t.nrows, l2, 4, kMuonIter);
     if (t.nwg < 0) return fail_inval("tensor of %lld elements is too large for one launch", (long long)n);
     out.key = k;

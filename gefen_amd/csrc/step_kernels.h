@@ -645,7 +645,8 @@ struct MuonTask {
     float mom;     // f32(momentum)
     float alpha;   // add_ alpha: f32(1 - momentum), rounded to D for reduced dtypes
     float tiny;    // finfo(D).tiny rounded to S
-    int32_t nesterov;
+    int32_t nesterov : 16;
+    int32_t out_bf16 : 16;  // out is bf16 (D wider or half): the blend rounded to D, then to bf16
     int32_t nwg;
     double* sumsq;  // if set: GEFEN_SUMSQ_SLOTS accumulators (16 doubles apart) of the sum of squares of the output
 };
@@ -765,6 +766,7 @@ __global__ __launch_bounds__(kThreads) void k_muon(const MuonBatch B) {
         const D* __restrict__ g = static_cast<const D*>(T.g) + ub;
         uint8_t* __restrict__ idx = T.idx + ub;
         D* __restrict__ out = static_cast<D*>(T.out) + ub;
+        bf16_t* __restrict__ out16 = static_cast<bf16_t*>(T.out) + ub;
         S* __restrict__ mag = static_cast<S*>(T.mag) + row0;
         const uint32_t base = (uint32_t)rsub * (uint32_t)T.rowlen;
         Vec<D, W> gv[R];
@@ -875,6 +877,7 @@ __global__ __launch_bounds__(kThreads) void k_muon(const MuonBatch B) {
         for (int j = 0; j < R; ++j) {
             Vec<uint8_t, W> io;
             Vec<D, W> oo;
+            Vec<bf16_t, W> ob;
             float sqj = 0.0f;
             int kw[W];
             if (kNb && all_fast) {
@@ -944,7 +947,11 @@ __global__ __launch_bounds__(kThreads) void k_muon(const MuonBatch B) {
                     io.v[w] = (uint8_t)k;
                     const float a = TAB ? otab[k] : out_base(k);
                     oo.v[w] = from_f32<D>(muon_blend<D>(a, to_f32(gv[j].v[w]), T));
-                    const float o = to_f32(oo.v[w]);
+                    float o = to_f32(oo.v[w]);
+                    if (!kNb && T.out_bf16) {
+                        ob.v[w] = from_f32<bf16_t>(o);
+                        o = to_f32(ob.v[w]);
+                    }
                     sqj = __builtin_fmaf(o, o, sqj);
                 }
             }
@@ -952,7 +959,8 @@ __global__ __launch_bounds__(kThreads) void k_muon(const MuonBatch B) {
             if (active && v < T.nvec) {
                 const uint32_t e = base + (uint32_t)(v * W);
                 sstore<uint8_t, W>(idx, e, io);
-                sstore<D, W>(out, e, oo);
+                if (!kNb && T.out_bf16) sstore<bf16_t, W>(out16, e, ob);
+                else sstore<D, W>(out, e, oo);
                 sq += sqj;
             }
         }
@@ -1007,8 +1015,14 @@ __global__ __launch_bounds__(kThreads) void k_muon_long(const MuonBatch B) {
         idx[base + j] = (uint8_t)k;
         const float q = round_to<D>(L.cbd[k] * ms);
         const D o = from_f32<D>(muon_out<D, S>(q, gf, T));
-        out[base + j] = o;
-        const float of = to_f32(o);
+        float of = to_f32(o);
+        if (T.out_bf16) {
+            const bf16_t o16 = from_f32<bf16_t>(of);
+            static_cast<bf16_t*>(T.out)[base + j] = o16;
+            of = to_f32(o16);
+        } else {
+            out[base + j] = o;
+        }
         sq = __builtin_fmaf(of, of, sq);
     }
     if (T.sumsq) add_sumsq(sq, T.sumsq, row);

@@ -178,8 +178,8 @@ class GefenMuon(Gefen):
         where = {}
         bufs = {}
         for key, idx in stacks.items():
-            rows, cols, dtype = key[0], key[1], key[2]
-            bufs[key] = torch.empty(len(idx), rows, cols, dtype=dtype, device=items[idx[0]][3].device)
+            rows, cols = key[0], key[1]
+            bufs[key] = torch.empty(len(idx), rows, cols, dtype=torch.bfloat16, device=items[idx[0]][3].device)
             for slot, i in enumerate(idx):
                 where[i] = (key, slot)
         outs = []
@@ -208,13 +208,17 @@ class GefenMuon(Gefen):
             t["state_dtype"] = _DTYPE_CODE[st["m_magnitude"].dtype]
             t["momentum"] = group["momentum"]
             t["nesterov"] = 1 if group["nesterov"] else 0
+            t["out_bf16"] = 1 if i in where else 0
         dev = items[0][3].device
         lib = _lib.load()
-        # the sums of squares of the written blends of bf16 stacks, for the
-        # Newton-Schulz normalisation (gathered by the momentum kernels)
+        # the sums of squares of the bf16 blends written into the stacks, for the
+        # Newton-Schulz normalisation (gathered by the momentum kernels).  The kernels
+        # write bf16 stacks for every gradient dtype: a float32 stack, its conversion
+        # and a pass for the norms cost 12 B per element more (twelve GPT-2 layers'
+        # float32 matrices: 3.38 -> 3.14 ms per step)
         sumsq = torch.empty(len(items) * _SUMSQ_STRIDE, dtype=torch.float64, device=dev)
         sum_index = {key: torch.tensor(idx, dtype=torch.int32, device=dev)
-                     for key, idx in stacks.items() if key[2] == torch.bfloat16}
+                     for key, idx in stacks.items()}
         with torch.cuda.device(dev):
             rc = lib.gefen_muon_tasks_sumsq(tasks.ctypes.data, len(items), tables.data_ptr(), sumsq.data_ptr(),
                                             torch.cuda.current_stream(dev).cuda_stream)
@@ -227,11 +231,9 @@ class GefenMuon(Gefen):
             for key, idx in stacks.items():
                 coeffs, steps, eps = key[3], key[4], key[5]
                 _check_ns_args(coeffs, steps)
-                x = bufs[key] if key[2] == torch.bfloat16 else bufs[key].bfloat16()
                 works[key] = {}
-                si = sum_index.get(key)
-                res = newton_schulz_batched(x, coeffs, steps, eps, work=works[key],
-                                            sumsq=sumsq if si is not None else None, index=si)
+                res = newton_schulz_batched(bufs[key], coeffs, steps, eps, work=works[key], sumsq=sumsq,
+                                            index=sum_index[key])
                 for slot, i in enumerate(idx):
                     updates[i] = res[slot]
         apply = np.zeros(len(items), dtype=_lib.MUON_APPLY_TASK)
@@ -283,7 +285,7 @@ class GefenMuon(Gefen):
             # the one-matrix Newton-Schulz in every run
             solo = [(i, outs[i], tuple(items[i][0]["ns_coefficients"]), items[i][0]["ns_steps"], items[i][0]["eps"])
                     for i in range(len(items)) if i not in where]
-            self._plan = _MuonPlan(self, items, tasks, apply, [(key, idx, bufs[key], works[key], sum_index.get(key))
+            self._plan = _MuonPlan(self, items, tasks, apply, [(key, idx, bufs[key], works[key], sum_index[key])
                                                                  for key, idx in stacks.items()], dev, sumsq, solo)
         del keep
 
@@ -403,21 +405,16 @@ class _MuonPlan:
             stream = torch.cuda.current_stream(self.device).cuda_stream
             _lib.check(lib.gefen_muon_tasks_sumsq(self.mtasks.ctypes.data, len(self.mtasks), tables.data_ptr(),
                                                   self.sumsq.data_ptr(), stream), "gefen_muon_tasks_sumsq")
-            # newton_schulz_batched may return its input (a bf16 copy of a non-bf16
-            # stack, with an even or zero step count): every input and result stays
-            # referenced here until the launch that reads them is enqueued
+            # every result stays referenced here until the launch that reads it is enqueued
             keep = []
             for (key, idx, buf, work, sum_index), fuse in zip(self.stacks, self.fuse):
                 coeffs, steps, eps = key[3], key[4], key[5]
-                x = buf if key[2] == torch.bfloat16 else buf.bfloat16()
-                sums = self.sumsq if sum_index is not None else None
                 if fuse:  # the last product updates the parameters (gefen_muon.py:47, 325-329)
-                    newton_schulz_batched(x, coeffs, steps, eps, work=work, sumsq=sums, index=sum_index,
+                    newton_schulz_batched(buf, coeffs, steps, eps, work=work, sumsq=self.sumsq, index=sum_index,
                                           apply=self.apply[idx])
-                    keep.append(x)
                     continue
-                res = newton_schulz_batched(x, coeffs, steps, eps, work=work, sumsq=sums, index=sum_index)
-                keep.append((x, res))
+                res = newton_schulz_batched(buf, coeffs, steps, eps, work=work, sumsq=self.sumsq, index=sum_index)
+                keep.append(res)
                 slot_bytes = res[0].numel() * res.element_size()
                 self.apply["update"][idx] = res.data_ptr() + np.arange(len(idx), dtype=np.uint64) * slot_bytes
             for i, out, coeffs, steps, eps in self.solo:

@@ -193,7 +193,9 @@ typedef struct gefen_muon_task {
     int32_t state_dtype;
     double momentum;
     int32_t nesterov;
-    int32_t pad;
+    int32_t out_bf16;           /* 1: out holds the blend rounded to bf16 (the Newton-Schulz
+                                   input, gefen_muon.py:33) instead of grad dtype values;
+                                   sums of squares are then those of the bf16 values */
 } gefen_muon_task;
 
 int gefen_muon_tasks(const gefen_muon_task* tasks, int ntasks, const void* tables,
