@@ -93,6 +93,11 @@ __device__ __forceinline__ float max_skip_nan(float a, float b) { return b > a ?
 template <typename T, int W>
 struct alignas(sizeof(T) * W) Vec { T v[W]; };
 
+// W consecutive elements at the alignment of one: the backend moves it with the
+// same wide accesses (global memory takes any alignment on gfx950).
+template <typename T, int W>
+struct AnyVec { T v[W]; };
+
 template <typename T, int W>
 __device__ __forceinline__ Vec<T, W> vload(const T* base, int64_t elem) {
     return *reinterpret_cast<const Vec<T, W>*>(base + elem);

@@ -21,6 +21,7 @@
 
 #include "capi_internal.h"
 #include "common.h"
+#include "ns_gemm.h"
 
 namespace gefen {
 namespace ns {
@@ -188,99 +189,106 @@ __global__ __launch_bounds__(NT) void k_gemm(const uint16_t* __restrict__ A, int
 }
 
 // ---------------------------------------------------------------------------
-// Large-tile batched GEMM for the Newton-Schulz products, all in "A B^T" form:
+// Tiled batched GEMM for the Newton-Schulz products, all in "A B^T" form:
 //
 //   C_b = alpha * A_b @ B_b^T + beta * D_b     (bf16 out, one rounding)
 //
 // A_b [M, K] and B_b [N, K] are row-major, so both operands are K-contiguous
 // (the Gram matrix X X^T, A A with A symmetric, and B X with X^T kept beside X).
-// A 512-thread workgroup owns a 256x256 tile; its eight waves (2 x 4) each own
-// 128x64 as 4x2 v_mfma_f32_32x32x16_bf16 tiles (128 fp32 accumulators per
-// lane).  K moves TK (64) at a time through one register stage and two LDS
-// stages (global loads run two steps ahead of the MFMAs that use them).  Symmetric outputs (X X^T, b A + c A A)
-// compute only the tiles on and above the diagonal and mirror them; CT
-// (optional) receives C^T.  Each XCD takes a contiguous run of tiles, in bands
-// of kGroupM tile rows, so workgroups that share operand panels share an L2.
-// M and N must be multiples of 256, K a multiple of TK, every row 16-byte
-// aligned; other shapes take k_gemm.
+// A workgroup owns a T x T tile; its waves each own (32 WI) x (32 WJ) of it as
+// WI x WJ v_mfma_f32_32x32x16_bf16 tiles.  K moves TK (64) at a time through one
+// register stage and two LDS stages (global loads run two steps ahead of the
+// MFMAs that use them).  Symmetric outputs (X X^T, b A + c A A) compute only the
+// tiles on and above the diagonal and mirror them; CT (optional) receives C^T.
+// Each XCD takes a contiguous run of tiles, in bands of kGroupM tile rows, so
+// workgroups that share operand panels share an L2.  M and N must be multiples
+// of T, K a multiple of TK, every row 16-byte aligned; other shapes take k_gemm.
+//
+// Two tiles (TileCfg): 256 x 256 by eight waves of 128 x 64 (one workgroup per
+// CU, the least operand traffic per flop), and 128 x 128 by four waves of 64 x 64
+// (two workgroups per CU), which fills the chip when a launch has few tiles.
+// Both add the products of K in the same MFMA order, so their results are
+// bit-identical.  product_us() chooses.
 #ifndef GEFEN_NS_TK
 #define GEFEN_NS_TK 64
 #endif
-constexpr int TM = 256, TN = 256, TK = GEFEN_NS_TK;
+constexpr int TK = GEFEN_NS_TK;
 constexpr int TLD = TK + 8;  // padded LDS row (bf16 elements)
 constexpr int CPR = TK / 8;  // 16-byte chunks per tile row
-#ifndef GEFEN_NS_WJ
-#define GEFEN_NS_WJ 2
-#endif
-constexpr int WI = 4, WJ = GEFEN_NS_WJ;  // 32x32 MFMA tiles per wave (rows, columns)
-constexpr int WAVES_N = TN / (32 * WJ), WAVES_M = TM / (32 * WI);
-constexpr int TT = 64 * WAVES_M * WAVES_N;
-constexpr int TCH = TM * TK / 8 / TT;  // 16-byte chunks per thread per operand tile
 
-struct TileGemm {
-    const uint16_t* A;
-    const uint16_t* B;
-    uint16_t* C;
-    uint16_t* CT;
-    const uint16_t* D;
-    int64_t lda, ldb, ldc, ldct, ldd;
-    int64_t sa, sb, sc, sct, sd;  // batch strides (elements)
-    int M, N, K;
-    float alpha, beta;
-    int tiles_n;   // N / TN
-    int tiles;     // tiles per matrix
-    int symmetric;
-    int d_t;       // D is given as D^T [N, M] (row stride ldd): four rows of one column are one 8-byte load
+template <int T_, int WI_, int WJ_>
+struct TileCfg {
+    static constexpr int T = T_, WI = WI_, WJ = WJ_;  // tile side; 32x32 MFMA tiles per wave (rows, columns)
+    static constexpr int WAVES_N = T / (32 * WJ), WAVES_M = T / (32 * WI);
+    static constexpr int TT = 64 * WAVES_M * WAVES_N;   // threads
+    static constexpr int TCH = T * TK / 8 / TT;         // 16-byte chunks per thread per operand tile
+    static constexpr int MCPR = T / 8;                  // 16-byte chunks per K row of an MN-major stage
+    static constexpr int TLDM = T + 32;                 // LDS row of an MN-major stage (bf16)
+    static constexpr int STAGE = T * TLD > TK * TLDM ? T * TLD : TK * TLDM;  // elements of one LDS stage
+    // Epilogue tile in LDS: C^T in rows of LDT bf16.  LDT / 2 = 2 (mod 32) dwords:
+    // the 8-byte accesses of 16 consecutive columns cover all banks once, and
+    // gathering one row from two column chunks 8 apart (16 mod 32 dwords) is
+    // conflict-free too.
+    static constexpr int LDT = T + 4;
+    static_assert(T * LDT <= 4 * STAGE, "the epilogue tile fits in the operand stages");
 };
+using Big = TileCfg<256, 4, 2>;
+using Small = TileCfg<128, 2, 2>;
+constexpr int TM = Big::T, TN = Big::T;
+static_assert(Small::T == kTileUnit && TK == kStepK, "ns_gemm.h");
 
-// Buffer resource over the 256 rows of one operand tile (rows r0 .. r0 + 255 of
+// Buffer resource over the T rows of one operand tile (rows r0 .. r0 + T - 1 of
 // a row-major matrix with row stride ld): the loads address it with a 32-bit
 // per-thread offset and a scalar offset, so no 64-bit address is formed per
-// load (the entry point checks that 256 rows fit in 2^31 bytes).
+// load (the entry point checks that T rows fit in 2^31 bytes).
+template <typename CF>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const uint16_t* rows, int64_t ld) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(rows), (short)0, (int)(TM * ld * 2), 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(rows), (short)0, (int)(CF::T * ld * 2), 0x00020000);
 }
-// The TCH 16-byte chunks of this thread in a 256 x TK operand tile at column k0:
+// The TCH 16-byte chunks of this thread in a T x TK operand tile at column k0:
 // chunk q = threadIdx.x + TT i is row q / CPR, k-chunk q % CPR.  voff is the
 // byte offset of chunk 0 (row threadIdx.x / CPR); chunk i is TT / CPR rows on.
-__device__ __forceinline__ void tile_load(__amdgpu_buffer_rsrc_t rs, int voff, int64_t ld, int k0, u32x4 out[TCH]) {
+template <typename CF>
+__device__ __forceinline__ void tile_load(__amdgpu_buffer_rsrc_t rs, int voff, int64_t ld, int k0, u32x4 out[CF::TCH]) {
 #pragma unroll
-    for (int i = 0; i < TCH; ++i)
+    for (int i = 0; i < CF::TCH; ++i)
         out[i] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, (int)(((int64_t)(TT / CPR) * i * ld + k0) * 2), 0));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, (int)(((int64_t)(CF::TT / CPR) * i * ld + k0) * 2), 0));
 }
-__device__ __forceinline__ void tile_store(uint16_t* lds, const u32x4 in[TCH]) {
+template <typename CF>
+__device__ __forceinline__ void tile_store(uint16_t* lds, const u32x4 in[CF::TCH]) {
 #pragma unroll
-    for (int i = 0; i < TCH; ++i) {
-        const int q = threadIdx.x + TT * i;
+    for (int i = 0; i < CF::TCH; ++i) {
+        const int q = threadIdx.x + CF::TT * i;
         *reinterpret_cast<u32x4*>(lds + (q / CPR) * TLD + (q % CPR) * 8) = in[i];
     }
 }
 
 // MN-major operand (the Gram product X X^T with only X^T stored): the operand is
-// given as its transpose [K, 256-column block], and a K step of the tile is
-// rows k0 .. k0 + TK of it, 256 elements each.  LDS keeps that layout, [k][m]
-// in rows of TLDM elements (576 bytes: consecutive rows start 16 banks apart,
+// given as its transpose [K, T-column block], and a K step of the tile is
+// rows k0 .. k0 + TK of it, T elements each.  LDS keeps that layout, [k][m]
+// in rows of TLDM elements (consecutive rows start 16 banks apart,
 // so the transposed fragment reads below are conflict-free), and fragments come
 // out of ds_read_b64_tr_b16.  Chunk q = threadIdx.x + TT i is row q / MCPR,
 // column chunk q % MCPR; chunk i is TT / MCPR rows on.
-constexpr int MCPR = TM / 8;   // 16-byte chunks per K row of the tile
-constexpr int TLDM = TM + 32;  // LDS row of an MN-major stage (bf16)
-static_assert(TK * TLDM == TM * TLD, "an MN-major stage has the size of a K-major one");
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc_mn(const uint16_t* cols, int64_t ld, int K) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(cols), (short)0, (int)(K * ld * 2), 0x00020000);
 }
-__device__ __forceinline__ void tile_load_mn(__amdgpu_buffer_rsrc_t rs, int voff, int64_t ld, int k0, u32x4 out[TCH]) {
+template <typename CF>
+__device__ __forceinline__ void tile_load_mn(__amdgpu_buffer_rsrc_t rs, int voff, int64_t ld, int k0,
+                                             u32x4 out[CF::TCH]) {
 #pragma unroll
-    for (int i = 0; i < TCH; ++i)
+    for (int i = 0; i < CF::TCH; ++i)
         out[i] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, (int)(((int64_t)(TT / MCPR) * i + k0) * ld * 2), 0));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                       rs, voff, (int)(((int64_t)(CF::TT / CF::MCPR) * i + k0) * ld * 2), 0));
 }
-__device__ __forceinline__ void tile_store_mn(uint16_t* lds, const u32x4 in[TCH]) {
+template <typename CF>
+__device__ __forceinline__ void tile_store_mn(uint16_t* lds, const u32x4 in[CF::TCH]) {
 #pragma unroll
-    for (int i = 0; i < TCH; ++i) {
-        const int q = threadIdx.x + TT * i;
-        *reinterpret_cast<u32x4*>(lds + (q / MCPR) * TLDM + (q % MCPR) * 8) = in[i];
+    for (int i = 0; i < CF::TCH; ++i) {
+        const int q = threadIdx.x + CF::TT * i;
+        *reinterpret_cast<u32x4*>(lds + (q / CF::MCPR) * CF::TLDM + (q % CF::MCPR) * 8) = in[i];
     }
 }
 // ds_read_b64_tr_b16: in each group of 16 lanes, lane 4 j + q gives the address
@@ -289,10 +297,12 @@ __device__ __forceinline__ void tile_store_mn(uint16_t* lds, const u32x4 in[TCH]
 // 8 (l / 32) + 0..7) is two such reads: lane l points at K row kk + 8 (l / 32) +
 // (l % 16) / 4 (+ 4 for the second read), column 16 ((l / 16) % 2) + 4 (l % 4).
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+template <int TLDM>
 __device__ __forceinline__ int mn_lane_offset(int lane) {
     const int g = lane >> 4, r = lane & 15;
     return (8 * (g >> 1) + (r >> 2)) * TLDM + 16 * (g & 1) + 4 * (r & 3);
 }
+template <int TLDM>
 __device__ __forceinline__ bf16x8 mn_frag(const uint16_t* p) {
     typedef __attribute__((address_space(3))) bf16x4 lds_v4;
     const auto* q = (const __attribute__((address_space(3))) uint16_t*)p;
@@ -325,14 +335,6 @@ __device__ __forceinline__ int logical_block(int b, int nwg) {
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 
-// Epilogue tile in LDS: T[c][r] = C[r][c] (the C^T orientation) in rows of LDT
-// bf16.  LDT / 2 = 130 dwords = 2 (mod 32): the 8-byte accesses of 16
-// consecutive columns cover all 32 banks once, and gathering one row from
-// two column chunks 8 apart (1040 dwords = 16 mod 32) is conflict-free too.
-constexpr int LDT = TM + 4;
-static_assert(TM == TN, "square tiles");
-static_assert(TN * LDT <= 4 * TM * TLD, "the epilogue tile fits in the operand stages");
-
 // GefenMuon's parameter update fused into the last Newton-Schulz product
 // (gefen_gemm_bf16_nt_batched_apply): matrix b of a launch is the update U of
 // parameter p[b], whose layout is U (rows of N elements) or, when transposed, U^T
@@ -350,12 +352,17 @@ struct FusedApply {
 // MN: both operands MN-major (the symmetric Gram product from X^T; no D, no C^T).
 // PD: void, or the parameter type of a fused update (fa != nullptr; C and C^T
 // are then not stored).
-template <bool MN, typename PD>
+// EDGE (fused update only): the parameter may end inside a tile (vm < M or vn <
+// N, the stack zero-padded) and rows need no alignment.
+template <typename CF, bool MN, typename PD, bool EDGE>
 __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApply* fa) {
-    // operand stages: A in [0, 2) and B in [2, 4) of TM x TLD each; the epilogue reuses them
-    __shared__ __attribute__((aligned(16))) uint16_t smem[4 * TM * TLD];
-    uint16_t* const As[2] = {smem, smem + TM * TLD};
-    uint16_t* const Bs[2] = {smem + 2 * TM * TLD, smem + 3 * TM * TLD};
+    constexpr int TS = CF::T, WI = CF::WI, WJ = CF::WJ, TT = CF::TT, TCH = CF::TCH, MCPR = CF::MCPR, TLDM = CF::TLDM;
+    constexpr int WAVES_N = CF::WAVES_N, LDT = CF::LDT;
+    constexpr int CR = TS / 8;  // 16-byte chunks per row of the output tile
+    // operand stages: A in [0, 2) and B in [2, 4); the epilogue reuses them
+    __shared__ __attribute__((aligned(16))) uint16_t smem[4 * CF::STAGE];
+    uint16_t* const As[2] = {smem, smem + CF::STAGE};
+    uint16_t* const Bs[2] = {smem + 2 * CF::STAGE, smem + 3 * CF::STAGE};
     const int lb = logical_block(blockIdx.x, gridDim.x);
     const int batch = lb / g.tiles;
     int t = lb - batch * g.tiles;
@@ -368,14 +375,14 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
         }
         tj = ti + t;
     } else {  // bands of kGroupM tile rows, column by column within a band
-        const int tiles_m = g.M / TM;
+        const int tiles_m = g.M / TS;
         const int band = t / (kGroupM * g.tiles_n);
         const int rows_in = min(kGroupM, tiles_m - band * kGroupM);
         const int w = t - band * kGroupM * g.tiles_n;
         ti = band * kGroupM + w % rows_in;
         tj = w / rows_in;
     }
-    const int m0 = ti * TM, n0 = tj * TN;
+    const int m0 = ti * TS, n0 = tj * TS;
     const uint16_t* __restrict__ A = g.A + batch * g.sa;
     const uint16_t* __restrict__ B = g.B + batch * g.sb;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -390,31 +397,31 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
 
     const int nk = g.K / TK;
     u32x4 ra[TCH], rb[TCH];  // register stage of the global -> LDS pipeline
-    const __amdgpu_buffer_rsrc_t rsa = MN ? tile_rsrc_mn(A + m0, g.lda, g.K) : tile_rsrc(A + (int64_t)m0 * g.lda, g.lda);
-    const __amdgpu_buffer_rsrc_t rsb = MN ? tile_rsrc_mn(B + n0, g.ldb, g.K) : tile_rsrc(B + (int64_t)n0 * g.ldb, g.ldb);
+    const __amdgpu_buffer_rsrc_t rsa = MN ? tile_rsrc_mn(A + m0, g.lda, g.K) : tile_rsrc<CF>(A + (int64_t)m0 * g.lda, g.lda);
+    const __amdgpu_buffer_rsrc_t rsb = MN ? tile_rsrc_mn(B + n0, g.ldb, g.K) : tile_rsrc<CF>(B + (int64_t)n0 * g.ldb, g.ldb);
     const int voa = MN ? (int)(((threadIdx.x / MCPR) * g.lda + (threadIdx.x % MCPR) * 8) * 2)
                        : (int)(((threadIdx.x / CPR) * g.lda + (threadIdx.x % CPR) * 8) * 2);
     const int vob = MN ? (int)(((threadIdx.x / MCPR) * g.ldb + (threadIdx.x % MCPR) * 8) * 2)
                        : (int)(((threadIdx.x / CPR) * g.ldb + (threadIdx.x % CPR) * 8) * 2);
     auto load_ops = [&](int k0) {
         if (MN) {
-            tile_load_mn(rsa, voa, g.lda, k0, ra);
-            tile_load_mn(rsb, vob, g.ldb, k0, rb);
+            tile_load_mn<CF>(rsa, voa, g.lda, k0, ra);
+            tile_load_mn<CF>(rsb, vob, g.ldb, k0, rb);
         } else {
-            tile_load(rsa, voa, g.lda, k0, ra);
-            tile_load(rsb, vob, g.ldb, k0, rb);
+            tile_load<CF>(rsa, voa, g.lda, k0, ra);
+            tile_load<CF>(rsb, vob, g.ldb, k0, rb);
         }
     };
     auto store_ops = [&](int stage) {
         if (MN) {
-            tile_store_mn(As[stage], ra);
-            tile_store_mn(Bs[stage], rb);
+            tile_store_mn<CF>(As[stage], ra);
+            tile_store_mn<CF>(Bs[stage], rb);
         } else {
-            tile_store(As[stage], ra);
-            tile_store(Bs[stage], rb);
+            tile_store<CF>(As[stage], ra);
+            tile_store<CF>(Bs[stage], rb);
         }
     };
-    const int mn_lofs = MN ? mn_lane_offset(lane) : 0;
+    const int mn_lofs = MN ? mn_lane_offset<TLDM>(lane) : 0;
     load_ops(0);
     store_ops(0);
     if (nk > 1) load_ops(TK);
@@ -433,8 +440,8 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
 #define GEFEN_LOAD_FRAGS(AS, BS, KK, AF, BF)                                                                      \
     {                                                                                                             \
     if (MN) {                                                                                                     \
-        _Pragma("unroll") for (int i = 0; i < WI; ++i) AF[i] = mn_frag((AS) + (KK) * TLDM + mn_lofs + wm + i * 32); \
-        _Pragma("unroll") for (int j = 0; j < WJ; ++j) BF[j] = mn_frag((BS) + (KK) * TLDM + mn_lofs + wn + j * 32); \
+        _Pragma("unroll") for (int i = 0; i < WI; ++i) AF[i] = mn_frag<TLDM>((AS) + (KK) * TLDM + mn_lofs + wm + i * 32); \
+        _Pragma("unroll") for (int j = 0; j < WJ; ++j) BF[j] = mn_frag<TLDM>((BS) + (KK) * TLDM + mn_lofs + wn + j * 32); \
     } else {                                                                                                      \
         _Pragma("unroll") for (int i = 0; i < WI; ++i) AF[i] =                                                    \
             *reinterpret_cast<const bf16x8*>((AS) + (wm + i * 32 + (lane & 31)) * TLD + (KK) + 8 * (lane >> 5));  \
@@ -453,7 +460,7 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
             _Pragma("unroll") for (int t_ = 0; t_ < WI * WJ; ++t_) {                                              \
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                \
                 if (s_ + 1 < TK / 16 && t_ < WI + WJ) __builtin_amdgcn_sched_group_barrier(0x100, MN ? 2 : 1, 0); \
-                if (s_ == 0 && t_ < 2 * TCH) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                   \
+                if (s_ * WI * WJ + t_ < 2 * TCH) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                   \
             }                                                                                                     \
         }                                                                                                         \
     }
@@ -495,7 +502,7 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
     const uint16_t* __restrict__ D = g.D ? g.D + batch * g.sd : nullptr;
     const bool mirror = g.symmetric && ti != tj;
     uint16_t* const T = smem;
-    constexpr int kChunks = TM * TN / 8 / TT;  // 16-byte chunks per thread
+    constexpr int kChunks = TS * TS / 8 / TT;  // 16-byte chunks per thread
     const bool d_lds = D && g.d_t;
     if (d_lds) {
         constexpr int kBatch = kChunks < 16 ? kChunks : 16;  // loads in flight per thread
@@ -505,13 +512,13 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
 #pragma unroll
             for (int i = 0; i < kBatch; ++i) {
                 const int q = threadIdx.x + TT * (i0 + i);
-                const int c = q >> 5, r8 = (q & 31) * 8;
+                const int c = q / CR, r8 = (q % CR) * 8;
                 dv[i] = *reinterpret_cast<const u32x4*>(D + (int64_t)(n0 + c) * g.ldd + m0 + r8);
             }
 #pragma unroll
             for (int i = 0; i < kBatch; ++i) {
                 const int q = threadIdx.x + TT * (i0 + i);
-                const int c = q >> 5, r8 = (q & 31) * 8;
+                const int c = q / CR, r8 = (q % CR) * 8;
                 uint2* t = reinterpret_cast<uint2*>(T + c * LDT + r8);
                 t[0] = make_uint2(dv[i].x, dv[i].y);
                 t[1] = make_uint2(dv[i].z, dv[i].w);
@@ -559,27 +566,17 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
         const float wdf = fa->wdf[batch], al = fa->alpha[batch];
         const bool dwd = fa->do_wd[batch] != 0, rp = fa->round_prod[batch] != 0;
         const bool tr = fa->transposed != 0;
-        int64_t e[kChunks];
-        Vec<PD, 8> pv[kChunks];
-#pragma unroll
-        for (int i = 0; i < kChunks; ++i) {
-            const int q = threadIdx.x + TT * i;
-            // transposed: parameter rows are rows of U^T, T row c -> row n0 + c;
-            // else rows of U, gathered from two column chunks of T as C below
-            e[i] = tr ? (int64_t)(n0 + (q >> 5)) * g.M + m0 + (q & 31) * 8
-                      : (int64_t)(m0 + (q & 31) + 32 * (q >> 10)) * g.N + n0 + ((q >> 5) & 31) * 8;
-            pv[i] = vload<PD, 8>(P, e[i]);
-        }
-#pragma unroll
-        for (int i = 0; i < kChunks; ++i) {
+        // transposed: parameter rows are rows of U^T, T row c -> row n0 + c;
+        // else rows of U, gathered from two column chunks of T as C below
+        auto update = [&](int i, PD* v) {
             const int q = threadIdx.x + TT * i;
             uint32_t w[4];
             if (tr) {
-                const uint2* t = reinterpret_cast<const uint2*>(T + (q >> 5) * LDT + (q & 31) * 8);
+                const uint2* t = reinterpret_cast<const uint2*>(T + (q / CR) * LDT + (q % CR) * 8);
                 const uint2 lo = t[0], hi = t[1];
                 w[0] = lo.x; w[1] = lo.y; w[2] = hi.x; w[3] = hi.y;
             } else {
-                const uint16_t* t = T + ((q >> 5) & 31) * 8 * LDT + (q & 31) + 32 * (q >> 10);
+                const uint16_t* t = T + ((q >> 5) % CR) * 8 * LDT + (q & 31) + 32 * (q / (32 * CR));
                 uint32_t h[8];
 #pragma unroll
                 for (int u = 0; u < 8; ++u) h[u] = t[u * LDT];
@@ -589,9 +586,59 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 const float uf = __uint_as_float((u & 1) ? (w[u >> 1] & 0xffff0000u) : (w[u >> 1] << 16));
-                pv[i].v[u] = from_f32<PD>(muon_apply_value<PD>(to_f32(pv[i].v[u]), uf, wdf, al, dwd, rp));
+                v[u] = from_f32<PD>(muon_apply_value<PD>(to_f32(v[u]), uf, wdf, al, dwd, rp));
             }
-            vstore<PD, 8>(P, e[i], pv[i]);
+        };
+        if constexpr (EDGE) {
+            // chunks of the parameter's own rows: whole ones as one access at the
+            // element's alignment, the last one of a row element by element
+            const int rows_v = tr ? g.vn : g.vm, ld = tr ? g.vm : g.vn;
+#pragma unroll
+            for (int i0 = 0; i0 < kChunks; i0 += 8) {
+                AnyVec<PD, 8> pv[8];
+                int cnt[8];
+                int64_t e[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int q = threadIdx.x + TT * (i0 + i);
+                    const int row = tr ? n0 + q / CR : m0 + (q & 31) + 32 * (q / (32 * CR));
+                    const int col = tr ? m0 + (q % CR) * 8 : n0 + ((q >> 5) % CR) * 8;
+                    cnt[i] = row < rows_v ? min(8, ld - col) : 0;
+                    e[i] = (int64_t)row * ld + col;
+                    if (cnt[i] == 8) {
+                        pv[i] = *reinterpret_cast<const AnyVec<PD, 8>*>(P + e[i]);
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) pv[i].v[u] = u < cnt[i] ? P[e[i] + u] : from_f32<PD>(0.0f);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    update(i0 + i, pv[i].v);
+                    if (cnt[i] == 8) {
+                        *reinterpret_cast<AnyVec<PD, 8>*>(P + e[i]) = pv[i];
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            if (u < cnt[i]) P[e[i] + u] = pv[i].v[u];
+                    }
+                }
+            }
+        } else {
+            int64_t e[kChunks];
+            Vec<PD, 8> pv[kChunks];
+#pragma unroll
+            for (int i = 0; i < kChunks; ++i) {
+                const int q = threadIdx.x + TT * i;
+                e[i] = tr ? (int64_t)(n0 + q / CR) * g.M + m0 + (q % CR) * 8
+                          : (int64_t)(m0 + (q & 31) + 32 * (q / (32 * CR))) * g.N + n0 + ((q >> 5) % CR) * 8;
+                pv[i] = vload<PD, 8>(P, e[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < kChunks; ++i) {
+                update(i, pv[i].v);
+                vstore<PD, 8>(P, e[i], pv[i]);
+            }
         }
         return;
     }
@@ -601,7 +648,7 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
 #pragma unroll
         for (int i = 0; i < kChunks; ++i) {
             const int q = threadIdx.x + TT * i;
-            const int c = q >> 5, r8 = (q & 31) * 8;
+            const int c = q / CR, r8 = (q % CR) * 8;
             const uint2* t = reinterpret_cast<const uint2*>(T + c * LDT + r8);
             const uint2 lo = t[0], hi = t[1];
             u32x4 v;
@@ -615,7 +662,7 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
 #pragma unroll
     for (int i = 0; i < kChunks; ++i) {
         const int q = threadIdx.x + TT * i;
-        const int r = (q & 31) + 32 * (q >> 10), c8 = ((q >> 5) & 31) * 8;
+        const int r = (q & 31) + 32 * (q / (32 * CR)), c8 = ((q >> 5) % CR) * 8;
         const uint16_t* t = T + c8 * LDT + r;
         uint32_t h[8];
 #pragma unroll
@@ -629,14 +676,110 @@ __device__ __forceinline__ void gemm_tile_body(const TileGemm& g, const FusedApp
     }
 }
 
-template <bool MN>
-__global__ __launch_bounds__(TT) void k_gemm_tile(const TileGemm g) {
-    gemm_tile_body<MN, void>(g, nullptr);
+template <typename CF, bool MN>
+__global__ __launch_bounds__(CF::TT, 2) void k_gemm_tile(const TileGemm g) {
+    gemm_tile_body<CF, MN, void, false>(g, nullptr);
 }
 
-template <typename PD>
-__global__ __launch_bounds__(TT) void k_gemm_tile_apply(const TileGemm g, const FusedApply fa) {
-    gemm_tile_body<false, PD>(g, &fa);
+template <typename CF, typename PD, bool EDGE>
+__global__ __launch_bounds__(CF::TT, 2) void k_gemm_tile_apply(const TileGemm g, const FusedApply fa) {
+    gemm_tile_body<CF, false, PD, EDGE>(g, &fa);
+}
+
+namespace {
+int64_t tile_count(int t, int m, int n, bool symmetric, int batch) {
+    const int64_t tn = n / t;
+    return (symmetric ? tn * (tn + 1) / 2 : (m / t) * tn) * batch;
+}
+}  // namespace
+
+// Measured per launch (microseconds, s = K / 64 steps): a round of 256 big tiles
+// (one per CU) takes 1.55 s + 14, a part of one 80% of that at least; 512 small
+// tiles (two per CU) take 1.06 s + 8.5, up to 256 of them alone 0.58 s + 8, and
+// as the tail of full rounds about 0.5 s.  So the small tile wins where big ones
+// leave CUs idle (twelve 768 x 2304 matrices: X X^T on 72 big tiles 62.8, on 252
+// small ones 29.5; sixteen 1024 x 2048: 64.5 and 59.2; eight 2048 x 6144: 293 and
+// 265), and the big one where there are rounds of them (56 of 2048 x 2048: 540 and
+// 645; a X + B X of eight 2048 x 6144: 410 and 504).
+double product_us(int m, int n, int k, bool symmetric, int batch, bool* small) {
+    const int64_t ts = tile_count(Small::T, m, n, symmetric, batch);
+    const double s = (double)k / TK;
+    const int64_t full = ts / 512, part = ts % 512;
+    double us_small = (double)full * (1.06 * s + 8.5);
+    if (part > 256) us_small += 1.06 * s + 8.5;
+    else if (part > 0) us_small += full ? 0.5 * s : 0.58 * s + 8.0;
+    *small = true;
+    if (m % Big::T || n % Big::T) return us_small;
+    const int64_t tb = tile_count(Big::T, m, n, symmetric, batch), left = tb % 256;
+    const double us_big = (1.55 * s + 14.0) * ((double)(tb / 256) + (left ? 0.8 + 0.2 * (double)left / 256.0 : 0.0));
+    *small = us_small < us_big;
+    return *small ? us_small : us_big;
+}
+
+int launch_product(TileGemm g, int batch, bool mn, hipStream_t st, const char* what) {
+    bool small;
+    product_us(g.M, g.N, g.K, g.symmetric != 0, batch, &small);
+    const int t = small ? Small::T : Big::T;
+    g.tiles_n = g.N / t;
+    const int64_t grid = tile_count(t, g.M, g.N, g.symmetric != 0, batch);
+    if (grid > INT32_MAX) return fail_inval("batched GEMM grid too large");
+    g.tiles = (int)(grid / batch);
+    const dim3 blocks((unsigned)grid);
+    if (small) {
+        if (mn) hipLaunchKernelGGL((k_gemm_tile<Small, true>), blocks, dim3(Small::TT), 0, st, g);
+        else hipLaunchKernelGGL((k_gemm_tile<Small, false>), blocks, dim3(Small::TT), 0, st, g);
+    } else {
+        if (mn) hipLaunchKernelGGL((k_gemm_tile<Big, true>), blocks, dim3(Big::TT), 0, st, g);
+        else hipLaunchKernelGGL((k_gemm_tile<Big, false>), blocks, dim3(Big::TT), 0, st, g);
+    }
+    return launch_status(what);
+}
+
+int launch_product_apply(TileGemm g0, int batch, const gefen_muon_apply_task* tasks, bool edge, hipStream_t st,
+                         const char* what) {
+    for (int c0 = 0; c0 < batch; c0 += kMaxFuse) {
+        const int nb = batch - c0 < kMaxFuse ? batch - c0 : kMaxFuse;
+        bool small;
+        product_us(g0.M, g0.N, g0.K, false, nb, &small);
+        const int t = small ? Small::T : Big::T;
+        TileGemm g = g0;
+        g.A += c0 * g.sa;
+        g.B += c0 * g.sb;
+        if (g.D) g.D += c0 * g.sd;
+        g.symmetric = 0;
+        g.tiles_n = g.N / t;
+        const int64_t grid = tile_count(t, g.M, g.N, false, nb);
+        if (grid > INT32_MAX) return fail_inval("batched GEMM grid too large");
+        g.tiles = (int)(grid / nb);
+        FusedApply fa;
+        memset(&fa, 0, sizeof(fa));
+        fa.transposed = tasks[0].transposed ? 1 : 0;
+        for (int i = 0; i < nb; ++i) {
+            const MuonApplyScalars sc = muon_apply_scalars(tasks[c0 + i]);
+            fa.p[i] = tasks[c0 + i].p;
+            fa.wdf[i] = sc.wdf;
+            fa.alpha[i] = sc.alpha;
+            fa.do_wd[i] = (uint8_t)sc.do_wd;
+            fa.round_prod[i] = (uint8_t)sc.round_prod;
+        }
+        const dim3 blocks((unsigned)grid);
+        auto launch = [&](auto ptag) {
+            using PD = decltype(ptag);
+            if (small) {
+                if (edge) hipLaunchKernelGGL((k_gemm_tile_apply<Small, PD, true>), blocks, dim3(Small::TT), 0, st, g, fa);
+                else hipLaunchKernelGGL((k_gemm_tile_apply<Small, PD, false>), blocks, dim3(Small::TT), 0, st, g, fa);
+            } else {
+                if (edge) hipLaunchKernelGGL((k_gemm_tile_apply<Big, PD, true>), blocks, dim3(Big::TT), 0, st, g, fa);
+                else hipLaunchKernelGGL((k_gemm_tile_apply<Big, PD, false>), blocks, dim3(Big::TT), 0, st, g, fa);
+            }
+        };
+        if (tasks[0].param_dtype == GEFEN_F32) launch(float{});
+        else if (tasks[0].param_dtype == GEFEN_BF16) launch(bf16_t{});
+        else launch(f16_t{});
+        const int rc = launch_status(what);
+        if (rc) return rc;
+    }
+    return GEFEN_OK;
 }
 
 }  // namespace ns
@@ -695,6 +838,7 @@ extern "C" int gefen_gemm_bf16_nt_batched(const void* a, int64_t lda, int64_t st
             return fail_inval("batched GEMM operands need 16-byte aligned rows");
     }
     ns::TileGemm g;
+    memset(&g, 0, sizeof(g));
     g.A = static_cast<const uint16_t*>(a);
     g.B = static_cast<const uint16_t*>(b);
     g.C = static_cast<uint16_t*>(c);
@@ -705,16 +849,10 @@ extern "C" int gefen_gemm_bf16_nt_batched(const void* a, int64_t lda, int64_t st
     g.M = m; g.N = n; g.K = k;
     g.alpha = (float)alpha;
     g.beta = (float)beta;
-    g.tiles_n = n / ns::TN;
     g.symmetric = symmetric ? 1 : 0;
-    g.tiles = symmetric ? g.tiles_n * (g.tiles_n + 1) / 2 : (m / ns::TM) * g.tiles_n;
     g.d_t = d_transposed ? 1 : 0;
     if (g.D && d_transposed && ldd % 4) return fail_inval("D^T rows must be 8-byte aligned");
-    const int64_t grid = (int64_t)g.tiles * batch;
-    if (grid > INT32_MAX) return fail_inval("batched GEMM grid too large");
-    hipLaunchKernelGGL(ns::k_gemm_tile<false>, dim3((unsigned)grid), dim3(ns::TT), 0, reinterpret_cast<hipStream_t>(stream),
-                       g);
-    return launch_status("gefen_gemm_bf16_nt_batched");
+    return ns::launch_product(g, batch, false, reinterpret_cast<hipStream_t>(stream), "gefen_gemm_bf16_nt_batched");
 }
 
 extern "C" int gefen_gram_bf16_batched(const void* xt, int64_t ldxt, int64_t stride_xt, void* c, int64_t ldc,
@@ -743,14 +881,8 @@ extern "C" int gefen_gram_bf16_batched(const void* xt, int64_t ldxt, int64_t str
     g.K = k;
     g.alpha = (float)alpha;
     g.beta = 0.0f;
-    g.tiles_n = m / ns::TN;
     g.symmetric = 1;
-    g.tiles = g.tiles_n * (g.tiles_n + 1) / 2;
-    const int64_t grid = (int64_t)g.tiles * batch;
-    if (grid > INT32_MAX) return fail_inval("batched GEMM grid too large");
-    hipLaunchKernelGGL(ns::k_gemm_tile<true>, dim3((unsigned)grid), dim3(ns::TT), 0, reinterpret_cast<hipStream_t>(stream),
-                       g);
-    return launch_status("gefen_gram_bf16_batched");
+    return ns::launch_product(g, batch, true, reinterpret_cast<hipStream_t>(stream), "gefen_gram_bf16_batched");
 }
 
 extern "C" int gefen_gemm_bf16_nt_batched_apply(const void* a, int64_t lda, int64_t stride_a, const void* b,
@@ -786,46 +918,20 @@ extern "C" int gefen_gemm_bf16_nt_batched_apply(const void* a, int64_t lda, int6
         if (!t.p) return fail_inval("null parameter pointer");
         if (!aligned(t.p, 8 * dtype_size(dt))) return fail_inval("parameters need %d-byte alignment", 8 * dtype_size(dt));
     }
-    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const int tiles = (m / ns::TM) * (n / ns::TN);
-    for (int c0 = 0; c0 < batch; c0 += ns::kMaxFuse) {
-        const int nb = batch - c0 < ns::kMaxFuse ? batch - c0 : ns::kMaxFuse;
-        ns::TileGemm g;
-        memset(&g, 0, sizeof(g));
-        g.A = static_cast<const uint16_t*>(a) + c0 * stride_a;
-        g.B = static_cast<const uint16_t*>(b) + c0 * stride_b;
-        g.D = beta != 0.0 ? static_cast<const uint16_t*>(d_t) + c0 * stride_d : nullptr;
-        g.lda = lda; g.ldb = ldb; g.ldd = ldd;
-        g.sa = stride_a; g.sb = stride_b; g.sd = stride_d;
-        g.M = m; g.N = n; g.K = k;
-        g.alpha = (float)alpha;
-        g.beta = (float)beta;
-        g.tiles_n = n / ns::TN;
-        g.symmetric = 0;
-        g.tiles = tiles;
-        g.d_t = 1;
-        if (g.D && ldd % 4) return fail_inval("D^T rows must be 8-byte aligned");
-        ns::FusedApply fa;
-        memset(&fa, 0, sizeof(fa));
-        fa.transposed = transposed;
-        for (int i = 0; i < nb; ++i) {
-            const MuonApplyScalars sc = muon_apply_scalars(tasks[c0 + i]);
-            fa.p[i] = tasks[c0 + i].p;
-            fa.wdf[i] = sc.wdf;
-            fa.alpha[i] = sc.alpha;
-            fa.do_wd[i] = (uint8_t)sc.do_wd;
-            fa.round_prod[i] = (uint8_t)sc.round_prod;
-        }
-        const int64_t grid = (int64_t)tiles * nb;
-        if (grid > INT32_MAX) return fail_inval("batched GEMM grid too large");
-        if (dt == GEFEN_F32)
-            hipLaunchKernelGGL(ns::k_gemm_tile_apply<float>, dim3((unsigned)grid), dim3(ns::TT), 0, st, g, fa);
-        else if (dt == GEFEN_BF16)
-            hipLaunchKernelGGL(ns::k_gemm_tile_apply<bf16_t>, dim3((unsigned)grid), dim3(ns::TT), 0, st, g, fa);
-        else
-            hipLaunchKernelGGL(ns::k_gemm_tile_apply<f16_t>, dim3((unsigned)grid), dim3(ns::TT), 0, st, g, fa);
-        const int rc = launch_status("gefen_gemm_bf16_nt_batched_apply");
-        if (rc) return rc;
-    }
-    return GEFEN_OK;
+    if (beta != 0.0 && ldd % 4) return fail_inval("D^T rows must be 8-byte aligned");
+    ns::TileGemm g;
+    memset(&g, 0, sizeof(g));
+    g.A = static_cast<const uint16_t*>(a);
+    g.B = static_cast<const uint16_t*>(b);
+    g.D = beta != 0.0 ? static_cast<const uint16_t*>(d_t) : nullptr;
+    g.lda = lda; g.ldb = ldb; g.ldd = ldd;
+    g.sa = stride_a; g.sb = stride_b; g.sd = stride_d;
+    g.M = g.vm = m;
+    g.N = g.vn = n;
+    g.K = k;
+    g.alpha = (float)alpha;
+    g.beta = (float)beta;
+    g.d_t = 1;
+    return ns::launch_product_apply(g, batch, tasks, false, reinterpret_cast<hipStream_t>(stream),
+                                    "gefen_gemm_bf16_nt_batched_apply");
 }
