@@ -52,6 +52,8 @@ SIGNATURES = {
     "gefen_ns_prepare_sumsq": (I32, [P, P, I32, I32, I32, DBL, P, P, P]),
     "gefen_ns_normalize_sumsq": (I32, [P, P, I32, I32, I32, DBL, P, P, I32, P]),
     "gefen_muon_apply_tasks": (I32, [P, I32, P]),
+    "gefen_newton_schulz_workspace_size": (SZ, [I32, I32, I32]),
+    "gefen_newton_schulz_apply": (I32, [P, I32, I32, I32, DBL, DBL, DBL, I32, DBL, P, P, P, P, P]),
     "gefen_exact_histogram": (I32, [P, I32, I64, I64, P, I32, P]),
     "gefen_accumulate_counts": (I32, [P, P, I32, P]),
     "gefen_exact_dp_workspace_size": (SZ, [I32, I32]),

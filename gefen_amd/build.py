@@ -35,7 +35,7 @@ COMMON = [
 LIBS = {
     "libgefen_hip.so": ["capi.cpp", "step.hip", "step_inst_bf16.hip", "step_inst_f16.hip", "step_inst_f32.hip",
                         "step_inst_bf16_f32.hip", "step_inst_f16_f32.hip", "codebook.hip", "period.hip", "ns_gemm.hip",
-                        "muon.hip"],
+                        "newton_schulz.hip", "muon.hip"],
     "libgefen_synth.so": ["capi.cpp", "synthetic.hip"],
 }
 

@@ -11,6 +11,7 @@ parameter update is one batched launch with the reference's CPU arithmetic
 from __future__ import annotations
 
 import math
+from itertools import chain
 from typing import Iterable, Optional, Tuple, Union
 
 import numpy as np
@@ -166,18 +167,22 @@ class GefenMuon(Gefen):
         tasks = np.zeros(len(items), dtype=_lib.MUON_TASK)
         # Matrices of one shape, dtype and Newton-Schulz setting share a stacked
         # buffer: the momentum kernel writes each one's Nesterov blend into its
-        # slice and Newton-Schulz runs on the whole stack.
-        from gefen_amd.newton_schulz import batched_shape_ok
+        # slice and Newton-Schulz runs on the whole stack.  Sides that fill no tile run
+        # zero-padded (one call per stack, its update included).
+        from gefen_amd.newton_schulz import batched_shape_ok, padded_shape_ok
 
         stacks = {}
+        padded = {}
         for i, (group, p, local_p, grad) in enumerate(items):
             rows, cols = grad.shape
+            key = (rows, cols, grad.dtype, tuple(group["ns_coefficients"]), group["ns_steps"], group["eps"])
             if batched_shape_ok(rows, cols):
-                key = (rows, cols, grad.dtype, tuple(group["ns_coefficients"]), group["ns_steps"], group["eps"])
                 stacks.setdefault(key, []).append(i)
+            elif group["ns_steps"] > 0 and padded_shape_ok(rows, cols):
+                padded.setdefault(key + (local_p.dtype,), []).append(i)
         where = {}
         bufs = {}
-        for key, idx in stacks.items():
+        for key, idx in chain(stacks.items(), padded.items()):
             rows, cols = key[0], key[1]
             bufs[key] = torch.empty(len(idx), rows, cols, dtype=torch.bfloat16, device=items[idx[0]][3].device)
             for slot, i in enumerate(idx):
@@ -218,7 +223,7 @@ class GefenMuon(Gefen):
         # float32 matrices: 3.38 -> 3.14 ms per step)
         sumsq = torch.empty(len(items) * _SUMSQ_STRIDE, dtype=torch.float64, device=dev)
         sum_index = {key: torch.tensor(idx, dtype=torch.int32, device=dev)
-                     for key, idx in stacks.items()}
+                     for key, idx in chain(stacks.items(), padded.items())}
         with torch.cuda.device(dev):
             rc = lib.gefen_muon_tasks_sumsq(tasks.ctypes.data, len(items), tables.data_ptr(), sumsq.data_ptr(),
                                             torch.cuda.current_stream(dev).cuda_stream)
@@ -237,12 +242,13 @@ class GefenMuon(Gefen):
                 for slot, i in enumerate(idx):
                     updates[i] = res[slot]
         apply = np.zeros(len(items), dtype=_lib.MUON_APPLY_TASK)
+        in_padded = {i for idx in padded.values() for i in idx}
         copy_back = []
         for i, ((group, p, local_p, grad), out) in enumerate(zip(items, outs)):
             st = self.state[p]
             st["step"] += 1
             update = updates.get(i)
-            if update is None:
+            if update is None and i not in in_padded:
                 update = _zeropower_via_newtonschulz(out.view_as(grad), group["ns_coefficients"], group["ns_steps"],
                                                      group["eps"]).contiguous()
             keep.append(update)
@@ -266,15 +272,21 @@ class GefenMuon(Gefen):
                 wd = 0.0
             t = apply[i]
             t["p"] = target.data_ptr()
-            t["update"] = update.data_ptr()
+            t["update"] = update.data_ptr() if update is not None else 0
             t["numel"] = target.numel()
             t["param_dtype"] = _DTYPE_CODE[target.dtype]
             t["transposed"] = 1 if grad.size(0) > grad.size(1) else 0
             t["lr"] = lr
             t["weight_decay"] = wd
             t["adjusted_lr"] = adjusted
+        pruns = []
+        for key, idx in padded.items():
+            _check_ns_args(key[3], key[4])
+            pruns.append(_PaddedStack(key, idx, bufs[key], sum_index[key]))
+            pruns[-1].run(apply, sumsq)
+        rest = np.ascontiguousarray(apply[[i for i in range(len(items)) if i not in in_padded]])
         with torch.cuda.device(dev):
-            rc = lib.gefen_muon_apply_tasks(apply.ctypes.data, len(items), torch.cuda.current_stream(dev).cuda_stream)
+            rc = lib.gefen_muon_apply_tasks(rest.ctypes.data, len(rest), torch.cuda.current_stream(dev).cuda_stream)
         _lib.check(rc, "gefen_muon_apply_tasks")
         for local_p, target in copy_back:
             local_p.copy_(target)
@@ -286,7 +298,7 @@ class GefenMuon(Gefen):
             solo = [(i, outs[i], tuple(items[i][0]["ns_coefficients"]), items[i][0]["ns_steps"], items[i][0]["eps"])
                     for i in range(len(items)) if i not in where]
             self._plan = _MuonPlan(self, items, tasks, apply, [(key, idx, bufs[key], works[key], sum_index[key])
-                                                                 for key, idx in stacks.items()], dev, sumsq, solo)
+                                                                 for key, idx in stacks.items()], dev, sumsq, solo, pruns)
         del keep
 
     @_step_entry
@@ -304,6 +316,28 @@ class GefenMuon(Gefen):
         return loss
 
 
+class _PaddedStack:
+    """A stack of matrices whose sides fill no tile: Newton-Schulz on zero-padded
+    copies and the parameters' updates, one library call per step
+    (gefen_newton_schulz_apply)."""
+
+    def __init__(self, key, idx, buf, index):
+        (self.rows, self.cols, _, self.coeffs, self.steps, self.eps, _) = key
+        self.idx, self.buf, self.index = idx, buf, index
+        nbytes = int(_lib.load().gefen_newton_schulz_workspace_size(len(idx), self.rows, self.cols))
+        self.work = torch.empty(nbytes, dtype=torch.uint8, device=buf.device)
+
+    def run(self, apply, sumsq):
+        tasks = np.ascontiguousarray(apply[self.idx])
+        a, b, c = self.coeffs
+        with torch.cuda.device(self.buf.device):
+            rc = _lib.load().gefen_newton_schulz_apply(
+                self.buf.data_ptr(), len(self.idx), self.rows, self.cols, a, b, c, self.steps, float(self.eps),
+                sumsq.data_ptr(), self.index.data_ptr(), self.work.data_ptr(), tasks.ctypes.data,
+                torch.cuda.current_stream(self.buf.device).cuda_stream)
+        _lib.check(rc, "gefen_newton_schulz_apply")
+
+
 class _MuonPlan:
     """Cached task tables of GefenMuon._step_all (the GefenMuon counterpart of
     gefen._StepPlan): the momentum and update task tables, the stacked Newton-
@@ -316,11 +350,12 @@ class _MuonPlan:
     A stack with Newton-Schulz steps applies its parameters' updates inside its
     last product (gefen_gemm_bf16_nt_batched_apply), so the updates are never
     stored and read back; the first step (the table build) applies them with
-    gefen_muon_apply_tasks, which the plan's results equal bit for bit.  Matrices
-    off the batched path keep their momentum output buffer and take the
-    one-matrix Newton-Schulz and gefen_muon_apply_tasks, as in the build."""
+    gefen_muon_apply_tasks, which the plan's results equal bit for bit.  Padded
+    stacks run one call each, as in the build.  Matrices off both paths keep their
+    momentum output buffer and take the one-matrix Newton-Schulz and
+    gefen_muon_apply_tasks, as in the build."""
 
-    def __init__(self, opt, items, mtasks, apply, stacks, device, sumsq, solo=()):
+    def __init__(self, opt, items, mtasks, apply, stacks, device, sumsq, solo=(), padded=()):
         self.params = [it[1] for it in items]
         self.pptr = [it[1].data_ptr() for it in items]
         self.numel = [it[3].numel() for it in items]
@@ -350,6 +385,9 @@ class _MuonPlan:
             self.fuse.append(ok)
             if ok:
                 fused[idx] = True
+        self.padded = list(padded)
+        for stack in self.padded:
+            fused[stack.idx] = True
         self.rest = np.nonzero(~fused)[0]
         # (item, momentum output, coefficients, steps, eps) of the matrices outside
         # the stacks: one-matrix Newton-Schulz, then gefen_muon_apply_tasks
@@ -417,6 +455,8 @@ class _MuonPlan:
                 keep.append(res)
                 slot_bytes = res[0].numel() * res.element_size()
                 self.apply["update"][idx] = res.data_ptr() + np.arange(len(idx), dtype=np.uint64) * slot_bytes
+            for stack in self.padded:
+                stack.run(self.apply, self.sumsq)
             for i, out, coeffs, steps, eps in self.solo:
                 upd = _zeropower_via_newtonschulz(out, coeffs, steps, eps).contiguous()
                 keep.append(upd)

@@ -8,8 +8,10 @@ newton_schulz_batched runs a stack of same-shaped matrices at once with the
 large-tile batched GEMM, keeping only X^T between iterations: X X^T comes from
 X^T through transposing LDS reads (gefen_gram_bf16_batched), b A + c A A is an
 A B^T product of the symmetric A, and B X = (X^T B)^T is written as X'^T (the
-last iteration writes the orientation it returns).  newton_schulz_bf16 is the
-one-matrix path for shapes the batched GEMM does not tile.
+last iteration writes the orientation it returns).  gefen_newton_schulz_apply does
+the same on zero-padded copies of matrices whose sides fill no tile, and
+newton_schulz_bf16 is the one-matrix path for the smallest ones and for matrices
+too large to address.
 """
 
 from __future__ import annotations
@@ -71,6 +73,24 @@ def batched_shape_ok(rows: int, cols: int) -> bool:
     and reads one bf16 matrix through a buffer of less than 2^31 bytes."""
     return (rows > 0 and cols > 0 and rows % 256 == 0 and cols % 256 == 0
             and rows * cols * 2 <= _BATCHED_MAX_BYTES)
+
+
+# Padding a matrix to tiles of 128 costs memory and products in proportion: at most
+# this many times its elements, unless the padded matrix is small anyway.
+_PADDED_MAX_WASTE, _PADDED_SMALL = 4, 1 << 22
+
+
+def padded_shape_ok(rows: int, cols: int) -> bool:
+    """Whether gefen_newton_schulz_apply takes a stack of such matrices (the tiled
+    products on zero-padded copies, many matrices per launch).  Matrices of one tile
+    or less stay on the one-matrix path, and so do those whose padding would cost
+    more memory than it saves launches."""
+    if rows <= 0 or cols <= 0 or max(rows, cols) <= 128:
+        return False
+    up = [-(-v // 128) * 128 for v in (rows, cols)]
+    if up[0] * up[1] > max(_PADDED_MAX_WASTE * rows * cols, _PADDED_SMALL):
+        return False
+    return int(_lib.load().gefen_newton_schulz_workspace_size(1, rows, cols)) > 0
 
 
 def gemm_nt_batched(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, out_t: torch.Tensor = None,

@@ -271,6 +271,21 @@ int gefen_gemm_bf16_nt_batched_apply(const void* a, int64_t lda, int64_t stride_
                                      int m, int n, int k, double alpha, double beta,
                                      const gefen_muon_apply_task* tasks, gefen_stream_t stream);
 
+/* Newton-Schulz of a stack and GefenMuon's update of its parameters in one call,
+ * for matrices of any size (gefen_muon.py:16-51, 325-329): x holds `batch` bf16
+ * matrices [rows, cols] (contiguous, the blends gefen_muon_tasks_sumsq wrote, with
+ * their sums of squares as in gefen_ns_prepare_sumsq), steps >= 1 iterations with
+ * coefficients a, b, c run on zero-padded copies in `workspace`
+ * (gefen_newton_schulz_workspace_size bytes, 16-byte aligned; 0 for a matrix whose
+ * padded form has 2^31 bytes or more, which is refused), and parameter tasks[i].p
+ * (layout of x, any element-aligned address) is updated as gefen_muon_apply_tasks
+ * updates it with the result (tasks[i].update is not read; transposed = rows > cols;
+ * one dtype per call).  The products equal the unpadded ones bit for bit. */
+size_t gefen_newton_schulz_workspace_size(int batch, int rows, int cols);
+int gefen_newton_schulz_apply(const void* x, int batch, int rows, int cols, double a, double b, double c, int steps,
+                              double eps, const double* sumsq, const int32_t* index, void* workspace,
+                              const gefen_muon_apply_task* tasks, gefen_stream_t stream);
+
 /* ------------------------------------------------------------------ first step
  * Replaces gefen_exact_histogram_cuda (exact_histogram_fused.py:10-58,
  * exact_histogram_fused_kernel.cu:131-160): per block absmax normalisation,
