@@ -4,9 +4,9 @@
 //
 // Histogram: gefen.py:350-366.  Exact DP: quantization.py:206-258 with the
 // histogram statistics of gefen.py:373-399; the DP is evaluated level by level
-// (one launch per cluster count), one wave per segment end, with the
-// reference's strict "<" (first best start wins) reproduced by a lexicographic
-// (cost, start) minimum.  All float64 arithmetic is written without
+// (one launch per cluster count), one wave per segment end, over the starts that
+// a bound on the cost leaves, with the reference's strict "<" (first best start
+// wins) reproduced by a lexicographic (cost, start) minimum.  All float64 arithmetic is written without
 // contraction, so every cost and codeword equals the reference's.
 #include <math.h>
 #include <string.h>
@@ -168,13 +168,18 @@ __global__ void k_accumulate_counts(float* __restrict__ acc, const int64_t* __re
 
 // ---------------------------------------------------------------------------
 // exact DP workspace:
-//   header  int32[64]      : [0] N active bins, [1] status (0 ok, 1 padded done, 2 empty)
+//   header  int32[64]      : [0] N active bins, [1] status (0 ok, 1 padded done, 2 empty),
+//                            [2..3] kDpSlack * sum(w) as a double
 //   pw, pwx, pwx2          : double[bins + 1] each (prefix sums, sequential order)
 //   dp                     : double[(K + 1) * (bins + 1)], level-major
 //   bt                     : int32[(K + 1) * (bins + 1)]
+//   jump                   : int32[kDpGroups * (bins + 1)], see k_dp_jump
 //   cw                     : float[bins] active centres
+constexpr int kDpMaxK = 256;
+constexpr int kDpGroup = 16;  // levels that one jump table crosses
+constexpr int kDpGroups = kDpMaxK / kDpGroup;
 struct DpLayout {
-    size_t pw, pwx, pwx2, dp, bt, cw, total;
+    size_t pw, pwx, pwx2, dp, bt, jump, cw, total;
     DpLayout(int bins, int K) {
         size_t o = 256;
         pw = o;  o += sizeof(double) * (bins + 1);
@@ -182,6 +187,7 @@ struct DpLayout {
         pwx2 = o; o += sizeof(double) * (bins + 1);
         dp = o;  o += sizeof(double) * (size_t)(K + 1) * (bins + 1);
         bt = o;  o += sizeof(int32_t) * (size_t)(K + 1) * (bins + 1);
+        jump = o; o += sizeof(int32_t) * (size_t)kDpGroups * (bins + 1);
         cw = o;  o += sizeof(float) * bins;
         total = o;
     }
@@ -189,130 +195,171 @@ struct DpLayout {
 
 constexpr int kDpMaxBins = 4096;
 constexpr int kDpInitThreads = 256;
+constexpr double kDpSlack = 0x1p-28;  // see k_dp_level
+
+// The first `n` values of v (LDS, n <= kDpMaxK) in ascending order, equal ones as
+// they stood (an insertion sort; in parallel it is only checked, since codewords
+// come out sorted), written to out.  Every thread of the workgroup takes part.
+__device__ __forceinline__ void sort_codewords(float* v, int n, float* __restrict__ out, int* unsorted) {
+    const int t = threadIdx.x;
+    if (t == 0) *unsorted = 0;
+    __syncthreads();
+    if (t > 0 && t < n && !(v[t - 1] <= v[t])) *unsorted = 1;
+    __syncthreads();
+    if (*unsorted && t == 0) {
+        for (int i = 1; i < n; ++i) {
+            const float x = v[i];
+            int j = i - 1;
+            while (j >= 0 && v[j] > x) { v[j + 1] = v[j]; --j; }
+            v[j + 1] = x;
+        }
+    }
+    __syncthreads();
+    if (t < n) out[t] = v[t];
+}
 
 // Active bins (count > 0) in bin order, their centres -1 + (2b+1)/bins (exact
 // for power-of-two bins), and the float64 prefix sums of w, w x, w x^2
 // (torch.cumsum on the CPU, quantization.py:226-231: the element products in
 // parallel, then the sums in sequential order).  The workgroup compacts the
-// active bins into LDS (a scan of per-thread counts); one thread then runs the
-// three running sums in registers.
+// active bins into LDS (a scan of per-thread counts); then one lane of each of
+// three waves runs one of the sums in order, the next 32 elements read while the
+// current ones are added: a chain of 4096 dependent additions, 18 ns each (one
+// lane for all three sums, 16 elements at a time: 132 us; now 76).
 __global__ __launch_bounds__(kDpInitThreads) void k_dp_init(const float* __restrict__ counts, int bins, int K,
                                                             int force, char* __restrict__ ws, DpLayout L,
                                                             float* __restrict__ out) {
     constexpr int kPer = kDpMaxBins / kDpInitThreads;  // bins per thread
-    __shared__ double sw_[kDpMaxBins], swx_[kDpMaxBins], swx2_[kDpMaxBins];
-    __shared__ int offs[kDpInitThreads + 1];
+    __shared__ __attribute__((aligned(16))) double sums[3][kDpMaxBins];
+    __shared__ int wave_total[kDpInitThreads / 64];
+    __shared__ float sorted[kDpMaxK];
+    __shared__ int unsorted;
     int32_t* hdr = reinterpret_cast<int32_t*>(ws);
     double* pw = reinterpret_cast<double*>(ws + L.pw);
     double* pwx = reinterpret_cast<double*>(ws + L.pwx);
     double* pwx2 = reinterpret_cast<double*>(ws + L.pwx2);
     double* dp = reinterpret_cast<double*>(ws + L.dp);
     float* cw = reinterpret_cast<float*>(ws + L.cw);
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63;
     const int b0 = t * kPer;  // this thread's bins b0 .. b0 + kPer - 1 (in order)
-    int mine = 0;
-    for (int k = 0; k < kPer; ++k) mine += (b0 + k < bins && counts[b0 + k] > 0.0f) ? 1 : 0;
-    offs[t + 1] = mine;
-    if (t == 0) offs[0] = 0;
-    __syncthreads();
-    if (t == 0)
-        for (int i = 1; i <= kDpInitThreads; ++i) offs[i] += offs[i - 1];
-    __syncthreads();
-    const double inv_bins = 1.0 / (double)bins;  // exact: bins is a power of two
-    int n = offs[t];
+    float mine[kPer];
+    int cnt = 0;
+#pragma unroll
     for (int k = 0; k < kPer; ++k) {
-        const int b = b0 + k;
-        if (b >= bins) break;
-        const float c = counts[b];
-        if (c > 0.0f) {
-            const float center = (float)(-1.0 + (2.0 * b + 1.0) * inv_bins);
-            const double w = (double)c, x = (double)center;
-            sw_[n] = w;
-            swx_[n] = w * x;
-            swx2_[n] = w * (x * x);
+        mine[k] = b0 + k < bins ? counts[b0 + k] : 0.0f;
+        cnt += mine[k] > 0.0f ? 1 : 0;
+    }
+    int incl = cnt;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
+    }
+    if (lane == 63) wave_total[t >> 6] = incl;
+    __syncthreads();
+    int n = incl - cnt, N = 0;
+    for (int w = 0; w < kDpInitThreads / 64; ++w) {
+        if (w < (t >> 6)) n += wave_total[w];
+        N += wave_total[w];
+    }
+    const double inv_bins = 1.0 / (double)bins;  // exact: bins is a power of two
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        if (mine[k] > 0.0f) {
+            const float center = (float)(-1.0 + (2.0 * (b0 + k) + 1.0) * inv_bins);
+            const double w = (double)mine[k], x = (double)center;
+            sums[0][n] = w;
+            sums[1][n] = w * x;
+            sums[2][n] = w * (x * x);
             cw[n] = center;
             ++n;
         }
     }
     __syncthreads();
-    const int N = offs[kDpInitThreads];
-    if (t == 0) {  // the running sums in bin order, in place in LDS (16 elements read ahead)
-        constexpr int kB = 16;
-        double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-        int i = 0;
-        for (; i + kB <= N; i += kB) {
-            double v0[kB], v1[kB], v2[kB];
+    if (lane == 0 && (t >> 6) < 3) {  // one running sum each, in bin order, in place
+        constexpr int kB = 32;
+        double* v = sums[t >> 6];
+        double a = 0.0, x[kB], y[kB];
+        const int whole = N / (2 * kB) * (2 * kB);
+        auto read = [&](double* r, int i) {
 #pragma unroll
-            for (int u = 0; u < kB; ++u) { v0[u] = sw_[i + u]; v1[u] = swx_[i + u]; v2[u] = swx2_[i + u]; }
+            for (int u = 0; u < kB; ++u) r[u] = v[i + u];
+        };
+        auto add = [&](double* r, int i) {
 #pragma unroll
             for (int u = 0; u < kB; ++u) {
-                a0 = a0 + v0[u];
-                a1 = a1 + v1[u];
-                a2 = a2 + v2[u];
-                v0[u] = a0;
-                v1[u] = a1;
-                v2[u] = a2;
+                a = a + r[u];
+                r[u] = a;
             }
 #pragma unroll
-            for (int u = 0; u < kB; ++u) { sw_[i + u] = v0[u]; swx_[i + u] = v1[u]; swx2_[i + u] = v2[u]; }
+            for (int u = 0; u < kB; ++u) v[i + u] = r[u];
+        };
+        if (whole) read(x, 0);
+        for (int i = 0; i < whole; i += 2 * kB) {
+            read(y, i + kB);
+            add(x, i);
+            if (i + 2 * kB < whole) read(x, i + 2 * kB);
+            add(y, i + kB);
         }
-        for (; i < N; ++i) {
-            a0 = a0 + sw_[i];
-            a1 = a1 + swx_[i];
-            a2 = a2 + swx2_[i];
-            sw_[i] = a0;
-            swx_[i] = a1;
-            swx2_[i] = a2;
+        for (int i = whole; i < N; ++i) {
+            a = a + v[i];
+            v[i] = a;
         }
     }
     __syncthreads();
     for (int i = t; i <= N; i += kDpInitThreads) {
-        pw[i] = i ? sw_[i - 1] : 0.0;
-        pwx[i] = i ? swx_[i - 1] : 0.0;
-        pwx2[i] = i ? swx2_[i - 1] : 0.0;
+        pw[i] = i ? sums[0][i - 1] : 0.0;
+        pwx[i] = i ? sums[1][i - 1] : 0.0;
+        pwx2[i] = i ? sums[2][i - 1] : 0.0;
     }
     if (N > 0 && K <= N)  // dp[0][e]: no segmentation of e > 0 points into zero clusters
         for (int e = t; e <= N; e += kDpInitThreads) dp[e] = e ? __builtin_inf() : 0.0;
-    if (t != 0) return;
-    hdr[0] = N;
-    if (N == 0) { hdr[1] = 2; return; }
-    if (K > N) {  // quantization.py:68-81 padded codebook
-        for (int k = 0; k < K; ++k) out[k] = cw[k < N ? k : N - 1];
-        if (force) { out[0] = -1.0f; out[K - 1] = 1.0f; }
-        for (int i = 1; i < K; ++i) {  // insertion sort (ascending)
-            const float v = out[i];
-            int j = i - 1;
-            while (j >= 0 && out[j] > v) { out[j + 1] = out[j]; --j; }
-            out[j + 1] = v;
-        }
-        hdr[1] = 1;
-        return;
+    if (N > 0 && K > N) {  // quantization.py:68-81 padded codebook
+        if (t < K) sorted[t] = cw[t < N ? t : N - 1];
+        if (force && t == 0) sorted[0] = -1.0f;
+        if (force && t == K - 1) sorted[K - 1] = 1.0f;
+        __syncthreads();
+        sort_codewords(sorted, K, out, &unsorted);
     }
-    hdr[1] = 0;
+    if (t == 0) {
+        hdr[0] = N;
+        hdr[1] = N == 0 ? 2 : (K > N ? 1 : 0);
+        *reinterpret_cast<double*>(hdr + 2) = N ? kDpSlack * sums[0][N - 1] : 0.0;
+    }
 }
 static_assert(kDpMaxBins % kDpInitThreads == 0, "whole bins per thread");
+static_assert(kDpInitThreads >= kDpMaxK && kDpInitThreads / 64 >= 3, "one codeword per thread, a wave per sum");
 
 // One DP level (quantization.py:158-186): for every segment end e in [c, N],
 // the first start s in [c, e] minimising dp[c-1][s-1] + cost(s, e), in
 // float64 with the reference's expression order; strict < keeps the first
 // minimum, and the cross-lane reduction takes the lexicographic (cost, start)
-// minimum.  The prefix sums and the previous level are staged in LDS (4 x
-// (N + 1) doubles, 131 KB at N = 4096) and every candidate reads them from
-// there.  Wave p of the grid takes the ends c + p and N - p, whose candidate
-// counts add up to N - c + 2, so the waves carry equal work.
-constexpr int kDpThreads = 512;
+// minimum.
+//
+// A wave takes one end and looks at the starts from the nearest one down, 128 at
+// a time, until the cost of the segment alone exceeds the best candidate by
+// kDpSlack * sum(w).  In exact arithmetic a segment's cost never falls when it
+// grows and dp >= 0, so no start further down can be as good.  In float64 each of
+// the three prefix sums is within 4096 * 2^-53 * sum(w) of the exact sum (|x| < 1,
+// the terms themselves are exact), which moves a cost by less than 2^-38 sum(w) and a
+// dp value of up to 256 costs by less than 2^-30 sum(w); 2^-28 covers both with
+// room, and is still far below the costs it is compared with (5e-6 sum(w) for 256
+// even levels).  A count that is not finite gives an infinite or NaN slack, and
+// then nothing is cut.
+//
+// The optimal segment spans about N / c points, and the bound cuts at N / c^(2/3),
+// so most levels are one or two passes per end, bound by the launch and one trip to
+// memory.  256 codewords from 4096 full bins: 3.95 -> 1.71 ms (every start of every
+// end, from copies of the prefix sums in LDS: 14.7 us a level; now 6.3).
+constexpr int kDpThreads = 256;
 constexpr int kDpWaves = kDpThreads / 64;
-static_assert(4 * (kDpMaxBins + 1) * sizeof(double) <= 160 * 1024, "the staged arrays fit in the LDS of one CU");
+constexpr int kDpUnroll = 2;  // independent candidates per lane and pass (4: 2% slower over all levels)
 
-// Segment cost of starts s (prefix index s - 1) for end e: MODE 0 the
+// Segment cost of starts s (prefix index i = s - 1) for end e: MODE 0 the
 // free-centre cost sum_wx2 - sum_wx^2 / sum_w, MODE -1 / +1 the cost about
 // the fixed centre -1 / +1 (force_endpoints, first / last cluster).
 template <int MODE>
-__device__ __forceinline__ double dp_cost(double Pe, double PXe, double PX2e, const double* spw, const double* spwx,
-                                          const double* spwx2, int i) {
-    const double sw = Pe - spw[i];
-    const double swx = PXe - spwx[i];
-    const double swx2 = PX2e - spwx2[i];
+__device__ __forceinline__ double dp_cost(double sw, double swx, double swx2) {
     if (MODE == 0) {
         const double sq = swx * swx;
         return swx2 - sq / sw;
@@ -323,133 +370,189 @@ __device__ __forceinline__ double dp_cost(double Pe, double PXe, double PX2e, co
     return (swx2 - t1) + t2;
 }
 
-// Best start for end e over this lane's starts s = c + lane + 64 j, in
-// ascending order (strict < keeps the first minimum); kDpUnroll independent
-// candidates per iteration.
-#ifndef GEFEN_DP_UNROLL
-#define GEFEN_DP_UNROLL 4
-#endif
-constexpr int kDpUnroll = GEFEN_DP_UNROLL;
-template <int MODE>
-__device__ __forceinline__ void dp_scan(int e, int c, int lane, const double* spw, const double* spwx,
-                                        const double* spwx2, const double* sprev, double& best, int& bs) {
-    const double Pe = spw[e], PXe = spwx[e], PX2e = spwx2[e];
-    int s = c + lane;
-    for (; s + 64 * (kDpUnroll - 1) <= e; s += 64 * kDpUnroll) {
-        double cand[kDpUnroll];
-#pragma unroll
-        for (int u = 0; u < kDpUnroll; ++u) {
-            const int i = s + 64 * u - 1;
-            cand[u] = sprev[i] + dp_cost<MODE>(Pe, PXe, PX2e, spw, spwx, spwx2, i);
-        }
-#pragma unroll
-        for (int u = 0; u < kDpUnroll; ++u)
-            if (cand[u] < best) { best = cand[u]; bs = s + 64 * u; }
-    }
-    for (; s <= e; s += 64) {
-        const double cand = sprev[s - 1] + dp_cost<MODE>(Pe, PXe, PX2e, spw, spwx, spwx2, s - 1);
-        if (cand < best) { best = cand; bs = s; }
-    }
+template <int OFF>
+__device__ __forceinline__ double min_xor(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint64_t o = ((uint64_t)lane_xor<OFF>((uint32_t)(b >> 32)) << 32) | lane_xor<OFF>((uint32_t)b);
+    const double w = __builtin_bit_cast(double, o);
+    return w < v ? w : v;
+}
+__device__ __forceinline__ double wave_min_f64(double v) {
+    v = min_xor<1>(v);
+    v = min_xor<2>(v);
+    v = min_xor<4>(v);
+    v = min_xor<8>(v);
+    v = min_xor<16>(v);
+    return min_xor<32>(v);
 }
 
-__device__ __forceinline__ void dp_end(int e, int c, int K, int force, int lane, const double* spw, const double* spwx,
-                                       const double* spwx2, const double* sprev, double* dpc, int32_t* btc) {
-    double best = __builtin_inf();
-    int bs = -1;
-    if (force && c == 1) dp_scan<-1>(e, c, lane, spw, spwx, spwx2, sprev, best, bs);
-    else if (force && c == K) dp_scan<1>(e, c, lane, spw, spwx, spwx2, sprev, best, bs);
-    else dp_scan<0>(e, c, lane, spw, spwx, spwx2, sprev, best, bs);
-    for (int off = 32; off > 0; off >>= 1) {
-        const double ob = __shfl_xor(best, off, 64);
-        const int os = __shfl_xor(bs, off, 64);
-        if (os >= 0 && (bs < 0 || ob < best || (ob == best && os < bs))) { best = ob; bs = os; }
+// The operands of one pass: starts top - lane - 64 u (prefix indices), not below lo.
+struct DpPass {
+    double p[kDpUnroll], px[kDpUnroll], px2[kDpUnroll], prev[kDpUnroll];
+};
+struct DpArrays {
+    const double *__restrict__ pw, *__restrict__ pwx, *__restrict__ pwx2, *__restrict__ prev;
+};
+__device__ __forceinline__ DpPass dp_load(const DpArrays& A, int top, int lo, int lane) {
+    DpPass r;
+#pragma unroll
+    for (int u = 0; u < kDpUnroll; ++u) {
+        const int i = max(top - lane - 64 * u, lo);
+        r.p[u] = A.pw[i];
+        r.px[u] = A.pwx[i];
+        r.px2[u] = A.pwx2[i];
+        r.prev[u] = A.prev[i];
+    }
+    return r;
+}
+
+template <int MODE>
+__device__ __forceinline__ void dp_end(DpPass d, double Pe, double PXe, double PX2e, double slack, int top, int lo,
+                                       int lane, const DpArrays& A, double* dp_out, int32_t* bt_out) {
+    double best = __builtin_inf(), least;
+    int bi = -1;  // prefix index s - 1 of the best start
+    for (;;) {
+        double seg = 0.0;
+#pragma unroll
+        for (int u = 0; u < kDpUnroll; ++u) {
+            const int i = max(top - lane - 64 * u, lo);
+            seg = dp_cost<MODE>(Pe - d.p[u], PXe - d.px[u], PX2e - d.px2[u]);
+            const double cand = d.prev[u] + seg;
+            if (cand < best || (cand == best && bi >= 0 && i < bi)) { best = cand; bi = i; }
+        }
+        least = wave_min_f64(best);
+        // lane 63's last start is the lowest of this pass
+        const uint64_t bits = __builtin_bit_cast(uint64_t, seg);
+        const uint64_t low = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(bits >> 32), 63) << 32) |
+                             (uint32_t)__builtin_amdgcn_readlane((int)bits, 63);
+        top -= 64 * kDpUnroll;
+        if (top < lo || __builtin_bit_cast(double, low) > least + slack) break;
+        d = dp_load(A, top, lo, lane);
+    }
+    const bool mine = bi >= 0 && best == least;
+    const uint64_t who = __builtin_amdgcn_ballot_w64(mine);
+    int s = who ? __builtin_amdgcn_readlane(bi, (int)__builtin_ctzll(who)) : -1;
+    if (who & (who - 1)) {  // equal candidates in several lanes: the first start
+        uint32_t key = mine ? (uint32_t)bi : 0xffffffffu;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) key = min(key, (uint32_t)__shfl_xor((int)key, off, 64));
+        s = (int)key;
     }
     if (lane == 0) {
-        dpc[e] = bs >= 0 ? best : __builtin_inf();
-        btc[e] = bs;
+        *dp_out = s >= 0 ? least : __builtin_inf();
+        *bt_out = s >= 0 ? s + 1 : -1;
     }
 }
 
 __global__ __launch_bounds__(kDpThreads) void k_dp_level(int c, int K, int force, int bins, char* __restrict__ ws,
                                                          DpLayout L) {
-    __shared__ double spw[kDpMaxBins + 1], spwx[kDpMaxBins + 1], spwx2[kDpMaxBins + 1], sprev[kDpMaxBins + 1];
+    const int32_t* hdr = reinterpret_cast<const int32_t*>(ws);
+    const size_t stride = (size_t)bins + 1;
+    double* dp = reinterpret_cast<double*>(ws + L.dp);
+    int32_t* bt = reinterpret_cast<int32_t*>(ws + L.bt);
+    const DpArrays A{reinterpret_cast<const double*>(ws + L.pw), reinterpret_cast<const double*>(ws + L.pwx),
+                     reinterpret_cast<const double*>(ws + L.pwx2), dp + (size_t)(c - 1) * stride};
+    const int lane = threadIdx.x & 63;
+    // ends 1 .. N; the last level needs only N.  Everything an end's first pass reads
+    // is loaded before the header is looked at (the indices stay inside the arrays
+    // for any end up to bins), so it is one trip to memory.
+    const int e = c == K ? hdr[0] : (int)blockIdx.x * kDpWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + 1;
+    const int lo = c - 1, top = c == 1 ? 0 : max(e - 1, lo);  // with one cluster, only start 1 has a predecessor
+    double Pe = A.pw[e], PXe = A.pwx[e], PX2e = A.pwx2[e];
+    DpPass d = dp_load(A, top, lo, lane);
+    int N = hdr[0], status = hdr[1];
+    double slack = *reinterpret_cast<const double*>(hdr + 2);
+#pragma unroll
+    for (int u = 0; u < kDpUnroll; ++u) __asm__ volatile("" : "+v"(d.p[u]), "+v"(d.px[u]), "+v"(d.px2[u]), "+v"(d.prev[u]));
+    __asm__ volatile("" : "+v"(Pe), "+v"(PXe), "+v"(PX2e), "+v"(slack), "+v"(N), "+v"(status));
+    N = __builtin_amdgcn_readfirstlane(N);
+    if (__builtin_amdgcn_readfirstlane(status) != 0 || e > N) return;
+    double* dp_out = dp + (size_t)c * stride + e;
+    int32_t* bt_out = bt + (size_t)c * stride + e;
+    if (e < c) {  // no segmentation of e points into c clusters
+        if (lane == 0) {
+            *dp_out = __builtin_inf();
+            *bt_out = -1;
+        }
+        return;
+    }
+    if (force && c == 1) dp_end<-1>(d, Pe, PXe, PX2e, slack, top, lo, lane, A, dp_out, bt_out);
+    else if (force && c == K) dp_end<1>(d, Pe, PXe, PX2e, slack, top, lo, lane, A, dp_out, bt_out);
+    else dp_end<0>(d, Pe, PXe, PX2e, slack, top, lo, lane, A, dp_out, bt_out);
+}
+
+// jump[g][e]: where the backtrack stands after the kDpGroup levels K - 16 g ..
+// K - 16 g - 15, starting them at end e; -1 where it breaks off.  Walking K levels
+// one by one is K dependent loads (171 us for 256); the groups' walks run side by
+// side, and k_dp_backtrack then takes 16 jumps and 16 short walks (8 + 11 us).
+__global__ __launch_bounds__(256) void k_dp_jump(int K, int bins, char* __restrict__ ws, DpLayout L) {
     const int32_t* hdr = reinterpret_cast<const int32_t*>(ws);
     if (hdr[1] != 0) return;
     const int N = hdr[0];
     const size_t stride = (size_t)bins + 1;
-    const double* pw = reinterpret_cast<const double*>(ws + L.pw);
-    const double* pwx = reinterpret_cast<const double*>(ws + L.pwx);
-    const double* pwx2 = reinterpret_cast<const double*>(ws + L.pwx2);
-    double* dp = reinterpret_cast<double*>(ws + L.dp);
-    int32_t* bt = reinterpret_cast<int32_t*>(ws + L.bt);
-    const double* prev = dp + (size_t)(c - 1) * stride;
-    double* dpc = dp + (size_t)c * stride;
-    int32_t* btc = bt + (size_t)c * stride;
-    if (blockIdx.x == 0) {  // ends below c have no segmentation into c clusters
-        for (int e = threadIdx.x; e < c && e <= N; e += kDpThreads) {
-            dpc[e] = __builtin_inf();
-            btc[e] = -1;
-        }
+    const int32_t* bt = reinterpret_cast<const int32_t*>(ws + L.bt);
+    int32_t* jump = reinterpret_cast<int32_t*>(ws + L.jump);
+    const int g = blockIdx.y, top = K - g * kDpGroup;
+    // the first group starts at end N alone
+    const int first = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    const int e0 = g == 0 ? (first == 0 ? N : N + 1) : first;
+    if (e0 > N) return;
+    int e = e0;
+    for (int c = top; c > top - kDpGroup && c >= 1; --c) {
+        const int s = e >= c ? bt[(size_t)c * stride + e] : -1;
+        e = s - 1;
+        if (s < 1) { e = -1; break; }
     }
-    const int cnt = N - c + 1;  // ends c .. N
-    if (blockIdx.x > 0 && 2 * (int)blockIdx.x * kDpWaves >= cnt) return;  // no pair of ends here (uniform)
-    // indices c - 1 .. N of the four arrays (s - 1 >= c - 1, e <= N); every load of
-    // a thread is issued before its first LDS store, so the staging waits for one
-    // round trip to L2 instead of one per pass
-    constexpr int kStage = (kDpMaxBins + 1 + kDpThreads - 1) / kDpThreads;
-    double st[4][kStage];
-#pragma unroll
-    for (int r = 0; r < kStage; ++r) {
-        const int i = c - 1 + (int)threadIdx.x + r * kDpThreads;
-        if (i <= N) {
-            st[0][r] = pw[i];
-            st[1][r] = pwx[i];
-            st[2][r] = pwx2[i];
-            st[3][r] = prev[i];
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < kStage; ++r) {
-        const int i = c - 1 + (int)threadIdx.x + r * kDpThreads;
-        if (i <= N) {
-            spw[i] = st[0][r];
-            spwx[i] = st[1][r];
-            spwx2[i] = st[2][r];
-            sprev[i] = st[3][r];
-        }
-    }
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    for (int p = blockIdx.x * kDpWaves + (int)(threadIdx.x >> 6); 2 * p < cnt; p += gridDim.x * kDpWaves) {
-        dp_end(c + p, c, K, force, lane, spw, spwx, spwx2, sprev, dpc, btc);
-        if (N - p != c + p) dp_end(N - p, c, K, force, lane, spw, spwx, spwx2, sprev, dpc, btc);
-    }
+    jump[(size_t)g * stride + e0] = e;
 }
 
-__global__ void k_dp_backtrack(int K, int force, int bins, char* __restrict__ ws, DpLayout L,
-                               float* __restrict__ out) {
+__global__ __launch_bounds__(kDpMaxK) void k_dp_backtrack(int K, int force, int bins, char* __restrict__ ws, DpLayout L,
+                                                          float* __restrict__ out) {
+    __shared__ int ends[kDpMaxK + 1];  // ends[c]: last point of cluster c; ends[0]: where cluster 1 begins
+    __shared__ int start[kDpGroups];
+    __shared__ int broken, unsorted;
+    __shared__ float cbk[kDpMaxK];
     int32_t* hdr = reinterpret_cast<int32_t*>(ws);
-    if (threadIdx.x != 0 || hdr[1] != 0) return;
-    const int N = hdr[0];
+    if (hdr[1] != 0) return;
+    const int N = hdr[0], t = threadIdx.x;
     const size_t stride = (size_t)bins + 1;
     const double* pw = reinterpret_cast<const double*>(ws + L.pw);
     const double* pwx = reinterpret_cast<const double*>(ws + L.pwx);
     const int32_t* bt = reinterpret_cast<const int32_t*>(ws + L.bt);
-    int e = N;
-    for (int c = K; c >= 1; --c) {
-        const int s = bt[(size_t)c * stride + e];
-        if (s < 1) { hdr[1] = 3; return; }
-        if (force && c == 1) out[c - 1] = -1.0f;
-        else if (force && c == K) out[c - 1] = 1.0f;
-        else out[c - 1] = (float)((pwx[e] - pwx[s - 1]) / (pw[e] - pw[s - 1]));
-        e = s - 1;
+    const int32_t* jump = reinterpret_cast<const int32_t*>(ws + L.jump);
+    const int groups = (K + kDpGroup - 1) / kDpGroup;
+    if (t == 0) {
+        int e = N;
+        broken = 0;
+        for (int g = 0; g < groups; ++g) {
+            start[g] = e;
+            if (e < 0) broken = 1;
+            else e = jump[(size_t)g * stride + e];
+        }
+        if (e < 0) broken = 1;
     }
-    for (int i = 1; i < K; ++i) {
-        const float v = out[i];
-        int j = i - 1;
-        while (j >= 0 && out[j] > v) { out[j + 1] = out[j]; --j; }
-        out[j + 1] = v;
+    __syncthreads();
+    if (broken) {
+        if (t == 0) hdr[1] = 3;
+        return;
     }
+    if (t < groups) {
+        int e = start[t];
+        for (int c = K - t * kDpGroup; c > K - (t + 1) * kDpGroup && c >= 1; --c) {
+            ends[c] = e;
+            e = bt[(size_t)c * stride + e] - 1;
+            if (c == 1) ends[0] = e;
+        }
+    }
+    __syncthreads();
+    if (t < K) {
+        const int c = t + 1, e = ends[c], i = ends[c - 1];
+        if (force && c == 1) cbk[t] = -1.0f;
+        else if (force && c == K) cbk[t] = 1.0f;
+        else cbk[t] = (float)((pwx[e] - pwx[i]) / (pw[e] - pw[i]));
+    }
+    __syncthreads();
+    sort_codewords(cbk, K, out, &unsorted);
 }
 
 // ---------------------------------------------------------------------------
@@ -659,14 +762,18 @@ extern "C" int gefen_exact_dp(const float* counts, int bins, int codebook_size, 
                        ws, L, codebook_out);
     int rc = launch_status("gefen_exact_dp init");
     if (rc) return rc;
-    // enough waves for one pair of ends each at the largest level width (bins ends)
-    const int grid = bins / 2 >= kDpWaves ? (bins / 2 + kDpWaves - 1) / kDpWaves : 1;
+    // one wave per end (at most bins ends); the last level has one end
+    const int grid = (bins + kDpWaves - 1) / kDpWaves;
     for (int c = 1; c <= K; ++c) {
-        hipLaunchKernelGGL(k_dp_level, dim3(grid), dim3(kDpThreads), 0, st, c, K, force_endpoints ? 1 : 0, bins, ws, L);
+        hipLaunchKernelGGL(k_dp_level, dim3(c == K ? 1 : grid), dim3(c == K ? 64 : kDpThreads), 0, st, c, K,
+                           force_endpoints ? 1 : 0, bins, ws, L);
         rc = launch_status("gefen_exact_dp level");
         if (rc) return rc;
     }
-    hipLaunchKernelGGL(k_dp_backtrack, dim3(1), dim3(64), 0, st, K, force_endpoints ? 1 : 0, bins, ws, L,
+    hipLaunchKernelGGL(k_dp_jump, dim3(bins / 256 + 1, (K + kDpGroup - 1) / kDpGroup), dim3(256), 0, st, K, bins, ws, L);
+    rc = launch_status("gefen_exact_dp jump");
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_dp_backtrack, dim3(1), dim3(kDpMaxK), 0, st, K, force_endpoints ? 1 : 0, bins, ws, L,
                        codebook_out);
     return launch_status("gefen_exact_dp backtrack");
 }
