@@ -61,6 +61,8 @@ SIGNATURES = {
     "gefen_average_adjacent_log_block_mean_difference": (I32, [P, I32, I64, I64, I32, DBL, P, P]),
     "gefen_period_scores_workspace_size": (SZ, [I64, P, I32]),
     "gefen_period_scores": (I32, [P, I32, I64, P, I32, I32, DBL, P, P, P]),
+    "gefen_period_scores_tasks_workspace_size": (SZ, [P, I32]),
+    "gefen_period_scores_tasks": (I32, [P, I32, I32, DBL, P, P]),
     "gefen_average_within_block_variance": (I32, [P, I32, I64, I64, I32, P, P]),
     "gefen_average_within_block_coefficient_of_variation": (I32, [P, I32, I64, I64, I32, P, P]),
     "gefen_lloyd_accumulate": (I32, [P, I32, I64, I64, P, I32, P, P, P]),
@@ -90,6 +92,11 @@ MUON_APPLY_TASK = np.dtype([
     ("p", np.uint64), ("update", np.uint64), ("numel", np.int64), ("param_dtype", np.int32),
     ("transposed", np.int32), ("lr", np.float64), ("weight_decay", np.float64), ("adjusted_lr", np.float64),
 ])
+PERIOD_TASK = np.dtype([
+    ("values", np.uint64), ("divs", np.uint64), ("scores", np.uint64), ("numel", np.int64), ("dtype", np.int32),
+    ("ndiv", np.int32),
+])
+assert PERIOD_TASK.itemsize == 40
 assert STEP_TASK.itemsize == 128 and MUON_TASK.itemsize == 72 and MUON_APPLY_TASK.itemsize == 56
 
 _LIB = None

@@ -7,10 +7,12 @@ gradient in one call (one sync for all divisors).
 
 from __future__ import annotations
 
-from typing import Sequence
+from typing import List, Sequence
 
 import numpy as np
 import torch
+
+from gefen_amd import _lib
 
 from .gefen_hip import check, device_guard, dtype_code, load_extension, stream_of
 
@@ -147,3 +149,33 @@ def period_scores_launch(values: torch.Tensor, divisors: Sequence[int], mode: in
 def period_scores_workspace_bytes(numel: int, divisors: Sequence[int]) -> int:
     divs = np.ascontiguousarray(np.asarray(list(divisors), dtype=np.int64))
     return int(load_extension().gefen_period_scores_workspace_size(int(numel), divs.ctypes.data, divs.size))
+
+
+def period_scores_tasks(items, mode: int, epsilon: float) -> List[List[float]]:
+    """The scores of many flat gradients: items of (contiguous values, ascending
+    divisors), all on one device; a list of len(divisors) + 1 floats each (the last
+    is the invalid-input count).  One library call and one synchronisation."""
+    lib = load_extension()
+    dev = items[0][0].device
+    tasks = np.zeros(len(items), dtype=_lib.PERIOD_TASK)
+    offsets, arrays, total = [], {}, 0
+    for t, (v, divs) in zip(tasks, items):
+        if v.device != dev or not v.is_contiguous():
+            raise ValueError("Expected contiguous tensors on one device.")
+        d = arrays.get(tuple(divs))
+        if d is None:
+            d = arrays[tuple(divs)] = np.asarray(divs, dtype=np.int64)
+        t["values"], t["divs"], t["numel"] = v.data_ptr(), d.ctypes.data, v.numel()
+        t["dtype"], t["ndiv"] = dtype_code(v.dtype), d.size
+        offsets.append(total)
+        total += d.size + 1
+    scores = torch.empty(total, dtype=torch.float64, device=dev)
+    tasks["scores"] = scores.data_ptr() + 8 * np.asarray(offsets, dtype=np.uint64)
+    nbytes = int(lib.gefen_period_scores_tasks_workspace_size(tasks.ctypes.data, len(tasks)))
+    workspace = torch.empty(max(nbytes, 8), dtype=torch.uint8, device=dev)
+    with device_guard(scores):
+        rc = lib.gefen_period_scores_tasks(tasks.ctypes.data, len(tasks), int(mode), float(epsilon),
+                                           workspace.data_ptr(), stream_of(scores))
+    check(rc, "gefen_period_scores_tasks")
+    host = scores.cpu().tolist()  # the one synchronisation
+    return [host[o:o + len(divs) + 1] for o, (_, divs) in zip(offsets, items)]

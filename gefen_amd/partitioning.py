@@ -114,8 +114,8 @@ def _finalize_period_results(list_periods_and_scores: Sequence[Tuple[int, float]
 class PeriodScorer:
     """Scores the candidate divisors of many gradients with one host sync.
 
-    add() enqueues the device scoring of one flat gradient; finish() copies all
-    scores to the host once and returns the chosen period of each gradient."""
+    add() takes one flat gradient; finish() scores them all in one library call,
+    copies the scores to the host once and returns the chosen period of each."""
 
     def __init__(self, mode: int = 1, epsilon: float = 1e-12, min_num_blocks: int = DMNB):
         self.mode = mode
@@ -130,32 +130,16 @@ class PeriodScorer:
         return len(self.items) - 1
 
     def finish(self) -> List[int]:
-        from gefen_amd.kernels.period_variance import period_scores_launch, period_scores_workspace_bytes
+        from gefen_amd.kernels.period_variance import period_scores_tasks
 
-        work = [(i, f, d) for i, (f, d, _) in enumerate(self.items) if d]
+        work = [(i, f.detach().reshape(-1).contiguous(), d) for i, (f, d, _) in enumerate(self.items) if d]
         results: List[Optional[int]] = [None if d else 1 for (_, d, _) in self.items]
         if work:
-            dev = work[0][1].device
-            ws_bytes = max(period_scores_workspace_bytes(f.numel(), d) for _, f, d in work)
-            workspace = torch.empty(max(ws_bytes, 8), dtype=torch.uint8, device=dev)
-            offsets = []
-            total = 0
-            for _, f, d in work:
-                offsets.append(total)
-                total += len(d) + 1
-            scores = torch.empty(total, dtype=torch.float64, device=dev)
-            keep = []
-            for (i, f, d), off in zip(work, offsets):
-                flat = f.detach().reshape(-1).contiguous()
-                keep.append(flat)
-                period_scores_launch(flat, d, self.mode, self.epsilon, scores[off:off + len(d) + 1], workspace)
-            host = scores.cpu().tolist()  # the one synchronisation
-            del keep, workspace
-            for (i, f, d), off in zip(work, offsets):
-                if host[off + len(d)] > 0:
+            scores = period_scores_tasks([(f, d) for _, f, d in work], self.mode, self.epsilon)
+            for (i, f, d), s in zip(work, scores):
+                if s[-1] > 0:
                     raise ValueError("Expected values plus epsilon to be positive before log transform.")
-                pairs = list(zip(d, host[off:off + len(d)]))
-                results[i] = _finalize_period_results(pairs, self.items[i][2], f.numel(), 0.25)
+                results[i] = _finalize_period_results(list(zip(d, s)), self.items[i][2], f.numel(), 0.25)
         self.items = []
         return results  # type: ignore[return-value]
 

@@ -324,6 +324,22 @@ int gefen_period_scores(const void* values, int dtype, int64_t numel, const int6
                         int ndiv, int mode, double epsilon, double* scores, void* workspace,
                         gefen_stream_t stream);
 
+/* gefen_period_scores for many tensors at once (the per-parameter loop of
+ * gefen.py:882-924): task i's scores go to scores[0 .. ndiv] (device), its divisors
+ * are divs[0 .. ndiv) (host array, ascending).  Tensors of one size, dtype and list
+ * share launches.  workspace: gefen_period_scores_tasks_workspace_size() bytes. */
+typedef struct gefen_period_task {
+    const void* values;
+    const int64_t* divs;
+    double* scores;
+    int64_t numel;
+    int32_t dtype;
+    int32_t ndiv;
+} gefen_period_task;
+size_t gefen_period_scores_tasks_workspace_size(const gefen_period_task* tasks, int ntasks);
+int gefen_period_scores_tasks(const gefen_period_task* tasks, int ntasks, int mode, double epsilon, void* workspace,
+                              gefen_stream_t stream);
+
 /* Replace average_within_block_variance_cuda and
  * average_within_block_coefficient_of_variation_cuda (period_variance.py:12-124,
  * period_variance_kernel.cu:177-318).  out: variance -> out[0] = sqrt(mean of
