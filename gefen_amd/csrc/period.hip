@@ -4,17 +4,17 @@
 // m_j the mean of L over block j of p elements, score = mean_j |m_{j+1} - m_j|.
 // The logarithms and everything that is large happen in one pass over the
 // values (k_score_pass): a workgroup holds the logarithms of a chunk of Q elements
-// in LDS and forms the block sums and adjacent differences of every listed divisor
-// of Q there, each divisor from its largest listed divisor.  A second pass with
-// another Q takes small divisors that the first does not have.  The other divisors
-// are multiples of a pass's ones: their sums come from block sums that a pass
-// stored (k_score_derived).  k_score_final adds the parts up.  float64 throughout, in
+// in LDS and forms the block sums and adjacent differences of the small divisors
+// (up to kPassMax) there, each from its largest listed divisor.  Small divisors that
+// do not fit take another pass.  The others come from block sums that a pass stored
+// (k_score_derived), in two stages, and those that share too little with a pass from
+// the values (k_log_block_sums).  k_score_final adds the parts up.  float64 throughout, in
 // a fixed order, with no host synchronisation; the scores agree with numpy's
 // pairwise sums to ~1e-15 relative.
 // (One launch and one pass over stored sums per divisor, from the logarithms of all
 // elements written out, took 16 B of workspace per element and about 60 B of
-// traffic: all 25 divisors of 64M float32 values 1.18 ms, now 0.41, and GPT-2 124M's
-// 111 gradients 4400 launches, now 25.)
+// traffic: all 25 divisors of 64M float32 values 1.18 ms, now 0.27, and GPT-2 124M's
+// 111 gradients 4400 launches, now 40.)
 #include <math.h>
 #include <string.h>
 
@@ -115,8 +115,10 @@ __device__ const LogEntry kLogTable[128] = {
     {0x1.779081163d694p-1, 0x1.3d54fa657c000p-2}, {0x1.756cac1dbdd05p-1, 0x1.432ef2a6c0000p-2}
 };
 
+__device__ __forceinline__ bool table_log_takes(double y) {  // not zero, negative, subnormal, inf or NaN
+    return (uint32_t)(__builtin_bit_cast(uint64_t, y) >> 32) - 0x00100000u < 0x7fe00000u;
+}
 __device__ __forceinline__ double table_log(double y, const LogEntry* table) {
-    if (!(y >= 0x1p-1022 && y < __builtin_inf())) return log(y);  // zero, negative, subnormal, inf, NaN
     const uint64_t b = __builtin_bit_cast(uint64_t, y);
     const uint64_t t = b - 0x3fe6000000000000ull;
     const LogEntry E = table[(t >> 45) & 127];
@@ -135,8 +137,13 @@ __device__ __forceinline__ double table_log(double y, const LogEntry* table) {
 
 constexpr int kScoreThreads = 256;
 constexpr int kScoreBudget = 4096;  // float64 sums a chunk keeps in LDS (32 KB: four workgroups per CU)
-constexpr int kScoreItems = 24;     // divisors of one pass (one accumulator register pair each)
-constexpr int kScoreUnroll = 4;
+constexpr int kScoreChunk = 2048;   // elements of a chunk, at most
+constexpr int kScoreItems = 14;     // divisors of one pass (an accumulator and five scalars each)
+// Largest divisor that a pass forms itself: the next ones have too few blocks in a
+// chunk for a workgroup, and cost less from stored sums (all 25 divisors of 64M
+// float32 values: 411 us with every divisor of the chunk in the pass).
+constexpr int kPassMax = 48;
+constexpr int kScorePer = 8;        // elements of a chunk per thread, at most
 constexpr int kScoreTensors = 128;  // tensors of one launch (their addresses travel in the kernel arguments)
 
 // One pass: chunks of Q consecutive elements (the last one shorter, a multiple of
@@ -161,20 +168,21 @@ struct ScorePass {
     int64_t bad_off;     // per unit: elements with x + eps <= 0; -1 if another pass counts them
     double eps;
     int32_t q, tail;     // elements of a chunk, of the last one
-    int32_t nitems, chunks_per_unit, nunits, mode;
+    int32_t nitems, chunks_per_unit, nunits, pad;
     ScoreItem item[kScoreItems];
 };
 static_assert(sizeof(ScorePass) <= 4000, "kernel arguments are limited to 4 KB");
 
 // A unit of consecutive chunks per workgroup, carried over from chunk to chunk; the
-// differences between units are formed from the records.  Bound by the logarithms
-// (22 of about 45 vector instructions per element) and the LDS traffic of the
-// first few divisors.
-template <typename T>
+// differences between units are formed from the records.  Bound by instructions:
+// about 30 vector instructions per element for the logarithm and its input, and 40
+// for the sums and differences of six to fourteen divisors; the next chunk's loads
+// run meanwhile (without them 12% slower).  64M float32 values: 230 us.
+template <typename T, int MODE>
 __global__ __launch_bounds__(kScoreThreads, 4) void k_score_pass(const ScorePass P) {
     __shared__ __attribute__((aligned(16))) double S[kScoreBudget];
     __shared__ __attribute__((aligned(16))) LogEntry table[128];
-    __shared__ ScoreItem items[kScoreItems];  // from LDS, so that two dozen items' fields are not kept in registers
+    __shared__ ScoreItem items[kScoreItems];  // from LDS: kept in scalar registers they spill
     __shared__ double last[kScoreItems];
     __shared__ double red[kScoreItems + 1][kScoreThreads / 64];
     const int t = threadIdx.x;
@@ -188,24 +196,32 @@ __global__ __launch_bounds__(kScoreThreads, 4) void k_score_pass(const ScorePass
 #pragma unroll
     for (int k = 0; k < kScoreItems; ++k) acc[k] = 0.0;
     double bad = 0.0;
+    // the next chunk's elements are loaded while this one's sums are formed
+    T raw[kScorePer];
+    auto load = [&](int64_t c) {
+        const int len = c + 1 == P.nchunks ? P.tail : P.q;
+        const T* __restrict__ v = src + c * P.q;
+#pragma unroll
+        for (int u = 0; u < kScorePer; ++u) raw[u] = v[min(t + kScoreThreads * u, len - 1)];
+    };
+    load(c0);
     __syncthreads();
     for (int64_t c = c0; c < c1; ++c) {
-        const T* __restrict__ v = src + c * P.q;
         const bool tail = c + 1 == P.nchunks;
         const int len = tail ? P.tail : P.q;
-        for (int e = t; e < len; e += kScoreThreads * kScoreUnroll) {
-            T raw[kScoreUnroll];
 #pragma unroll
-            for (int u = 0; u < kScoreUnroll; ++u) raw[u] = v[min(e + kScoreThreads * u, len - 1)];
-#pragma unroll
-            for (int u = 0; u < kScoreUnroll; ++u) {
-                const double y = transform(raw[u], P.mode) + P.eps;
-                if (e + kScoreThreads * u < len) {
+        for (int u = 0; u < kScorePer; ++u) {
+            if (t + kScoreThreads * u < len) {
+                const double y = transform(raw[u], MODE) + P.eps;
+                double l = table_log(y, table);
+                if (!table_log_takes(y)) {
                     if (y <= 0.0) bad = bad + 1.0;  // numpy / the reference: NaN does not count
-                    S[e + kScoreThreads * u] = table_log(y, table);
+                    l = log(y);
                 }
+                S[t + kScoreThreads * u] = l;
             }
         }
+        if (c + 1 < c1) load(c + 1);
         int level = 0;
         for (int k = 1; k < P.nitems; ++k) {
             const ScoreItem I = items[k];
@@ -214,11 +230,16 @@ __global__ __launch_bounds__(kScoreThreads, 4) void k_score_pass(const ScorePass
                 level = I.level;
             }
             const int cnt = tail ? I.tail : I.count;
-            for (int j = t; j < cnt; j += kScoreThreads) {
-                const double* x = S + I.parent + j * I.ratio;
-                double s = x[0];
-                for (int u = 1; u < I.ratio; ++u) s = s + x[u];
-                S[I.at + j] = s;
+            if (I.ratio == 2) {
+                for (int j = t; j < cnt; j += kScoreThreads)
+                    S[I.at + j] = S[I.parent + 2 * j] + S[I.parent + 2 * j + 1];
+            } else {
+                for (int j = t; j < cnt; j += kScoreThreads) {
+                    const double* x = S + I.parent + j * I.ratio;
+                    double s = x[0];
+                    for (int u = 1; u < I.ratio; ++u) s = s + x[u];
+                    S[I.at + j] = s;
+                }
             }
         }
         __syncthreads();
@@ -261,11 +282,10 @@ __global__ __launch_bounds__(kScoreThreads, 4) void k_score_pass(const ScorePass
     if (t == kScoreItems && P.bad_off >= 0)
         ws[P.bad_off + blockIdx.x] = (red[t][0] + red[t][1]) + (red[t][2] + red[t][3]);
 }
-static_assert(kScoreThreads == 256, "four waves");
+static_assert(kScoreThreads == 256 && kScoreThreads * kScorePer == kScoreChunk, "four waves, a chunk in registers");
 
 // out[j] = sum of log(x + eps) over block j of p elements, from the values: for
-// periods beyond a chunk that share no useful divisor with one (a large prime
-// times little).  A wave per block; each lane sums its strided items in order,
+// divisors that share too little with a pass (multiples of a prime above kPassMax).  A wave per block; each lane sums its strided items in order,
 // then a butterfly.  `bad`: where blocks count x + eps <= 0, or null.
 template <typename T>
 __global__ __launch_bounds__(256) void k_log_block_sums(const T* __restrict__ src, int64_t nblocks, int64_t p, int mode,
@@ -280,28 +300,27 @@ __global__ __launch_bounds__(256) void k_log_block_sums(const T* __restrict__ sr
         for (int64_t j = lane; j < p; j += 64) {
             const double y = transform(v[j], mode) + eps;
             if (y <= 0.0) b = b + 1.0;
-            s = s + table_log(y, table);
+            s = s + (table_log_takes(y) ? table_log(y, table) : log(y));
         }
-        for (int off = 32; off > 0; off >>= 1) {
-            s = s + __shfl_xor(s, off, 64);
-            b = b + __shfl_xor(b, off, 64);
-        }
-        if (lane == 0) {
-            out[blk] = s;
-            if (bad) bad[blk] = b;
+        for (int off = 32; off > 0; off >>= 1) s = s + __shfl_xor(s, off, 64);
+        if (lane == 0) out[blk] = s;
+        if (bad) {
+            for (int off = 32; off > 0; off >>= 1) b = b + __shfl_xor(b, off, 64);
+            if (lane == 0) bad[blk] = b;
         }
     }
 }
 
 // Divisors summed from stored block sums: blocks of `ratio` entries of src, and the
 // sum of |S[j+1] - S[j]| of each workgroup's share of the differences.
-constexpr int kDerivedMax = 64;
+constexpr int kDerivedMax = 56;
 constexpr int kDerivedTile = 1024;  // block sums in LDS at a time
 struct DerivedItem {
     int64_t src;    // workspace offset of the source's sums
     int64_t ratio;  // source entries per block
     int64_t nblocks;
     int64_t part;   // workspace offset of this divisor's partial sums, one per workgroup
+    int64_t store;  // workspace offset of its block sums for a later stage, or -1
 };
 struct DerivedBatch {
     double* ws;
@@ -339,10 +358,21 @@ __global__ __launch_bounds__(256) void k_score_derived(const DerivedBatch B) {
             double x = 0.0;
             if (b <= m) {
                 const double* v = src + (d + b) * I.ratio;
-                for (int64_t j = lane & (lpr - 1); j < I.ratio; j += lpr) x = x + v[j];
+                int64_t j = lane & (lpr - 1);
+                if (I.ratio >= 8 * 64) {  // long blocks: eight loads in flight per lane
+                    double a[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+                    for (; j + 7 * 64 < I.ratio; j += 8 * 64)
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) a[u] = a[u] + v[j + 64 * u];
+                    x = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+                }
+                for (; j < I.ratio; j += lpr) x = x + v[j];
             }
             for (int off = lpr >> 1; off > 0; off >>= 1) x = x + __shfl_xor(x, off, 64);
-            if (b <= m && (lane & (lpr - 1)) == 0) sums[b] = x;
+            if (b <= m && (lane & (lpr - 1)) == 0) {
+                sums[b] = x;
+                if (I.store >= 0) ws[I.store + d + b] = x;  // a share's last block is its neighbour's first: the same value
+            }
         }
         __syncthreads();
         for (int j = threadIdx.x; j < m; j += 256) s = s + fabs(sums[j + 1] - sums[j]);
@@ -454,29 +484,21 @@ struct ValueSums { int64_t p, off, bad_off; };  // block sums straight from the 
 struct SizePlan {
     std::vector<PassPlan> pass;
     std::vector<ValueSums> value;
-    std::vector<DerivedItem> derived;
-    std::vector<int> derived_wgs;
+    std::vector<DerivedItem> derived[2];
+    std::vector<int> derived_wgs[2];
     std::vector<FinalItem> final;   // one per divisor, then the count
     int64_t total = 0;
 };
 
-int64_t gcd64(int64_t a, int64_t b) {
-    while (b) {
-        const int64_t r = a % b;
-        a = b;
-        b = r;
-    }
-    return a;
-}
+constexpr int64_t kUsefulSource = 6;    // stored sums of at least this many elements: 8 B written and read for each
+constexpr int64_t kStageOneMax = 1024;  // longer divisors are read from the first stage's sums where that is much less
 
-constexpr int64_t kUsefulSource = 32;  // stored sums over at least this many elements: 8 B per 32 elements to read
-
-// The pass over chunks that takes `need` (a divisor of n, at most half of
-// kScoreBudget) and the most of the open divisors: chunks are multiples of `need`
-// that divide n, whose small divisors' sums all fit in LDS.
+// The pass over chunks that takes `need` (a divisor of n, at most kPassMax) and the
+// most of the other open divisors up to kPassMax: their least common multiple q
+// divides n, and the sums of q elements fit in LDS.
 PassPlan choose_pass(int64_t n, int64_t need, const std::vector<int64_t>& divs, const std::vector<char>& open) {
     PassPlan best;
-    for (int64_t q = need; q <= kScoreBudget; q += need) {
+    for (int64_t q = need; q <= kScoreChunk; q += need) {
         if (n % q) continue;
         std::vector<int> list(1, 1);
         int64_t room = kScoreBudget - q;
@@ -484,26 +506,16 @@ PassPlan choose_pass(int64_t n, int64_t need, const std::vector<int64_t>& divs, 
             list.push_back((int)need);
             room -= q / need;
         }
-        bool fits = room >= 0;
-        for (size_t d = 0; d < divs.size() && fits && (int)list.size() < kScoreItems; ++d) {
+        for (size_t d = 0; d < divs.size() && divs[d] <= kPassMax && (int)list.size() < kScoreItems; ++d) {
             const int64_t p = divs[d];
-            if (p == 1 || p == need || !open[d] || q % p) continue;
-            if (q / p <= room) {
-                room -= q / p;
-                list.push_back((int)p);
-            } else if (p < kUsefulSource) {
-                fits = false;  // a small divisor left out would need a pass of its own
-            }
+            if (p == 1 || p == need || !open[d] || q % p || q / p > room) continue;
+            room -= q / p;
+            list.push_back((int)p);
         }
-        if (fits && list.size() >= best.p.size()) {  // equal: the longer chunk
+        if (list.size() > best.p.size()) {
             best.q = (int)q;
             best.p = list;
         }
-    }
-    if (best.q == 0) {
-        best.q = (int)need;
-        best.p.assign(1, 1);
-        if (need > 1) best.p.push_back((int)need);
     }
     std::sort(best.p.begin(), best.p.end());
     return best;
@@ -518,64 +530,44 @@ int make_plan(int64_t n, const int64_t* dv, int ndiv, SizePlan& P) {
     }
     const std::vector<int64_t> divs(dv, dv + ndiv);
     std::vector<char> open(ndiv, 1);
-    // the longest stored or storable sums that p is made of: (pass index, q) or (-1 - value index, q)
-    auto source = [&](int64_t p, int& where) {
-        int64_t best = 0;
-        for (size_t k = 0; k < P.pass.size(); ++k) {
-            const int64_t g = gcd64(p, P.pass[k].q);
-            if (g > best) { best = g; where = (int)k; }
-        }
-        for (size_t k = 0; k < P.value.size(); ++k)
-            if (p % P.value[k].p == 0 && P.value[k].p > best) { best = P.value[k].p; where = -1 - (int)k; }
-        return best;
-    };
     auto add_pass = [&](int64_t need) {
         PassPlan pass = choose_pass(n, need, divs, open);
         for (int d = 0; d < ndiv; ++d)
-            if (std::find(pass.p.begin(), pass.p.end(), (int64_t)divs[d]) != pass.p.end() && (divs[d] > 1 || P.pass.empty()))
-                open[d] = 0;
+            if (std::find(pass.p.begin(), pass.p.end(), divs[d]) != pass.p.end()) open[d] = 0;
         P.pass.push_back(pass);
     };
+    for (int d = 0; d < ndiv && divs[d] <= kPassMax; ++d)
+        if (open[d]) add_pass(divs[d]);
+    // The others, ascending: each from the longest block sums at hand that it is a
+    // multiple of.  Sums of a pass or from the values (stage 0) are read n / q at a
+    // time, so long ones from sums that the first stage forms.
+    struct Source { int kind; int at; int64_t q; };  // kind 0: a pass's item, 1: values, 2: a derived divisor
+    std::vector<Source> from(ndiv, Source{-1, 0, 0});
     for (int d = 0; d < ndiv; ++d) {
         if (!open[d]) continue;
         const int64_t p = divs[d];
-        int where = 0;
-        if (source(p, where) >= std::min(kUsefulSource, p)) continue;  // from stored sums, below
-        if (p <= kScoreBudget / 2) {
-            add_pass(p);
-            continue;
-        }
-        int64_t part = 1;  // the largest divisor of p that a chunk holds
-        for (int64_t q = kScoreBudget / 2; q > 1 && part == 1; --q)
-            if (p % q == 0) part = q;
-        if (part >= kUsefulSource) add_pass(part);
-        else P.value.push_back(ValueSums{p, 0, -1});
-    }
-    // which sums the open divisors read: one more item of a pass where it is not
-    // among its divisors
-    struct Want { int where; int64_t q; };
-    std::vector<Want> want(ndiv, Want{0, 0});
-    for (int d = 0; d < ndiv; ++d) {
-        if (!open[d]) continue;
-        int where = 0;
-        int64_t q = source(divs[d], where);
-        if (where >= 0) {
-            PassPlan& pass = P.pass[where];
-            int64_t room = kScoreBudget;
-            for (int p : pass.p) room -= pass.q / p;
-            if (std::find(pass.p.begin(), pass.p.end(), (int)q) == pass.p.end()) {
-                if ((int)pass.p.size() < kScoreItems && pass.q / q <= room) {
-                    pass.p.push_back((int)q);
-                    std::sort(pass.p.begin(), pass.p.end());
-                } else {  // no room: the longest listed divisor instead
-                    int64_t have = 1;
-                    for (int p : pass.p)
-                        if (divs[d] % p == 0) have = std::max<int64_t>(have, p);
-                    q = have;
-                }
+        Source best{-1, 0, 0}, late{-1, 0, 0};
+        for (size_t k = 0; k < P.pass.size(); ++k)
+            for (int q : P.pass[k].p)
+                if (p % q == 0 && q > best.q) best = Source{0, (int)k, q};
+        for (size_t k = 0; k < P.value.size(); ++k)
+            if (p % P.value[k].p == 0 && P.value[k].p > best.q) best = Source{1, (int)k, P.value[k].p};
+        for (int e = 0; e < d; ++e)
+            if (open[e] && from[e].kind < 2 && p % divs[e] == 0 && divs[e] > late.q) late = Source{2, e, divs[e]};
+        if (p > kStageOneMax && late.q >= 8 * std::max<int64_t>(best.q, 1)) best = late;
+        if (best.q < kUsefulSource) {
+            int64_t part = 1;  // a part of p that a pass can take, if none has
+            for (int64_t q = kPassMax; q >= kUsefulSource && part == 1; --q)
+                if (p % q == 0) part = q;
+            if (part > 1) {
+                P.pass.push_back(choose_pass(n, part, divs, open));
+                best = Source{0, (int)P.pass.size() - 1, part};
+            } else {
+                P.value.push_back(ValueSums{p, 0, -1});
+                best = Source{1, (int)P.value.size() - 1, p};
             }
         }
-        want[d] = Want{where, q};
+        from[d] = best;
     }
     // offsets
     int64_t o = 0;
@@ -592,7 +584,7 @@ int make_plan(int64_t n, const int64_t* dv, int ndiv, SizePlan& P) {
         int64_t sums = 0;
         for (int p : pass.p) sums += pass.q / p;
         const int64_t aim = std::max<int64_t>(512, n / 1024);
-        pass.times = (int)std::max<int64_t>(1, std::min({kScoreBudget / sums, (aim + pass.q - 1) / pass.q, n / pass.q}));
+        pass.times = (int)std::max<int64_t>(1, std::min({kScoreBudget / sums, (aim + pass.q - 1) / pass.q, n / pass.q, (int64_t)kScoreChunk / pass.q}));
         const int64_t len = (int64_t)pass.q * pass.times;
         pass.nchunks = (n + len - 1) / len;
         // about a thousand units, of up to 16 chunks
@@ -652,24 +644,28 @@ int make_plan(int64_t n, const int64_t* dv, int ndiv, SizePlan& P) {
         v.off = take(n / v.p);
         if (P.pass.empty() && k == 0) v.bad_off = take(n / v.p);
     }
+    std::vector<int> slot(ndiv, -1);  // of a first-stage divisor among P.derived[0]
     for (int d = 0; d < ndiv; ++d) {
         if (!open[d]) continue;
-        const int64_t p = divs[d], nb = n / p;
-        int64_t src;
-        if (want[d].where >= 0) {
-            PassPlan& pass = P.pass[want[d].where];
-            ScoreItem& it = pass.item[std::find(pass.p.begin(), pass.p.end(), (int)want[d].q) - pass.p.begin()];
-            if (it.store < 0) it.store = take(n / want[d].q);
-            src = it.store;
+        const int64_t p = divs[d], nb = n / p, q = from[d].q;
+        const int stage = from[d].kind == 2 ? 1 : 0;
+        int64_t* src;
+        if (from[d].kind == 0) {
+            PassPlan& pass = P.pass[from[d].at];
+            src = &pass.item[std::find(pass.p.begin(), pass.p.end(), (int)q) - pass.p.begin()].store;
+        } else if (from[d].kind == 1) {
+            src = &P.value[from[d].at].off;
         } else {
-            src = P.value[-1 - want[d].where].off;
+            src = &P.derived[0][slot[from[d].at]].store;
         }
-        // a workgroup for every 16384 source entries, no more than there are differences
-        const int64_t wgs = std::min<int64_t>(std::min<int64_t>(nb - 1, 1024), std::max<int64_t>(1, n / want[d].q / 16384));
-        DerivedItem it{src, p / want[d].q, nb, take(wgs)};
-        P.derived.push_back(it);
-        P.derived_wgs.push_back((int)wgs);
-        P.final[d] = FinalItem{it.part, (int32_t)wgs, 0, (double)p, (double)(nb - 1)};
+        if (*src < 0) *src = take(n / q);
+        // a workgroup for every 4096 source entries, no more than there are differences
+        const int64_t wgs = std::min<int64_t>(std::min<int64_t>(nb - 1, 1024), std::max<int64_t>(1, n / q / 4096));
+        const int64_t at = *src;
+        if (stage == 0) slot[d] = (int)P.derived[0].size();
+        P.derived[stage].push_back(DerivedItem{at, p / q, nb, take(wgs), -1});
+        P.derived_wgs[stage].push_back((int)wgs);
+        P.final[d] = FinalItem{P.derived[stage].back().part, (int32_t)wgs, 0, (double)p, (double)(nb - 1)};
     }
     if (!P.pass.empty()) P.final[ndiv] = FinalItem{P.pass[0].bad_off, P.pass[0].nunits, 0, 0.0, 0.0};
     else P.final[ndiv] = FinalItem{P.value[0].bad_off, (int32_t)std::min<int64_t>(n / P.value[0].p, INT32_MAX), 0, 0.0, 0.0};
@@ -678,8 +674,11 @@ int make_plan(int64_t n, const int64_t* dv, int ndiv, SizePlan& P) {
 }
 
 template <typename T>
-void launch_pass(const ScorePass& A, int ntensors, hipStream_t st) {
-    hipLaunchKernelGGL(k_score_pass<T>, dim3((unsigned)A.nunits, (unsigned)ntensors), dim3(kScoreThreads), 0, st, A);
+void launch_pass(const ScorePass& A, int mode, int ntensors, hipStream_t st) {
+    const dim3 grid((unsigned)A.nunits, (unsigned)ntensors), wg(kScoreThreads);
+    if (mode == 0) hipLaunchKernelGGL((k_score_pass<T, 0>), grid, wg, 0, st, A);
+    else if (mode == 1) hipLaunchKernelGGL((k_score_pass<T, 1>), grid, wg, 0, st, A);
+    else hipLaunchKernelGGL((k_score_pass<T, 2>), grid, wg, 0, st, A);
 }
 template <typename T>
 void launch_value_sums(const void* v, int64_t nblocks, int64_t p, int mode, double eps, double* out, double* bad,
@@ -707,11 +706,10 @@ int run_scores(const void* const* values, double* const* scores, int nt, int dty
         A.nitems = (int)pass.item.size();
         A.chunks_per_unit = pass.chunks_per_unit;
         A.nunits = pass.nunits;
-        A.mode = mode;
         for (size_t i = 0; i < pass.item.size(); ++i) A.item[i] = pass.item[i];
-        if (dtype == GEFEN_F32) launch_pass<float>(A, nt, st);
-        else if (dtype == GEFEN_BF16) launch_pass<bf16_t>(A, nt, st);
-        else launch_pass<f16_t>(A, nt, st);
+        if (dtype == GEFEN_F32) launch_pass<float>(A, mode, nt, st);
+        else if (dtype == GEFEN_BF16) launch_pass<bf16_t>(A, mode, nt, st);
+        else launch_pass<f16_t>(A, mode, nt, st);
         const int rc = launch_status("gefen period pass");
         if (rc) return rc;
     }
@@ -725,17 +723,18 @@ int run_scores(const void* const* values, double* const* scores, int nt, int dty
             const int rc = launch_status("gefen period block sums");
             if (rc) return rc;
         }
-    for (size_t first = 0; first < P.derived.size(); first += kDerivedMax) {
+    for (int stage = 0; stage < 2; ++stage)
+    for (size_t first = 0; first < P.derived[stage].size(); first += kDerivedMax) {
         DerivedBatch B;
         memset(&B, 0, sizeof(B));
         B.ws = ws;
         B.stride = stride;
-        B.count = (int)std::min<size_t>(kDerivedMax, P.derived.size() - first);
+        B.count = (int)std::min<size_t>(kDerivedMax, P.derived[stage].size() - first);
         int wg = 0;
         for (int i = 0; i < B.count; ++i) {
-            B.item[i] = P.derived[first + i];
+            B.item[i] = P.derived[stage][first + i];
             B.wg_begin[i] = wg;
-            wg += P.derived_wgs[first + i];
+            wg += P.derived_wgs[stage][first + i];
         }
         B.wg_begin[B.count] = wg;
         hipLaunchKernelGGL(k_score_derived, dim3((unsigned)wg, (unsigned)nt), dim3(256), 0, st, B);
