@@ -55,6 +55,7 @@ SIGNATURES = {
     "gefen_newton_schulz_workspace_size": (SZ, [I32, I32, I32]),
     "gefen_newton_schulz_apply": (I32, [P, I32, I32, I32, DBL, DBL, DBL, I32, DBL, P, P, P, P, P]),
     "gefen_exact_histogram": (I32, [P, I32, I64, I64, P, I32, P]),
+    "gefen_exact_histogram_tasks": (I32, [P, I32, P, I32, P, P]),
     "gefen_accumulate_counts": (I32, [P, P, I32, P]),
     "gefen_exact_dp_workspace_size": (SZ, [I32, I32]),
     "gefen_exact_dp": (I32, [P, I32, I32, I32, P, P, P]),
@@ -96,7 +97,10 @@ PERIOD_TASK = np.dtype([
     ("values", np.uint64), ("divs", np.uint64), ("scores", np.uint64), ("numel", np.int64), ("dtype", np.int32),
     ("ndiv", np.int32),
 ])
-assert PERIOD_TASK.itemsize == 40
+HISTOGRAM_TASK = np.dtype([
+    ("grad", np.uint64), ("numel", np.int64), ("period", np.int64), ("dtype", np.int32), ("pad", np.int32),
+])
+assert PERIOD_TASK.itemsize == 40 and HISTOGRAM_TASK.itemsize == 32
 assert STEP_TASK.itemsize == 128 and MUON_TASK.itemsize == 72 and MUON_APPLY_TASK.itemsize == 56
 
 _LIB = None

@@ -11,6 +11,9 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
+#include <vector>
+
 #include "capi_internal.h"
 #include "common.h"
 
@@ -122,43 +125,195 @@ __global__ __launch_bounds__(256) void k_prepare_codebook(const float* __restric
 }
 
 // ---------------------------------------------------------------------------
-// histogram: one lane group per block row, LDS-privatised counts per workgroup
-template <typename G>
-__global__ __launch_bounds__(256) void k_histogram(const G* __restrict__ g, int64_t nrows, int64_t period,
-                                                   int lpr_log2, int bins, float bw,
-                                                   unsigned long long* __restrict__ counts) {
-    __shared__ uint32_t h[4096];
-    for (int i = threadIdx.x; i < bins; i += 256) h[i] = 0;
+// histogram: a lane group per block row, LDS-privatised counts per workgroup, many
+// tensors per launch.
+constexpr int kHistTasks = 56;
+constexpr int kHistBins = 4096;
+constexpr int kHistMaxWgs = 1024;  // of one tensor
+struct HistTask {
+    const void* g;
+    unsigned long long* counts;
+    int64_t nrows;
+    int64_t rowlen;
+    int32_t nvec;      // vectors of W elements per row, the last one shifted back to end with the row
+    int32_t lpr_log2;  // lanes per row
+};
+struct HistBatch {
+    HistTask t[kHistTasks];
+    int32_t wg_begin[kHistTasks + 1];
+    int32_t ntasks;
+    int32_t bins;
+    int32_t pow2;      // bins is a power of two: dividing by the bin width is exact scaling by its reciprocal
+    float bw, scale;
+};
+static_assert(sizeof(HistBatch) <= 4000, "kernel arguments are limited to 4 KB");
+
+// clamp(floor((x + 1) / bw), 0, bins - 1), NaN -> 0 (its conversion to int64 is INT64_MIN)
+__device__ __forceinline__ int hist_bin(float x, const HistBatch& B) {
+    const float y = B.pow2 ? (x + 1.0f) * B.scale : (x + 1.0f) / B.bw;
+    return (int)fminf(fmaxf(y, 0.0f), (float)(B.bins - 1));
+}
+
+// A row's maximum as its elements are divided by it.  The quotient is Markstein's:
+// q = v * (1 / amax), x = q + (v - q amax) (1 / amax), which is the IEEE quotient
+// when 1 / amax is rounded correctly and v - q amax is exact; with amax >= 2^-60 that
+// holds for every v above 2^-86 (the subnormal bits reach 2^-149), and a smaller v
+// has |x| < 2^-26, whose bin does not depend on its last bits (x + 1 = 1).
+struct RowMax {
+    float amax, inv;
+    bool fast, positive;
+    __device__ __forceinline__ explicit RowMax(float m) : amax(m), inv(1.0f / m) {
+        fast = m >= 0x1p-60f && m <= 0x1p120f;
+        positive = m > 0.0f;  // NaN and zero maxima normalise to zero
+    }
+    __device__ __forceinline__ float divide(float v) const {
+        if (fast) {
+            const float q = v * inv;
+            return __builtin_fmaf(__builtin_fmaf(-q, amax, v), inv, q);
+        }
+        return positive ? v / amax : 0.0f;
+    }
+};
+
+__device__ __forceinline__ int hist_task(const HistBatch& B) {
+    int lo = 0, hi = B.ntasks - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (B.wg_begin[mid] <= (int)blockIdx.x) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// Rows of up to lanes * W * R elements, held in registers: read once, 16 bytes per
+// lane at any alignment.  R = 0: longer rows, a wave each, read twice.  Bound by
+// the LDS atomics and the instructions around them (about a dozen per element).
+// 64M float32 values in rows of 2048: 65 us (two reads and an IEEE division: 151).
+template <typename T, int W, int R>
+__global__ __launch_bounds__(256) void k_histogram(const HistBatch B) {
+    __shared__ uint32_t h[kHistBins];
+    for (int i = threadIdx.x; i < B.bins; i += 256) h[i] = 0;
     __syncthreads();
+    const int ti = hist_task(B);
+    const HistTask K = B.t[ti];
+    const T* __restrict__ g = static_cast<const T*>(K.g);
     const int lane = threadIdx.x & 63;
-    const int lpr = 1 << lpr_log2;
-    const int lir = lane & (lpr - 1);
-    const int64_t rpw = 64 >> lpr_log2;
-    const int64_t units = (nrows + rpw - 1) / rpw;
-    for (int64_t unit = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); unit < units;
-         unit += (int64_t)gridDim.x * 4) {
-        const int64_t row = unit * rpw + (lane >> lpr_log2);
-        const bool active = row < nrows;
-        const int64_t base = row * period;
-        float amax = 0.0f;
-        if (active)
-            for (int64_t j = lir; j < period; j += lpr) amax = nanmax(amax, fabsf(to_f32(g[base + j])));
-        amax = group_max(amax, lpr);
-        if (!active) continue;
-        for (int64_t j = lir; j < period; j += lpr) {
-            const float v = to_f32(g[base + j]);
-            const float x = (amax > 0.0f) ? v / amax : 0.0f;
-            const float y = floorf((x + 1.0f) / bw);
-            int b;
-            if (!(y >= 0.0f)) b = 0;  // negative, or NaN (-> INT64_MIN) clamps to 0
-            else if (y >= (float)(bins - 1)) b = bins - 1;
-            else b = (int)y;
-            atomicAdd(&h[b], 1u);
+    const int nwg = B.wg_begin[ti + 1] - B.wg_begin[ti];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t first = ((int64_t)blockIdx.x - B.wg_begin[ti]) * 4 + wave, step = (int64_t)nwg * 4;
+    if constexpr (R > 0) {
+        const int lpr = 1 << K.lpr_log2, lir = lane & (lpr - 1);
+        const int rpw = 64 >> K.lpr_log2;
+        const int64_t units = (K.nrows + rpw - 1) / rpw;
+        for (int64_t unit = first; unit < units; unit += step) {
+            const int64_t row = unit * rpw + (lane >> K.lpr_log2);
+            const bool active = row < K.nrows;
+            const T* __restrict__ src = g + (active ? row : K.nrows - 1) * K.rowlen;
+            AnyVec<T, W> v[R];
+            uint32_t key = 0;
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                const int64_t e = min((int64_t)min(lir + j * lpr, K.nvec - 1) * W, K.rowlen - W);
+                v[j] = *reinterpret_cast<const AnyVec<T, W>*>(src + e);
+            }
+#pragma unroll
+            for (int j = 0; j < R; ++j)
+#pragma unroll
+                for (int w = 0; w < W; ++w) key = max(key, abs_key(to_f32(v[j].v[w])));
+            const RowMax M(__uint_as_float(wave_group_max_u32(key, lpr)));
+            if (!active) continue;
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                const int q = lir + j * lpr;
+                if (q >= K.nvec) continue;
+                // elements of the last vector that the one before it has counted
+                const int skip = (int)max((int64_t)(q + 1) * W - K.rowlen, (int64_t)0);
+#pragma unroll
+                for (int w = 0; w < W; ++w)
+                    if (w >= skip) atomicAdd(&h[hist_bin(M.divide(to_f32(v[j].v[w])), B)], 1u);
+            }
+        }
+    } else {
+        for (int64_t row = first; row < K.nrows; row += step) {
+            const T* __restrict__ src = g + row * K.rowlen;
+            uint32_t key = 0;
+            for (int64_t j = lane; j < K.rowlen; j += 64) key = max(key, abs_key(to_f32(src[j])));
+            const RowMax M(__uint_as_float(wave_group_max_u32(key, 64)));
+            for (int64_t j = lane; j < K.rowlen; j += 64) atomicAdd(&h[hist_bin(M.divide(to_f32(src[j])), B)], 1u);
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < bins; i += 256)
-        if (h[i]) atomicAdd(&counts[i], (unsigned long long)h[i]);
+    for (int i = threadIdx.x; i < B.bins; i += 256)
+        if (h[i]) atomicAdd(&K.counts[i], (unsigned long long)h[i]);
+}
+
+// Rows of one element: x = v / |v| is -1, 1, 0 for a zero (or a NaN, whose maximum is
+// not positive) or NaN for an infinity: three bins, counted in registers (in LDS all
+// lanes' atomics would meet in two addresses).
+template <typename T, int W>
+__global__ __launch_bounds__(256) void k_histogram_signs(const HistBatch B) {
+    __shared__ uint32_t red[4][4];
+    const int ti = hist_task(B);
+    const HistTask K = B.t[ti];
+    const T* __restrict__ g = static_cast<const T*>(K.g);
+    const int64_t nwg = B.wg_begin[ti + 1] - B.wg_begin[ti];
+    const int64_t me = ((int64_t)blockIdx.x - B.wg_begin[ti]) * 256 + threadIdx.x;
+    uint32_t neg = 0, pos = 0, inf = 0, all = 0;
+    auto count = [&](float v) {
+        const uint32_t b = __float_as_uint(v), m = b & 0x7fffffffu;
+        const bool finite = m - 1u < 0x7f7fffffu;  // not zero, infinite or NaN
+        neg += finite && (b >> 31) ? 1u : 0u;
+        pos += finite && !(b >> 31) ? 1u : 0u;
+        inf += m == 0x7f800000u ? 1u : 0u;
+    };
+    const int64_t whole = K.nrows / W;
+    for (int64_t q = me; q < whole; q += nwg * 256) {
+        const AnyVec<T, W> v = *reinterpret_cast<const AnyVec<T, W>*>(g + q * W);
+#pragma unroll
+        for (int w = 0; w < W; ++w) count(to_f32(v.v[w]));
+        all += W;
+    }
+    if (me < K.nrows - whole * W) {
+        count(to_f32(g[whole * W + me]));
+        all += 1;
+    }
+    uint32_t c[4] = {neg, pos, inf, all};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        for (int off = 32; off > 0; off >>= 1) c[k] += (uint32_t)__shfl_xor((int)c[k], off, 64);
+        if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = c[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        auto total = [&](int k) { return (red[k][0] + red[k][1]) + (red[k][2] + red[k][3]); };
+        const uint32_t n = total(0), p = total(1), i = total(2), a = total(3);
+        const uint32_t mine = threadIdx.x == 0 ? n : threadIdx.x == 1 ? p : threadIdx.x == 2 ? i : a - n - p - i;
+        const float x = threadIdx.x == 0 ? -1.0f : threadIdx.x == 1 ? 1.0f : threadIdx.x == 2 ? __builtin_nanf("") : 0.0f;
+        if (mine) atomicAdd(&K.counts[hist_bin(x, B)], (unsigned long long)mine);
+    }
+}
+
+// acc[b] += float(counts[t][b]) for the tasks in order (gefen.py:331, 347, 365 sum in float32)
+__global__ __launch_bounds__(64) void k_accumulate_tasks(float* __restrict__ acc, const int64_t* __restrict__ counts,
+                                                         int ntasks, int bins) {
+    const int b = blockIdx.x * 64 + threadIdx.x;
+    if (b >= bins) return;
+    float a = acc[b];
+    int t = 0;
+    for (; t + 16 <= ntasks; t += 16) {
+        float c[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) c[u] = (float)counts[(int64_t)(t + u) * bins + b];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) a = a + c[u];
+    }
+    for (; t < ntasks; ++t) a = a + (float)counts[(int64_t)t * bins + b];
+    acc[b] = a;
+}
+
+__global__ __launch_bounds__(256) void k_zero_i64(int64_t* __restrict__ p, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) p[i] = 0;
 }
 
 __global__ void k_accumulate_counts(float* __restrict__ acc, const int64_t* __restrict__ counts, int bins) {
@@ -663,12 +818,6 @@ int grid_for_rows(int64_t units, int cap) {
     if (g > cap) g = cap;
     return (int)g;
 }
-int lpr_log2_for_len(int64_t len) {
-    int l = 0;
-    while ((1LL << l) < len && l < 6) ++l;
-    return l;
-}
-
 struct TempTables {
     void* ptr = nullptr;
     hipStream_t st = nullptr;
@@ -709,30 +858,114 @@ extern "C" int gefen_prepare_codebook(const float* codebook, int codebook_size, 
     return launch_status("gefen_prepare_codebook");
 }
 
+namespace gefen {
+namespace {
+// The kernel of a row length: signs for rows of one element, W = 1 for rows shorter
+// than a 16-byte vector, two vectors per lane up to half a wave's rows, eight up to
+// 64 lanes of them, else rows read twice.
+struct HistKind {
+    int w, r, lpr_log2, nvec;  // r = -1: signs
+};
+HistKind hist_kind(int dtype, int64_t rowlen) {
+    const int wide = dtype == GEFEN_F32 ? 4 : 8;
+    if (rowlen == 1) return {wide, -1, 0, 0};
+    const int w = rowlen < wide ? 1 : wide;
+    const int64_t nvec = (rowlen + w - 1) / w;
+    if (nvec > 64 * 8) return {1, 0, 6, 0};
+    const int r = w == 1 || nvec > 64 * 2 ? 8 : 2;
+    int l2 = 0;
+    while ((int64_t)r << l2 < nvec) ++l2;
+    return {w, r, l2, (int)nvec};
+}
+
+template <typename T, int WIDE>
+hipError_t launch_histogram(const HistKind& k, const HistBatch& b, int grid, hipStream_t st) {
+    if (k.r == -1) hipLaunchKernelGGL((k_histogram_signs<T, WIDE>), dim3(grid), dim3(256), 0, st, b);
+    else if (k.r == 0) hipLaunchKernelGGL((k_histogram<T, 1, 0>), dim3(grid), dim3(256), 0, st, b);
+    else if (k.w == 1) hipLaunchKernelGGL((k_histogram<T, 1, 8>), dim3(grid), dim3(256), 0, st, b);
+    else if (k.r == 2) hipLaunchKernelGGL((k_histogram<T, WIDE, 2>), dim3(grid), dim3(256), 0, st, b);
+    else hipLaunchKernelGGL((k_histogram<T, WIDE, 8>), dim3(grid), dim3(256), 0, st, b);
+    return hipGetLastError();
+}
+
+// Task i adds to counts + i * stride.
+int run_histograms(const gefen_histogram_task* tasks, int ntasks, int64_t* counts, int64_t stride, int bins,
+                   hipStream_t st) {
+    for (int i = 0; i < ntasks; ++i) {
+        const int rc = check_rows(tasks[i].grad, tasks[i].dtype, tasks[i].numel, tasks[i].period);
+        if (rc) return rc;
+    }
+    std::vector<char> done(ntasks, 0);
+    for (int i = 0; i < ntasks; ++i) {
+        if (done[i] || tasks[i].numel == 0) continue;
+        const HistKind kind = hist_kind(tasks[i].dtype, tasks[i].period);
+        HistBatch b;
+        memset(&b, 0, sizeof(b));
+        b.bins = bins;
+        b.bw = (float)(2.0 / (double)bins);
+        b.pow2 = (bins & (bins - 1)) == 0;
+        b.scale = (float)bins * 0.5f;
+        int64_t wg = 0;
+        for (int j = i; j < ntasks && b.ntasks < kHistTasks; ++j) {
+            const gefen_histogram_task& t = tasks[j];
+            if (done[j] || t.numel == 0 || t.dtype != tasks[i].dtype) continue;
+            const HistKind k = hist_kind(t.dtype, t.period);
+            if (k.w != kind.w || k.r != kind.r) continue;
+            HistTask& o = b.t[b.ntasks];
+            o.g = t.grad;
+            o.counts = reinterpret_cast<unsigned long long*>(counts + (int64_t)j * stride);
+            o.nrows = t.numel / t.period;
+            o.rowlen = t.period;
+            o.nvec = k.nvec;
+            o.lpr_log2 = k.lpr_log2;
+            b.wg_begin[b.ntasks++] = (int32_t)wg;
+            // every workgroup adds its counts to the tensor's at the end: no more of them
+            // than fill the chip, each with 16384 elements or more (signs: three sums)
+            wg += std::max<int64_t>(1, std::min<int64_t>(kHistMaxWgs, t.numel / 16384));
+            done[j] = 1;
+        }
+        b.wg_begin[b.ntasks] = (int32_t)wg;
+        hipError_t e;
+        if (tasks[i].dtype == GEFEN_F32) e = launch_histogram<float, 4>(kind, b, (int)wg, st);
+        else if (tasks[i].dtype == GEFEN_BF16) e = launch_histogram<bf16_t, 8>(kind, b, (int)wg, st);
+        else e = launch_histogram<f16_t, 8>(kind, b, (int)wg, st);
+        if (e != hipSuccess) return hip_status(e, "gefen_exact_histogram");
+    }
+    return GEFEN_OK;
+}
+}  // namespace
+}  // namespace gefen
+
 extern "C" int gefen_exact_histogram(const void* grad, int grad_dtype, int64_t numel, int64_t period,
                                      int64_t* bin_counts, int bins, gefen_stream_t stream) {
     int rc = check_rows(grad, grad_dtype, numel, period);
     if (rc) return rc;
-    if (bins <= 0 || bins > 4096) return fail_inval("Expected histogram bins in [1, 4096], got %d", bins);
+    if (bins <= 0 || bins > kHistBins) return fail_inval("Expected histogram bins in [1, 4096], got %d", bins);
     if (!bin_counts) return fail_inval("null bin_counts");
-    if (numel == 0) return GEFEN_OK;
-    const int64_t nrows = numel / period;
-    const int l2 = lpr_log2_for_len(period);
-    const int64_t units = (nrows + (64 >> l2) - 1) / (64 >> l2);
-    const int grid = grid_for_rows(units, 2048);
-    const float bw = (float)(2.0 / (double)bins);
+    gefen_histogram_task t;
+    memset(&t, 0, sizeof(t));
+    t.grad = grad;
+    t.numel = numel;
+    t.period = period;
+    t.dtype = grad_dtype;
+    return run_histograms(&t, 1, bin_counts, 0, bins, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int gefen_exact_histogram_tasks(const gefen_histogram_task* tasks, int ntasks, float* acc, int bins,
+                                           int64_t* counts, gefen_stream_t stream) {
+    if (ntasks < 0 || (ntasks > 0 && !tasks)) return fail_inval("invalid task array");
+    if (bins <= 0 || bins > kHistBins) return fail_inval("Expected histogram bins in [1, 4096], got %d", bins);
+    if (ntasks == 0) return GEFEN_OK;
+    if (!acc || !counts) return fail_inval("null pointer");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    auto* cnt = reinterpret_cast<unsigned long long*>(bin_counts);
-    if (grad_dtype == GEFEN_F32)
-        hipLaunchKernelGGL(k_histogram<float>, dim3(grid), dim3(256), 0, st, static_cast<const float*>(grad), nrows,
-                           period, l2, bins, bw, cnt);
-    else if (grad_dtype == GEFEN_BF16)
-        hipLaunchKernelGGL(k_histogram<bf16_t>, dim3(grid), dim3(256), 0, st, static_cast<const bf16_t*>(grad), nrows,
-                           period, l2, bins, bw, cnt);
-    else
-        hipLaunchKernelGGL(k_histogram<f16_t>, dim3(grid), dim3(256), 0, st, static_cast<const f16_t*>(grad), nrows,
-                           period, l2, bins, bw, cnt);
-    return launch_status("gefen_exact_histogram");
+    const int64_t n = (int64_t)ntasks * bins;
+    hipLaunchKernelGGL(k_zero_i64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, counts, n);
+    int rc = launch_status("gefen_exact_histogram_tasks (zero)");
+    if (rc) return rc;
+    rc = run_histograms(tasks, ntasks, counts, bins, bins, st);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_accumulate_tasks, dim3((bins + 63) / 64), dim3(64), 0, st, acc, counts, ntasks, bins);
+    return launch_status("gefen_exact_histogram_tasks (sum)");
 }
 
 extern "C" int gefen_accumulate_counts(float* acc, const int64_t* counts, int bins, gefen_stream_t stream) {

@@ -202,28 +202,20 @@ def learn_gefen_exact_codebook_from_grad_periods(*, grad_periods, codebook_devic
                 raise ValueError(
                     "Gefen exact codebook learning does not support SAVE_CODEBOOK_PREFIX exports. "
                     "Disable exports or use a non-exact research path outside the publishable Gefen optimizer.")
-    from gefen_amd.kernels.exact_histogram_fused import gefen_exact_histogram_cuda
+    from gefen_amd.kernels.exact_histogram_fused import accumulate_histograms
 
     bins = num_codebooks * 16
-    lib = _lib.load()
-    acc = None
-    local = None
+    items = []
     total = 0
     for _, flat, period, _ in grad_periods:
         if flat.device.type != "cuda":
             raise ValueError("gefen_amd learns the codebook from HIP device gradients, got {}".format(flat.device))
-        if acc is None:
-            acc = torch.zeros(bins, dtype=torch.float32, device=flat.device)
-            local = torch.zeros(bins, dtype=torch.int64, device=flat.device)
-        else:
-            local.zero_()
-        gefen_exact_histogram_cuda(flat, period, local)
-        with torch.cuda.device(flat.device):
-            _lib.check(lib.gefen_accumulate_counts(acc.data_ptr(), local.data_ptr(), bins,
-                                                   torch.cuda.current_stream(flat.device).cuda_stream))
+        items.append((flat if not items else flat.to(items[0][0].device), period))
         total += flat.numel()
     if total == 0:
         return None
+    acc = torch.zeros(bins, dtype=torch.float32, device=items[0][0].device)
+    accumulate_histograms(items, acc)
     codebook = quantization_module.exact_dp_from_counts(acc, num_codebooks, force_endpoints).to(codebook_device)
     if verbose and compute_mse_logging:
         edges = torch.linspace(-1.0, 1.0, steps=bins + 1, dtype=torch.float32)
@@ -788,22 +780,14 @@ class Gefen(torch.optim.Optimizer):
             raise ValueError("LIST_STEPS_SAVE_HIST_GRAD requires SAVE_CODEBOOK_PREFIX to be set.")
         if self._gefen_codebook is None:
             raise ValueError("Expected Gefen codebook to be initialized before saving gradient histogram.")
-        from gefen_amd.kernels.exact_histogram_fused import gefen_exact_histogram_cuda
+        from gefen_amd.kernels.exact_histogram_fused import accumulate_histograms
 
-        bins = self._gefen_codebook.numel() * 16
-        lib = _lib.load()
-        acc = None
-        total = 0
-        for _, flat, period, _ in self._iter_gefen_grad_periods(reuse_existing_periods=True):
-            if acc is None:
-                acc = torch.zeros(bins, dtype=torch.float32, device=flat.device)
-            local = torch.zeros(bins, dtype=torch.int64, device=flat.device)
-            gefen_exact_histogram_cuda(flat, period, local)
-            _lib.check(lib.gefen_accumulate_counts(acc.data_ptr(), local.data_ptr(), bins,
-                                                   torch.cuda.current_stream(flat.device).cuda_stream))
-            total += flat.numel()
+        items = [(flat, period) for _, flat, period, _ in self._iter_gefen_grad_periods(reuse_existing_periods=True)]
+        total = sum(flat.numel() for flat, _ in items)
         if total == 0:
             raise ValueError("Cannot save Gefen gradient histogram because no gradients were available.")
+        acc = torch.zeros(self._gefen_codebook.numel() * 16, dtype=torch.float32, device=items[0][0].device)
+        accumulate_histograms(items, acc)
         quantization_module.save_distribution_histogram_pt_from_counts(
             hist=acc.cpu(), prefix=prefix, suffix="grad_hist_step_{}".format(self._gefen_global_step),
             num_samples=total)

@@ -2,7 +2,10 @@
 
 from __future__ import annotations
 
+import numpy as np
 import torch
+
+from gefen_amd import _lib
 
 from .gefen_hip import check, device_guard, dtype_code, load_extension, stream_of
 
@@ -36,3 +39,27 @@ def gefen_exact_histogram_cuda(grad_flat: torch.Tensor, period: int, bin_counts:
         rc = lib.gefen_exact_histogram(g.data_ptr(), dtype_code(g.dtype), g.numel(), int(period),
                                        bin_counts.data_ptr(), bin_counts.numel(), stream_of(g))
     check(rc, "gefen_exact_histogram_cuda")
+
+
+def accumulate_histograms(items, acc: torch.Tensor) -> None:
+    """acc (float32, one entry per bin) += float32(histogram) of each (flat gradient,
+    period) of items in order (gefen.py:331-366), in a few launches; the gradients are
+    on acc's device."""
+    lib = load_extension()
+    tasks = np.zeros(len(items), dtype=_lib.HISTOGRAM_TASK)
+    keep = []
+    for t, (flat, period) in zip(tasks, items):
+        if flat.dim() != 1:
+            raise ValueError("Expected grad_flat to be 1D, got dim={}".format(flat.dim()))
+        if period <= 0:
+            raise ValueError("Expected period to be positive, got {}".format(period))
+        if flat.numel() % period != 0:
+            raise ValueError("Expected grad_flat.numel()={} to be divisible by period={}.".format(flat.numel(), period))
+        g = flat.contiguous()
+        keep.append(g)
+        t["grad"], t["numel"], t["period"], t["dtype"] = g.data_ptr(), g.numel(), int(period), dtype_code(g.dtype)
+    counts = torch.empty(len(items) * acc.numel(), dtype=torch.int64, device=acc.device)
+    with device_guard(acc):
+        rc = lib.gefen_exact_histogram_tasks(tasks.ctypes.data, len(tasks), acc.data_ptr(), acc.numel(),
+                                             counts.data_ptr(), stream_of(acc))
+    check(rc, "gefen_exact_histogram_tasks")

@@ -294,6 +294,20 @@ int gefen_newton_schulz_apply(const void* x, int batch, int rows, int cols, doub
 int gefen_exact_histogram(const void* grad, int grad_dtype, int64_t numel, int64_t period,
                           int64_t* bin_counts, int bins, gefen_stream_t stream);
 
+/* The histograms of many tensors and their fp32 sum (the loop of gefen.py:331-366):
+ * counts (ntasks * bins int64 of device memory, set by the call) receives each
+ * task's histogram, and acc[b] = f32(acc[b] + f32(counts[i][b])) over the tasks in
+ * order. */
+typedef struct gefen_histogram_task {
+    const void* grad;
+    int64_t numel;
+    int64_t period;
+    int32_t dtype;
+    int32_t pad;
+} gefen_histogram_task;
+int gefen_exact_histogram_tasks(const gefen_histogram_task* tasks, int ntasks, float* acc, int bins, int64_t* counts,
+                                gefen_stream_t stream);
+
 /* acc[b] = f32(acc[b] + f32(counts[b])): the fp32 host accumulation of
  * gefen.py:331, 347 performed on the device. */
 int gefen_accumulate_counts(float* acc, const int64_t* counts, int bins, gefen_stream_t stream);
