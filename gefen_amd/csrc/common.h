@@ -148,6 +148,28 @@ __device__ __forceinline__ void vstore32_nt(T* base, uint32_t elem, const Vec<T,
     __builtin_nontemporal_store(r, reinterpret_cast<R*>(reinterpret_cast<char*>(base) + off));
 }
 
+// The same at the alignment of one element.
+template <int BYTES, int ALIGN> struct RawAny {
+    typedef typename RawVec<BYTES>::type type __attribute__((aligned(ALIGN)));
+};
+template <typename T, int W>
+__device__ __forceinline__ Vec<T, W> vload32_nt_any(const T* base, uint32_t elem) {
+    using R = typename RawAny<sizeof(T) * W, sizeof(T)>::type;
+    const uint32_t off = elem * (uint32_t)sizeof(T);
+    const auto r = __builtin_nontemporal_load(reinterpret_cast<const R*>(reinterpret_cast<const char*>(base) + off));
+    Vec<T, W> x;
+    __builtin_memcpy(&x, &r, sizeof(x));
+    return x;
+}
+template <typename T, int W>
+__device__ __forceinline__ void vstore32_nt_any(T* base, uint32_t elem, const Vec<T, W>& x) {
+    using R = typename RawAny<sizeof(T) * W, sizeof(T)>::type;
+    const uint32_t off = elem * (uint32_t)sizeof(T);
+    typename RawVec<sizeof(T) * W>::type r;
+    __builtin_memcpy(&r, &x, sizeof(r));
+    __builtin_nontemporal_store(r, reinterpret_cast<R*>(reinterpret_cast<char*>(base) + off));
+}
+
 // ----------------------------------------------------------------- wave reductions
 // Butterfly over groups of `width` lanes (width a power of two <= 64).
 __device__ __forceinline__ float group_max(float v, int width) {

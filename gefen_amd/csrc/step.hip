@@ -372,8 +372,14 @@ int make_step_task(const gefen_step_task& in, int mode, const float* stepsize, P
     if (p1 && rowlen > 256 * 64) return fail_inval("period_one_divisor %lld is too large", (long long)rowlen);
     if (P > INT32_MAX) return fail_inval("period %lld is too large", (long long)P);
     const int dsz = dtype_size(in.param_dtype), ssz = dtype_size(in.state_dtype);
-    const int W = pick_width(dsz, rowlen, {in.p, in.grad}, 1, in.m_codebook, ssz, p1 ? in.vmean : nullptr);
-    const int64_t nvec = rowlen / W;
+    int W = pick_width(dsz, rowlen, {in.p, in.grad}, 1, in.m_codebook, ssz, p1 ? in.vmean : nullptr);
+    // rows of at least one wide vector that aligned accesses would take one element
+    // at a time: wide vectors at any alignment, the last one shifted back
+    const int wide = dsz == 2 ? 8 : 4;
+    const bool rag = W == 1 && rowlen >= wide;
+    if (rag && p1 && rowlen > 256) return fail_inval("period_one_divisor %lld is too large", (long long)rowlen);
+    if (rag) W = wide;
+    const int64_t nvec = (rowlen + W - 1) / W;
     // period-one rows (at most 256 * 64 elements) take half the lanes with
     // twice the vectors per lane: more bytes in flight per lane
     int l2 = lpr_log2_for(nvec);
@@ -384,7 +390,7 @@ int make_step_task(const gefen_step_task& in, int mode, const float* stepsize, P
     const int tab = (R != 0 && l2 >= 5 && !p1) ? 1 : 0;
     // the kernels keep one row table per wave when R >= 2 (whole-wave rows)
     if (tab && R >= 2 && l2 != 6) return fail_inval("internal: row tables of a %d-lane row", 1 << l2);
-    Key k{in.param_dtype, in.state_dtype, R == 0 ? 1 : W, R, p1 ? 1 : 0, tab};
+    Key k{in.param_dtype, in.state_dtype, R == 0 ? 1 : W, R, p1 ? 1 : 0, tab, rag && R != 0};
     StepTask& t = out.task;
     memset(&t, 0, sizeof(t));
     t.p = in.p;
@@ -922,7 +928,7 @@ extern "C" int gefen_step_plan_create(const gefen_step_task* tasks, int ntasks, 
             if (rc == GEFEN_OK) {
                 P->pend.push_back(ps);
                 P->row.push_back(i);
-                P->galign.push_back((ps.key.R == 0 ? 1 : ps.key.W) * dtype_size(ps.key.d));
+                P->galign.push_back((ps.key.R == 0 || ps.key.rag ? 1 : ps.key.W) * dtype_size(ps.key.d));
             }
         }
         if (rc) {

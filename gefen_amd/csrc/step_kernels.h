@@ -65,15 +65,29 @@ constexpr int kStepThreads = 64 * kStepWaves;
 
 constexpr bool kStreamNT = GEFEN_STEP_NT != 0;  // non-temporal loads / stores of the streamed tensors
 
-template <typename T, int W>
+// ANY: at the alignment of one element (the same accesses; gfx950 takes any alignment).
+template <typename T, int W, bool ANY = false>
 __device__ __forceinline__ Vec<T, W> sload(const T* base, uint32_t elem) {
-    if constexpr (kStreamNT) return vload32_nt<T, W>(base, elem);
+    if constexpr (ANY) return vload32_nt_any<T, W>(base, elem);
+    else if constexpr (kStreamNT) return vload32_nt<T, W>(base, elem);
     else return vload32<T, W>(base, elem);
 }
-template <typename T, int W>
+template <typename T, int W, bool ANY = false>
 __device__ __forceinline__ void sstore(T* base, uint32_t elem, const Vec<T, W>& x) {
-    if constexpr (kStreamNT) vstore32_nt<T, W>(base, elem, x);
+    if constexpr (ANY) vstore32_nt_any<T, W>(base, elem, x);
+    else if constexpr (kStreamNT) vstore32_nt<T, W>(base, elem, x);
     else vstore32<T, W>(base, elem, x);
+}
+
+// First element of vector v of a row.  RAG: rows that are no whole number of
+// vectors, or are not aligned for them: the last vector is shifted back to end with
+// the row, so some elements are in two vectors.  Both lanes load the old values
+// before either stores (every load of a row precedes its stores in the wave), form
+// the same results and store the same bytes; only the sum of squares leaves the
+// repeats out.
+template <bool RAG, int W>
+__device__ __forceinline__ int vec_first(int v, int64_t rowlen) {
+    return RAG ? min(v * W, (int)rowlen - W) : v * W;
 }
 constexpr int kMaxBatch = 30;  // tasks per launch (the task table is the kernel argument block, < 4 KB)
 
@@ -306,7 +320,7 @@ __device__ __forceinline__ int nearest_one_probe(float x, const float* thr, cons
 // in-row vectors of active rows are stored.  WD: weight decay
 // (gefen.py:1280-1281) is applied to the parameter first.  root: the LDS
 // square-root table of a period-one bf16 state, or nullptr.
-template <typename D, typename S, int W, int R, bool P1, bool TAB, int PROBES, bool WD, bool FINE, typename UF>
+template <typename D, typename S, int W, int R, bool P1, bool TAB, bool RAG, int PROBES, bool WD, bool FINE, typename UF>
 __device__ __forceinline__ void step_sweep2(const StepTask& T, const LdsTables<FINE>& L, const float* utab,
                                             const float* root, const UF& upd_of, const Vec<D, W> (&gv)[R],
                                             const Vec<D, W> (&pv)[R], const Vec<S, W> (&vv)[R], uint8_t* idx, D* p,
@@ -378,10 +392,10 @@ __device__ __forceinline__ void step_sweep2(const StepTask& T, const LdsTables<F
         }
         const int v = lir + j * lpr;
         if (active && v < T.nvec) {
-            const uint32_t e = base + (uint32_t)(v * W);
-            sstore<uint8_t, W>(idx, e, io);
-            sstore<D, W>(p, e, po);
-            if (P1) sstore<S, W>(vm, e, vo);
+            const uint32_t e = base + (uint32_t)vec_first<RAG, W>(v, T.rowlen);
+            sstore<uint8_t, W, RAG>(idx, e, io);
+            sstore<D, W, RAG>(p, e, po);
+            if (P1) sstore<S, W, RAG>(vm, e, vo);
         }
     }
 }
@@ -395,7 +409,11 @@ __device__ __forceinline__ void step_sweep2(const StepTask& T, const LdsTables<F
 // reads the last row, a vector past the row end reads the row's last vector,
 // so each lane has all of its row's bytes in flight at once.  Absmax is
 // idempotent under such copies; the sum of squares masks them out.
-template <typename D, typename S, int W, int R, bool P1, bool TAB>
+//
+// RAG: see vec_first.  Odd rows took one element per lane and load before: 30000
+// period-one rows of 250 bf16 elements (53 MB) went from 53 to 31 us, and rows of
+// 513 to 4096 elements left the two-sweep kernel.
+template <typename D, typename S, int W, int R, bool P1, bool TAB, bool RAG>
 __global__ __launch_bounds__(kStepThreads) void k_gefen_step(const StepBatch B) {
     constexpr bool kRoot = P1 && std::is_same<S, bf16_t>::value;
     // 16-bit parameters search the fine bucket with one probe where the codebook
@@ -456,11 +474,11 @@ __global__ __launch_bounds__(kStepThreads) void k_gefen_step(const StepBatch B) 
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             const int v = min(lir + j * lpr, T.nvec - 1);
-            const uint32_t e = base + (uint32_t)(v * W);
-            gv[j] = sload<D, W>(g, e);
-            iv[j] = sload<uint8_t, W>(idx, e);
-            pv[j] = sload<D, W>(p, e);
-            if (P1) vv[j] = sload<S, W>(vm, e);
+            const uint32_t e = base + (uint32_t)vec_first<RAG, W>(v, T.rowlen);
+            gv[j] = sload<D, W, RAG>(g, e);
+            iv[j] = sload<uint8_t, W, RAG>(idx, e);
+            pv[j] = sload<D, W, RAG>(p, e);
+            if (P1) vv[j] = sload<S, W, RAG>(vm, e);
         }
         const S mold_s = mag[rsub];
         S vold_s = S();
@@ -489,6 +507,8 @@ __global__ __launch_bounds__(kStepThreads) void k_gefen_step(const StepBatch B) 
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             float sj = 0.0f;
+            // elements of the row's last vector that the one before it holds too
+            const int skip = RAG ? (lir + j * lpr + 1) * W - (int)T.rowlen : 0;
 #pragma unroll
             for (int w = 0; w < W; ++w) {
                 const float gf = to_f32(gv[j].v[w]);
@@ -497,7 +517,7 @@ __global__ __launch_bounds__(kStepThreads) void k_gefen_step(const StepBatch B) 
                 upd[j][w] = u;
                 const uint32_t key = abs_key(u);
                 mxk = key > mxk ? key : mxk;
-                if (!P1) sj = __builtin_fmaf(gf, gf, sj);
+                if (!P1) sj = __builtin_fmaf(gf, RAG && w < skip ? 0.0f : gf, sj);
             }
             if (!P1) sumsq = sumsq + ((lir + j * lpr < T.nvec) ? sj : 0.0f);
         }
@@ -542,7 +562,7 @@ __global__ __launch_bounds__(kStepThreads) void k_gefen_step(const StepBatch B) 
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
 #define GEFEN_SWEEP2(PROBES, WD)                                                                                 \
-    step_sweep2<D, S, W, R, P1, TAB, PROBES, WD>(T, L, utab, root, upd_of, gv, pv, vv, idx, p, vm, base, lir, lpr, active, \
+    step_sweep2<D, S, W, R, P1, TAB, RAG, PROBES, WD>(T, L, utab, root, upd_of, gv, pv, vv, idx, p, vm, base, lir, lpr, active, \
                                                  K, mn, rb, ss)
         // (one_probe is false without the fine bucket: kFine ? 1 : 2 only keeps
         // the single-probe sweep from being instantiated there)
@@ -1200,21 +1220,25 @@ __global__ __launch_bounds__(kThreads) void k_muon_packed(const MuonBatch B) {
 
 // kernel key: dtype pair, W, R (0 = long rows), P1
 struct Key {
-    int d, s, W, R, p1, tab;
+    int d, s, W, R, p1, tab, rag;
     bool operator==(const Key& o) const {
-        return d == o.d && s == o.s && W == o.W && R == o.R && p1 == o.p1 && tab == o.tab;
+        return d == o.d && s == o.s && W == o.W && R == o.R && p1 == o.p1 && tab == o.tab && rag == o.rag;
     }
 };
 
 template <typename D, typename S>
 hipError_t launch_step(const Key& k, const StepBatch& b, int grid, hipStream_t st) {
-#define GEFEN_STEP_CASE(WW, RR)                                                                          \
-    if (k.W == WW && k.R == RR) {                                                                       \
-        if (k.p1) {                                                                                     \
-            hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, true, false>), dim3(grid), dim3(kStepThreads), 0, st, b);           \
+#define GEFEN_STEP_CASE(WW, RR, RAG)                                                                     \
+    if (k.W == WW && k.R == RR && k.rag == RAG) {                                                       \
+        if (k.p1) { /* ragged period-one rows have at most 256 elements: two vectors per lane */        \
+            if constexpr (!RAG || RR <= 2)                                                              \
+                hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, true, false, RAG>), dim3(grid), dim3(kStepThreads), 0, st, b);  \
+            else return hipErrorInvalidValue;                                                           \
+        } else if constexpr (WW > 1) {                                                                  \
+            if (k.tab) hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, false, true, RAG>), dim3(grid), dim3(kStepThreads), 0, st, b); \
+            else hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, false, false, RAG>), dim3(grid), dim3(kStepThreads), 0, st, b);     \
         } else {                                                                                        \
-            if (k.tab) hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, false, true>), dim3(grid), dim3(kStepThreads), 0, st, b); \
-            else hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, false, false>), dim3(grid), dim3(kStepThreads), 0, st, b);      \
+            hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, false, false, RAG>), dim3(grid), dim3(kStepThreads), 0, st, b);     \
         }                                                                                               \
         return hipGetLastError();                                                                       \
     }
@@ -1222,13 +1246,15 @@ hipError_t launch_step(const Key& k, const StepBatch& b, int grid, hipStream_t s
         hipLaunchKernelGGL((k_gefen_step_long<D, S>), dim3(grid), dim3(kThreads), 0, st, b);
         return hipGetLastError();
     }
-    if (sizeof(D) == 2) {
-        GEFEN_STEP_CASE(8, 1) GEFEN_STEP_CASE(8, 2) GEFEN_STEP_CASE(8, 4) GEFEN_STEP_CASE(8, 8)
-        GEFEN_STEP_CASE(4, 1) GEFEN_STEP_CASE(4, 2) GEFEN_STEP_CASE(4, 4) GEFEN_STEP_CASE(4, 8)
-    } else {
-        GEFEN_STEP_CASE(4, 1) GEFEN_STEP_CASE(4, 2) GEFEN_STEP_CASE(4, 4) GEFEN_STEP_CASE(4, 8)
+    constexpr int kWide = sizeof(D) == 2 ? 8 : 4;
+    GEFEN_STEP_CASE(kWide, 1, false) GEFEN_STEP_CASE(kWide, 2, false)
+    GEFEN_STEP_CASE(kWide, 4, false) GEFEN_STEP_CASE(kWide, 8, false)
+    if constexpr (sizeof(D) == 2) {
+        GEFEN_STEP_CASE(4, 1, false) GEFEN_STEP_CASE(4, 2, false) GEFEN_STEP_CASE(4, 4, false) GEFEN_STEP_CASE(4, 8, false)
     }
-    GEFEN_STEP_CASE(1, 1) GEFEN_STEP_CASE(1, 2) GEFEN_STEP_CASE(1, 4) GEFEN_STEP_CASE(1, 8)
+    GEFEN_STEP_CASE(kWide, 1, true) GEFEN_STEP_CASE(kWide, 2, true)
+    GEFEN_STEP_CASE(kWide, 4, true) GEFEN_STEP_CASE(kWide, 8, true)
+    GEFEN_STEP_CASE(1, 1, false) GEFEN_STEP_CASE(1, 2, false)  // rows shorter than a vector
 #undef GEFEN_STEP_CASE
     return hipErrorInvalidValue;
 }

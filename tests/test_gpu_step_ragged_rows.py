@@ -1,0 +1,91 @@
+"""The step kernels on rows that are no whole number of vectors (the last vector is
+shifted back over the one before it) against the oracle, with the bars of
+test_gpu_step.py; and on tensors at unaligned addresses, whose rows are the aligned
+ones' vectors, bit for bit against aligned copies, through gefen_step_tasks and a
+kept plan."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import gpu_util as gu
+from gefen_amd import _lib
+from test_gpu_step import _codebook, _run_case, _tables
+
+pytestmark = pytest.mark.gpu
+
+# one vector and a bit, lane groups' ends, whole waves with two to eight vectors per
+# lane, the longest register rows and the first ones past them
+LENGTHS = {"bf16": [9, 11, 15, 17, 31, 127, 250, 257, 509, 511, 515, 1021, 1027, 2047, 2049, 4090, 4095, 4097],
+           "f32": [5, 6, 7, 9, 31, 127, 129, 253, 255, 257, 511, 1021, 1027, 2045, 2047, 2049]}
+
+
+@pytest.mark.parametrize("dt,sdt", [("bf16", "bf16"), ("f16", "f16"), ("f32", "f32"), ("bf16", "f32"), ("f16", "f32")])
+def test_odd_block_rows_match_oracle(dt, sdt):
+    for i, length in enumerate(LENGTHS["f32" if dt == "f32" else "bf16"]):
+        _run_case("rag_{}_{}_{}".format(dt, sdt, length), dt, sdt, length * (3 + 70 // length * (i % 2 + 1)), length,
+                  0.1 * (i % 2))
+
+
+@pytest.mark.parametrize("dt,sdt", [("bf16", "bf16"), ("f16", "f16"), ("f32", "f32"), ("bf16", "f32")])
+@pytest.mark.parametrize("n", [9 * 1009, 251 * 67, 253 * 1013, 17 * 1021, 5 * 1013, 3 * 1019, 1021, 250 * 1009])
+def test_odd_period_one_rows_match_oracle(dt, sdt, n):
+    _run_case("rag_p1_{}_{}_{}".format(dt, sdt, n), dt, sdt, n, 1, 0.05)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+def test_unaligned_tensors_step_as_aligned_ones(dt):
+    lib = _lib.load()
+    cb = torch.from_numpy(_codebook()).to("cuda:0")
+    tables = _tables(cb)
+    gen = torch.Generator().manual_seed(11)
+    tdt = gu.TORCH[dt]
+    shapes = [(40, 2048, 0), (50, 512, 0), (60, 64, 0), (256 * 40, 1, 256), (1000, 1, 250), (30, 12, 0), (9, 20, 0)]
+
+    def build(offset):
+        rows = []
+        for i, (rows_v, period, pod) in enumerate(shapes):
+            n = rows_v * period
+            blocks = n // (pod or period)
+
+            def at(values, dtype, shift):
+                buf = torch.zeros(values.numel() + 16, dtype=dtype, device="cuda:0")
+                v = buf[shift:shift + values.numel()]
+                v.copy_(values)
+                return v, buf
+
+            r = torch.Generator().manual_seed(100 + i)
+            p, g = torch.randn(n, generator=r) * 0.02, torch.randn(n, generator=r) * 0.05
+            idx = torch.randint(0, 256, (n,), generator=r, dtype=torch.uint8)
+            mag = torch.rand(blocks, generator=r) * 0.05 + 0.01
+            vm = torch.rand(rows_v, generator=r) * 1e-3
+            o = offset and 1 + i % 3
+            rows.append([at(p, tdt, o), at(g, tdt, o), at(idx, torch.uint8, offset and 1 + i % 5), at(mag, tdt, 0),
+                         at(vm, tdt, o if pod else 0)])
+        tasks = np.zeros(len(shapes), dtype=_lib.STEP_TASK)
+        for t, (rows_v, period, pod), r in zip(tasks, shapes, rows):
+            for key, (v, _) in zip(("p", "grad", "m_codebook", "m_magnitude", "vmean"), r):
+                t[key] = v.data_ptr()
+            t["numel"], t["period"], t["period_one_divisor"] = rows_v * period, period, pod
+            t["param_dtype"] = t["state_dtype"] = gu.CODE[dt]
+            t["beta1"], t["beta2"], t["lr"], t["eps"], t["weight_decay"] = 0.9, 0.999, 1e-3, 1e-8, 0.1
+            t["bias_correction_1"], t["bias_correction_2"] = 1 - 0.9 ** 3, 1 - 0.999 ** 3
+        return rows, tasks
+
+    (ra, ta), (rb, tb), (rc, tc) = build(0), build(1), build(1)
+    plan = ctypes.c_void_p()
+    _lib.check(lib.gefen_step_plan_create(tc.ctypes.data, len(tc), tables.data_ptr(), ctypes.byref(plan)))
+    for _ in range(2):
+        _lib.check(lib.gefen_step_tasks(ta.ctypes.data, len(ta), tables.data_ptr(), gu.stream()))
+        _lib.check(lib.gefen_step_tasks(tb.ctypes.data, len(tb), tables.data_ptr(), gu.stream()))
+        _lib.check(lib.gefen_step_plan_run(plan, tc.ctypes.data, len(tc), gu.stream()))
+    torch.cuda.synchronize()
+    lib.gefen_step_plan_destroy(plan)
+    for i, (a, b, c) in enumerate(zip(ra, rb, rc)):
+        for key, x, y, z in zip(("p", "g", "idx", "mag", "vmean"), a, b, c):
+            assert torch.equal(x[0].view(torch.uint8), y[0].contiguous().view(torch.uint8)), (shapes[i], key)
+            assert torch.equal(x[0].view(torch.uint8), z[0].contiguous().view(torch.uint8)), (shapes[i], key)
+            shift = y[0].storage_offset()
+            assert not y[1][:shift].any() and not y[1][shift + y[0].numel():].any(), (shapes[i], key)  # nothing beside it
