@@ -189,7 +189,7 @@ static_assert(kStepThreads <= 256 && kThreads <= 256, "launch cap assumes at mos
 // launch's grid (the caller rejects the tensor).
 int32_t task_wgs(const Key& k, int64_t nrows, int lpr_log2, int waves, int iters) {
     int64_t wgs = nrows;
-    if (k.R != 0) {
+    if (k.R != 0 && k.tab != 3) {
         const int64_t rpw = 64 >> lpr_log2;
         const int64_t units = (nrows + rpw - 1) / rpw;
         wgs = (units + waves * iters - 1) / (waves * iters);
@@ -200,6 +200,7 @@ int32_t task_wgs(const Key& k, int64_t nrows, int lpr_log2, int waves, int iters
 struct PendingStep {
     Key key;
     StepTask task;
+    int galign;  // gradient alignment (bytes) that the kernel needs
 };
 
 // A second stream per device (default priority) for the small launches of a
@@ -256,6 +257,48 @@ struct StepLaunch {
     int wg;
     int64_t elems;
 };
+
+// Launches of fewer elements than this join their dtype's mixed launch: 4M take
+// about as long to stream as a launch's latency.  25 float16 tensors of 11M elements
+// in 13 launches: 108 us unmixed, 73, 47 and 45 with 1M, 2M and 4M here.
+constexpr int64_t kMixedElems = 4 << 20;
+
+// The k_gefen_step_mixed form of a task with this key, or -1.
+int mixed_form(const Key& k) {
+    if (k.R == 0) return kFormLong;
+    if (k.W == 1) return !k.p1 ? kFormOne : (k.R == 1 ? kFormOneP1 : kFormOneP2);
+    if (k.p1 && k.W != (dtype_size(k.d) == 2 ? 8 : 4)) return k.R == 1 ? kFormHalfP1 : (k.R == 2 ? kFormHalfP2 : -1);
+    if (k.p1) return k.R == 1 ? kFormWideP1 : (k.R == 2 ? kFormWideP2 : -1);
+    if (k.tab == 3) return k.R == 2 ? kFormRow2 : (k.R == 4 ? kFormRow4 : -1);
+    return k.R == 1 ? (k.tab ? kFormWide1Tab : kFormWide1) : (k.R == 2 ? kFormWide2 : (k.R == 4 ? kFormWide4 : -1));
+}
+
+// Turn the tasks that would make small launches into tasks of one mixed launch per
+// dtype pair, where there are two or more such launches.
+void mark_mixed(std::vector<PendingStep>& pend) {
+    struct Group { Key key; int64_t elems; };
+    std::vector<Group> groups;
+    std::vector<int> group(pend.size());
+    for (size_t i = 0; i < pend.size(); ++i) {
+        size_t q = 0;
+        while (q < groups.size() && !(groups[q].key == pend[i].key)) ++q;
+        if (q == groups.size()) groups.push_back({pend[i].key, 0});
+        groups[q].elems += pend[i].task.nrows * pend[i].task.rowlen;
+        group[i] = (int)q;
+    }
+    auto small = [&](const Group& g) { return mixed_form(g.key) >= 0 && g.elems < kMixedElems; };
+    for (size_t i = 0; i < pend.size(); ++i) {
+        PendingStep& ps = pend[i];
+        if (!small(groups[group[i]])) continue;
+        int launches = 0;
+        for (const Group& g : groups)
+            launches += g.key.d == ps.key.d && g.key.s == ps.key.s && small(g);
+        if (launches < 2) continue;
+        ps.task.form = (int16_t)mixed_form(ps.key);
+        ps.task.nwg = task_wgs(ps.key, ps.task.nrows, ps.task.lpr_log2, kStepWaves, 1);
+        ps.key = Key{ps.key.d, ps.key.s, 0, 0, 0, 0, 0, 1};
+    }
+}
 
 // Group the pending tasks into launches: per kernel key, up to kMaxBatch tasks
 // and one stepsize table per launch, in order of first appearance.  slot_of
@@ -372,13 +415,16 @@ int make_step_task(const gefen_step_task& in, int mode, const float* stepsize, P
     if (p1 && rowlen > 256 * 64) return fail_inval("period_one_divisor %lld is too large", (long long)rowlen);
     if (P > INT32_MAX) return fail_inval("period %lld is too large", (long long)P);
     const int dsz = dtype_size(in.param_dtype), ssz = dtype_size(in.state_dtype);
-    int W = pick_width(dsz, rowlen, {in.p, in.grad}, 1, in.m_codebook, ssz, p1 ? in.vmean : nullptr);
-    // rows of at least one wide vector that aligned accesses would take one element
-    // at a time: wide vectors at any alignment, the last one shifted back
+    const int whole = pick_width(dsz, rowlen, {in.p, in.grad}, 1, in.m_codebook, ssz, p1 ? in.vmean : nullptr);
+    if (p1 && rowlen > 256 * whole) return fail_inval("period_one_divisor %lld is too large", (long long)rowlen);
+    // rows that are no whole number of aligned wide vectors take them at any
+    // alignment, the last one shifted back: 32M bf16 elements in rows of 12, 100 and
+    // 252 took 100, 126 and 99 us in aligned vectors of 4, now 69, 63 and 64.  Period-one
+    // rows, with three more conversions per element, keep the aligned vectors of 4 (rows
+    // of 12 and 100: 146 and 144 us, against 161 and 159).
     const int wide = dsz == 2 ? 8 : 4;
-    const bool rag = W == 1 && rowlen >= wide;
-    if (rag && p1 && rowlen > 256) return fail_inval("period_one_divisor %lld is too large", (long long)rowlen);
-    if (rag) W = wide;
+    const bool rag = rowlen >= wide && (p1 ? whole == 1 : whole != wide);
+    const int W = rag ? wide : (p1 || whole == wide ? whole : 1);
     const int64_t nvec = (rowlen + W - 1) / W;
     // period-one rows (at most 256 * 64 elements) take half the lanes with
     // twice the vectors per lane: more bytes in flight per lane
@@ -387,10 +433,20 @@ int make_step_task(const gefen_step_task& in, int mode, const float* stepsize, P
     int R = r_bucket(nvec, l2);
     if (p1 && R == 0) return fail_inval("period_one_divisor %lld is too large", (long long)rowlen);
     // row tables pay off when a row has at least as many elements as codewords per lane group
-    const int tab = (R != 0 && l2 >= 5 && !p1) ? 1 : 0;
-    // the kernels keep one row table per wave when R >= 2 (whole-wave rows)
-    if (tab && R >= 2 && l2 != 6) return fail_inval("internal: row tables of a %d-lane row", 1 << l2);
-    Key k{in.param_dtype, in.state_dtype, R == 0 ? 1 : W, R, p1 ? 1 : 0, tab, rag && R != 0};
+    int tab = (R != 0 && l2 >= 5 && !p1) ? (l2 == 6 ? 1 : 2) : 0;
+    // Rows that would take more than four vectors per lane of a wave go to a whole
+    // workgroup: 24M bf16 elements in rows of 4092 and 5120 take 38 and 39 us, against
+    // 49 (a wave, eight vectors per lane) and 52 (two sweeps); float32 in rows of 2304
+    // and 5120, 57 and 59 us against 75 and 78.  Shorter rows stay with a wave: with a
+    // workgroup float32 rows of 768 took 69 us instead of 61, and a step of 1B bf16
+    // elements in rows of 2048 and less 2.59 ms instead of 2.46.
+    if (!p1 && nvec > 256 && nvec <= 8192 / wide) {
+        l2 = 8;
+        tab = 3;
+        R = nvec <= 512 ? 2 : (nvec <= 1024 ? 4 : 8);
+    }
+    Key k{in.param_dtype, in.state_dtype, R == 0 ? 1 : W, R, p1 ? 1 : 0, tab, rag && R != 0, 0};
+    out.galign = (rag || R == 0 ? 1 : W) * dsz;
     StepTask& t = out.task;
     memset(&t, 0, sizeof(t));
     t.p = in.p;
@@ -668,6 +724,7 @@ int step_tasks_general(const gefen_step_task* tasks, int ntasks, const CodebookT
         if (rc) return rc;
         pend.push_back(ps);
     }
+    mark_mixed(pend);
     return run_steps_pooled(pend, tables, st);
 }
 
@@ -722,6 +779,9 @@ extern "C" int gefen_step_tasks_noalloc(const gefen_step_task* tasks, int ntasks
                           "(at most %zu f16-state or %zu bf16-state (sqrt(bc2), eps, 1/bc1) settings per call)",
                           lp.total * sizeof(float), kNoAllocScratchFloats * sizeof(float), kNoAllocScratchFloats / kLutSlot,
                           kNoAllocScratchFloats / kRootSlot);
+    // the limit above is of the call's settings, whichever launches read them
+    mark_mixed(pend);
+    plan_luts(pend, lp);
     if (lp.keys.empty()) return flush_steps(pend, static_cast<const CodebookTables*>(tables), st, false);
     int dev = 0;
     int rc = stream_device(st, &dev);
@@ -757,7 +817,6 @@ struct gefen_step_plan {
     int ntasks = 0;
     std::vector<gefen_step_task> shape;  // the creation rows
     std::vector<int> row;                // caller row of each pending task
-    std::vector<int> galign;             // gradient alignment (bytes) each pending task's kernel needs
     std::vector<PendingStep> pend;
     std::vector<StepLaunch> launches;
     std::vector<int> slot;               // launch * kMaxBatch + position of each pending task
@@ -794,7 +853,7 @@ int plan_run_fast(gefen_step_plan& P, const gefen_step_task* tasks, hipStream_t 
     const StepTask* prev_t = nullptr;
     for (size_t i = 0; i < P.pend.size(); ++i) {
         const gefen_step_task& in = tasks[P.row[i]];
-        if (!same_tensors(in, P.shape[P.row[i]]) || !in.grad || !aligned(in.grad, P.galign[i])) return -1;
+        if (!same_tensors(in, P.shape[P.row[i]]) || !in.grad || !aligned(in.grad, P.pend[i].galign)) return -1;
         int rc = check_step_task(in);
         if (rc) return rc;
         StepTask& t = P.pend[i].task;
@@ -928,7 +987,6 @@ extern "C" int gefen_step_plan_create(const gefen_step_task* tasks, int ntasks, 
             if (rc == GEFEN_OK) {
                 P->pend.push_back(ps);
                 P->row.push_back(i);
-                P->galign.push_back((ps.key.R == 0 || ps.key.rag ? 1 : ps.key.W) * dtype_size(ps.key.d));
             }
         }
         if (rc) {
@@ -937,6 +995,7 @@ extern "C" int gefen_step_plan_create(const gefen_step_task* tasks, int ntasks, 
         }
     }
     // group as gefen_step_tasks would, with the creation rows' stepsize-table keys
+    mark_mixed(P->pend);
     plan_luts(P->pend, P->lp);
     for (size_t i = 0; i < P->pend.size(); ++i)
         P->pend[i].task.lut = P->lp.which[i] >= 0 ? reinterpret_cast<const float*>((uintptr_t)(P->lp.which[i] + 1) * 256)

@@ -108,7 +108,8 @@ struct StepTask {
     int32_t lpr_log2;  // log2(lanes per row)
     int32_t mode;      // StepMode
     float b1c, b2, omb2, sqrt_bc2, eps, inv_bc1, lr, wdf;
-    int32_t do_wd;
+    int16_t do_wd;
+    int16_t form;      // StepForm of a k_gefen_step_mixed task
     int32_t nwg;       // workgroups of this task
 };
 
@@ -317,10 +318,10 @@ __device__ __forceinline__ int nearest_one_probe(float x, const float* thr, cons
 // and positive and the search with that many probes is exact (0: the general
 // search).  Every lane computes all R
 // vectors (out-of-row vectors hold a copy of the row's last vector); only
-// in-row vectors of active rows are stored.  WD: weight decay
-// (gefen.py:1280-1281) is applied to the parameter first.  root: the LDS
+// in-row vectors of active rows are stored.  WD 1: weight decay
+// (gefen.py:1280-1281) is applied to the parameter first; 2: where the task asks.  root: the LDS
 // square-root table of a period-one bf16 state, or nullptr.
-template <typename D, typename S, int W, int R, bool P1, bool TAB, bool RAG, int PROBES, bool WD, bool FINE, typename UF>
+template <typename D, typename S, int W, int R, bool P1, int TAB, bool RAG, int PROBES, int WD, bool FINE, typename UF>
 __device__ __forceinline__ void step_sweep2(const StepTask& T, const LdsTables<FINE>& L, const float* utab,
                                             const float* root, const UF& upd_of, const Vec<D, W> (&gv)[R],
                                             const Vec<D, W> (&pv)[R], const Vec<S, W> (&vv)[R], uint8_t* idx, D* p,
@@ -387,7 +388,7 @@ __device__ __forceinline__ void step_sweep2(const StepTask& T, const LdsTables<F
                 u = (q * s) * T.lr;
             }
             float pf = to_f32(pv[j].v[w]);
-            if (WD) pf = round_to<D>(pf * T.wdf);
+            if (WD == 1 || (WD == 2 && T.do_wd)) pf = round_to<D>(pf * T.wdf);
             po.v[w] = from_f32<D>(pf - u);
         }
         const int v = lir + j * lpr;
@@ -400,8 +401,15 @@ __device__ __forceinline__ void step_sweep2(const StepTask& T, const LdsTables<F
     }
 }
 
+// 16-bit parameters search the fine bucket with one probe where the codebook
+// allows; fp32 kernels keep the 6 KB tables, which leave them one more
+// workgroup per CU.
+template <typename D> constexpr bool step_fine() { return sizeof(D) == 2; }
+
 // TAB: a lane group of >= 32 lanes owns the row and keeps two row tables in
-// LDS, cur[i] = cb_D[i] * old magnitude and upd[i] = the parameter step of
+// LDS (TAB 1: rows of a whole wave; 2: two rows of 32 lanes in a wave, two such
+// pairs; the smaller footprint lets more workgroups share a CU; 3: rows of more than
+// 256 vectors, which a whole workgroup owns), cur[i] = cb_D[i] * old magnitude and upd[i] = the parameter step of
 // codeword i (gefen.py:1205-1206, 1328-1332 for this row's magnitude and
 // stepsize), so the element loops look both up instead of recomputing.
 //
@@ -413,20 +421,169 @@ __device__ __forceinline__ void step_sweep2(const StepTask& T, const LdsTables<F
 // RAG: see vec_first.  Odd rows took one element per lane and load before: 30000
 // period-one rows of 250 bf16 elements (53 MB) went from 53 to 31 us, and rows of
 // 513 to 4096 elements left the two-sweep kernel.
-template <typename D, typename S, int W, int R, bool P1, bool TAB, bool RAG>
+// MIXED: the copy inside k_gefen_step_mixed.
+template <typename D, typename S, int W, int R, bool P1, int TAB, bool RAG, bool MIXED, bool FINE>
+__device__ __forceinline__ void step_unit(const StepTask& T, const LdsTables<FINE>& L, float* tabs, float* red,
+                                          const float* root, int K, int max_probe, int64_t unit) {
+    constexpr bool kFine = FINE, WG = TAB == 3;
+    static_assert(kStepWaves == 4, "red holds a maximum and a sum of four waves");
+    // the row's lanes have stored what the others read next
+    auto lds_sync = [] {
+        if constexpr (WG) {
+            __syncthreads();
+        } else {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+    };
+    const bool two_probe = max_probe <= 2, one_probe = kFine && max_probe <= 1;
+    const int lane = WG ? threadIdx.x : threadIdx.x & 63;
+    const int lpr = WG ? kStepThreads : 1 << T.lpr_log2;
+    const int rpw = WG ? 1 : 64 >> T.lpr_log2;
+    const int lir = lane & (lpr - 1);
+    const int sub = WG ? 0 : lane >> T.lpr_log2;
+    float* ctab = tabs + (TAB == 2 ? (sub & 1) * 512 : 0);
+    float* utab = ctab + 256;
+    const int64_t row0 = unit * rpw;
+    if (row0 >= T.nrows) return;  // uniform across the wave
+    const int64_t row = row0 + sub;
+    const bool active = row < T.nrows;
+    const int rsub = active ? sub : (int)(T.nrows - 1 - row0);  // row within the unit
+    // the unit's rows start here; lanes address them with 32-bit offsets
+    // (64 rows of at most 64 * 8 * 8 elements)
+    const int64_t ub = row0 * T.rowlen;
+    D* __restrict__ p = static_cast<D*>(T.p) + ub;
+    const D* __restrict__ g = static_cast<const D*>(T.g) + ub;
+    uint8_t* __restrict__ idx = T.idx + ub;
+    S* __restrict__ mag = static_cast<S*>(T.mag) + row0;
+    S* __restrict__ vm = static_cast<S*>(T.vmean) + (P1 ? ub : row0);
+    const float* stepsize = T.stepsize + row0;
+    const uint32_t base = (uint32_t)rsub * (uint32_t)T.rowlen;
+
+    // every element vector of the row, then the row scalars
+    Vec<D, W> gv[R], pv[R];
+    Vec<uint8_t, W> iv[R];
+    Vec<S, W> vv[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int v = min(lir + j * lpr, T.nvec - 1);
+        const uint32_t e = base + (uint32_t)vec_first<RAG, W>(v, T.rowlen);
+        gv[j] = sload<D, W, RAG>(g, e);
+        iv[j] = sload<uint8_t, W, RAG>(idx, e);
+        pv[j] = sload<D, W, RAG>(p, e);
+        if (P1) vv[j] = sload<S, W, RAG>(vm, e);
+    }
+    const S mold_s = mag[rsub];
+    S vold_s = S();
+    float step_given = 0.0f;
+    if (!P1) {
+        if (T.mode == kStepsizeGiven) step_given = stepsize[rsub];
+        else vold_s = vm[rsub];
+    }
+    const float mold = to_f32(mold_s);
+    // vmean (vmean modes) or stepsize (given-stepsize mode) of the row
+    const float rowv = (T.mode == kStepsizeGiven) ? step_given : to_f32(vold_s);
+    if (TAB) {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const int i = lir + t * lpr;
+            if (i < 256) ctab[i] = L.cbd[i] * mold;
+        }
+        lds_sync();
+    }
+    float upd[R][W];
+    uint32_t mxk = 0;
+    float sumsq = 0.0f;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        float sj = 0.0f;
+        // elements of the row's last vector that the one before it holds too
+        const int skip = RAG ? (lir + j * lpr + 1) * W - (int)T.rowlen : 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const float gf = to_f32(gv[j].v[w]);
+            const float cur = TAB ? ctab[iv[j].v[w]] : L.cbd[iv[j].v[w]] * mold;
+            const float u = __builtin_fmaf(T.b1c, gf - cur, cur);  // lerp, weight < 0.5
+            upd[j][w] = u;
+            const uint32_t key = abs_key(u);
+            mxk = key > mxk ? key : mxk;
+            if (!P1) sj = __builtin_fmaf(gf, RAG && w < skip ? 0.0f : gf, sj);
+        }
+        if (!P1) sumsq = sumsq + ((lir + j * lpr < T.nvec) ? sj : 0.0f);
+    }
+    float mx = __uint_as_float(wave_group_max_u32(mxk, WG ? 64 : lpr)), tot = 0.0f;
+    if (!P1) tot = wave_group_sum(sumsq, WG ? 64 : lpr);
+    if constexpr (WG) {
+        if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6] = mx; red[4 + (threadIdx.x >> 6)] = tot; }
+        __syncthreads();  // also: every thread has read mag and vm of the row
+        mx = nanmax(nanmax(red[0], red[1]), nanmax(red[2], red[3]));
+        tot = (red[4] + red[5]) + (red[6] + red[7]);
+    }
+    float ss = 0.0f;
+    if (!P1) {
+        if (T.mode == kVmeanUpdate) {
+            const float ms = mean_of(tot, T.period);
+            const S vnew = from_f32<S>(__builtin_fmaf(ms, T.omb2, rowv * T.b2));
+            if (active && lir == 0) vm[rsub] = vnew;
+            ss = stepsize_of(to_f32(vnew), T);
+        } else if (T.mode == kVmeanGiven) {
+            ss = stepsize_of(rowv, T);
+        } else {
+            ss = rowv;
+        }
+    }
+    const S mag_s = from_f32<S>(mx);
+    if (active && lir == 0) mag[rsub] = mag_s;
+    const float mn = to_f32(mag_s);
+    auto upd_of = [&](int j, int w) -> float { return upd[j][w]; };
+    // x = upd / mn where mn > 0, else 0 (gefen.py:1184-1187).  A block whose
+    // magnitude is 0, NaN or inf takes the general element path.
+    const bool plain = (mn > 0.0f) && (mn < __builtin_inff());
+    const double rb = plain ? 1.0 / (double)mn : 0.0;
+    const bool fast = plain && two_probe;
+    if (TAB && !P1) {
+        if (fast) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const int i = lir + t * lpr;
+                if (i < 256) {
+                    float q = L.cbd[i] * mn;
+                    if (sizeof(D) == sizeof(S)) q = round_to<D>(q);
+                    utab[i] = (q * ss) * T.lr;
+                }
+            }
+        }
+        lds_sync();
+    }
+#define GEFEN_SWEEP2(PROBES, WD)                                                                                 \
+step_sweep2<D, S, W, R, P1, TAB, RAG, PROBES, WD>(T, L, utab, root, upd_of, gv, pv, vv, idx, p, vm, base, lir, lpr, active, \
+                                             K, mn, rb, ss)
+    // (one_probe is false without the fine bucket: kFine ? 1 : 2 only keeps
+    // the single-probe sweep from being instantiated there)
+    if constexpr (MIXED) {  // fewer copies of the sweep: the kernel holds them for every form
+        if (fast) GEFEN_SWEEP2(2, 2);
+        else GEFEN_SWEEP2(0, 2);
+    } else if (T.do_wd) {
+        if (fast && one_probe) GEFEN_SWEEP2(kFine ? 1 : 2, 1);
+        else if (fast) GEFEN_SWEEP2(2, 1);
+        else GEFEN_SWEEP2(0, 1);
+    } else {
+        if (fast && one_probe) GEFEN_SWEEP2(kFine ? 1 : 2, 0);
+        else if (fast) GEFEN_SWEEP2(2, 0);
+        else GEFEN_SWEEP2(0, 0);
+    }
+#undef GEFEN_SWEEP2
+}
+
+template <typename D, typename S, int W, int R, bool P1, int TAB, bool RAG>
 __global__ __launch_bounds__(kStepThreads) void k_gefen_step(const StepBatch B) {
     constexpr bool kRoot = P1 && std::is_same<S, bf16_t>::value;
-    // 16-bit parameters search the fine bucket with one probe where the codebook
-    // allows; fp32 kernels keep the 6 KB tables, which leave them one more
-    // workgroup per CU
-    constexpr bool kFine = sizeof(D) == 2;
+    constexpr bool kFine = step_fine<D>();
     __shared__ LdsTables<kFine> L;
-    // row tables of the wave's rows: rows of at least two vectors per lane own a
-    // whole wave (64 lanes), so one slot per wave; single-vector rows may take 32
-    // lanes, two rows per wave (make_step_task keeps to this).  The smaller LDS
-    // footprint lets more workgroups share a CU.
-    constexpr int kRowSlots = (TAB && R == 1) ? 2 : 1;
-    __shared__ float row_tab[TAB ? kStepWaves : 1][kRowSlots][2][256];
+    __shared__ float row_tab[TAB == 1 || TAB == 2 ? kStepWaves : 1][TAB == 2 ? 2 : 1][2][256];
+    __shared__ float red[8];
     __shared__ __attribute__((aligned(16))) float root_lds[kRoot ? kRootTab : 4];
     // every task of a launch has the same stepsize table (flush_steps)
     const float* root_src = kRoot ? B.t[0].lut : nullptr;
@@ -434,219 +591,202 @@ __global__ __launch_bounds__(kStepThreads) void k_gefen_step(const StepBatch B) 
     int K;
     load_tables<D, kStepThreads>(L, B.tables, K, root_src, root_lds);
     const int max_probe = kFine ? B.tables->max_probe_fine : B.tables->max_probe;
-    const bool two_probe = max_probe <= 2, one_probe = kFine && max_probe <= 1;
     const int ti = find_task(B.wg_begin, B.ntasks);
     const StepTask T = B.t[ti];
-
-    const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lpr = 1 << T.lpr_log2;
-    const int rpw = 64 >> T.lpr_log2;
-    const int lir = lane & (lpr - 1);
-    const int sub = lane >> T.lpr_log2;
     const int64_t lw = blockIdx.x - B.wg_begin[ti];
-    float* ctab = row_tab[TAB ? wave : 0][kRowSlots == 2 ? (sub & 1) : 0][0];
-    float* utab = row_tab[TAB ? wave : 0][kRowSlots == 2 ? (sub & 1) : 0][1];
-
-    constexpr int kIt = step_iter<P1>();
-    for (int it = 0; it < kIt; ++it) {
-        const int64_t unit = (lw * kIt + it) * kStepWaves + wave;
-        const int64_t row0 = unit * rpw;
-        if (row0 >= T.nrows) break;  // uniform across the wave
-        const int64_t row = row0 + sub;
-        const bool active = row < T.nrows;
-        const int rsub = active ? sub : (int)(T.nrows - 1 - row0);  // row within the unit
-        // the unit's rows start here; lanes address them with 32-bit offsets
-        // (64 rows of at most 64 * 8 * 8 elements)
-        const int64_t ub = row0 * T.rowlen;
-        D* __restrict__ p = static_cast<D*>(T.p) + ub;
-        const D* __restrict__ g = static_cast<const D*>(T.g) + ub;
-        uint8_t* __restrict__ idx = T.idx + ub;
-        S* __restrict__ mag = static_cast<S*>(T.mag) + row0;
-        S* __restrict__ vm = static_cast<S*>(T.vmean) + (P1 ? ub : row0);
-        const float* stepsize = T.stepsize + row0;
-        const uint32_t base = (uint32_t)rsub * (uint32_t)T.rowlen;
-
-        // every element vector of the row, then the row scalars
-        Vec<D, W> gv[R], pv[R];
-        Vec<uint8_t, W> iv[R];
-        Vec<S, W> vv[R];
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-            const int v = min(lir + j * lpr, T.nvec - 1);
-            const uint32_t e = base + (uint32_t)vec_first<RAG, W>(v, T.rowlen);
-            gv[j] = sload<D, W, RAG>(g, e);
-            iv[j] = sload<uint8_t, W, RAG>(idx, e);
-            pv[j] = sload<D, W, RAG>(p, e);
-            if (P1) vv[j] = sload<S, W, RAG>(vm, e);
-        }
-        const S mold_s = mag[rsub];
-        S vold_s = S();
-        float step_given = 0.0f;
-        if (!P1) {
-            if (T.mode == kStepsizeGiven) step_given = stepsize[rsub];
-            else vold_s = vm[rsub];
-        }
-        const float mold = to_f32(mold_s);
-        // vmean (vmean modes) or stepsize (given-stepsize mode) of the row
-        const float rowv = (T.mode == kStepsizeGiven) ? step_given : to_f32(vold_s);
-        if (TAB) {
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int i = lir + t * lpr;
-                if (i < 256) ctab[i] = L.cbd[i] * mold;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-        float upd[R][W];
-        uint32_t mxk = 0;
-        float sumsq = 0.0f;
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-            float sj = 0.0f;
-            // elements of the row's last vector that the one before it holds too
-            const int skip = RAG ? (lir + j * lpr + 1) * W - (int)T.rowlen : 0;
-#pragma unroll
-            for (int w = 0; w < W; ++w) {
-                const float gf = to_f32(gv[j].v[w]);
-                const float cur = TAB ? ctab[iv[j].v[w]] : L.cbd[iv[j].v[w]] * mold;
-                const float u = __builtin_fmaf(T.b1c, gf - cur, cur);  // lerp, weight < 0.5
-                upd[j][w] = u;
-                const uint32_t key = abs_key(u);
-                mxk = key > mxk ? key : mxk;
-                if (!P1) sj = __builtin_fmaf(gf, RAG && w < skip ? 0.0f : gf, sj);
-            }
-            if (!P1) sumsq = sumsq + ((lir + j * lpr < T.nvec) ? sj : 0.0f);
-        }
-        const float mx = __uint_as_float(wave_group_max_u32(mxk, lpr));
-        float ss = 0.0f;
-        if (!P1) {
-            if (T.mode == kVmeanUpdate) {
-                const float tot = wave_group_sum(sumsq, lpr);
-                const float ms = mean_of(tot, T.period);
-                const S vnew = from_f32<S>(__builtin_fmaf(ms, T.omb2, rowv * T.b2));
-                if (active && lir == 0) vm[rsub] = vnew;
-                ss = stepsize_of(to_f32(vnew), T);
-            } else if (T.mode == kVmeanGiven) {
-                ss = stepsize_of(rowv, T);
-            } else {
-                ss = rowv;
-            }
-        }
-        const S mag_s = from_f32<S>(mx);
-        if (active && lir == 0) mag[rsub] = mag_s;
-        const float mn = to_f32(mag_s);
-        auto upd_of = [&](int j, int w) -> float { return upd[j][w]; };
-        // x = upd / mn where mn > 0, else 0 (gefen.py:1184-1187).  A block whose
-        // magnitude is 0, NaN or inf takes the general element path.
-        const bool plain = (mn > 0.0f) && (mn < __builtin_inff());
-        const double rb = plain ? 1.0 / (double)mn : 0.0;
-        const bool fast = plain && two_probe;
-        if (TAB && !P1) {
-            if (fast) {
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const int i = lir + t * lpr;
-                    if (i < 256) {
-                        float q = L.cbd[i] * mn;
-                        if (sizeof(D) == sizeof(S)) q = round_to<D>(q);
-                        utab[i] = (q * ss) * T.lr;
-                    }
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-#define GEFEN_SWEEP2(PROBES, WD)                                                                                 \
-    step_sweep2<D, S, W, R, P1, TAB, RAG, PROBES, WD>(T, L, utab, root, upd_of, gv, pv, vv, idx, p, vm, base, lir, lpr, active, \
-                                                 K, mn, rb, ss)
-        // (one_probe is false without the fine bucket: kFine ? 1 : 2 only keeps
-        // the single-probe sweep from being instantiated there)
-        if (T.do_wd) {
-            if (fast && one_probe) GEFEN_SWEEP2(kFine ? 1 : 2, true);
-            else if (fast) GEFEN_SWEEP2(2, true);
-            else GEFEN_SWEEP2(0, true);
-        } else {
-            if (fast && one_probe) GEFEN_SWEEP2(kFine ? 1 : 2, false);
-            else if (fast) GEFEN_SWEEP2(2, false);
-            else GEFEN_SWEEP2(0, false);
-        }
-#undef GEFEN_SWEEP2
-    }
+    constexpr int kIt = TAB == 3 ? 1 : step_iter<P1>();
+    for (int it = 0; it < kIt; ++it)
+        step_unit<D, S, W, R, P1, TAB, RAG, false>(T, L, row_tab[TAB == 1 || TAB == 2 ? wave : 0][0][0], red, root, K,
+                                                   max_probe, TAB == 3 ? lw : (lw * kIt + it) * kStepWaves + wave);
 }
 
 // ---------------------------------------------------------------------------
 // Gefen step, two-sweep path for rows longer than the register path holds
-// (P > 1 only): one workgroup per row, the second sweep re-reads g and idx.
-template <typename D, typename S>
-__global__ __launch_bounds__(kThreads) void k_gefen_step_long(const StepBatch B) {
-    __shared__ LdsTables<false> L;
-    __shared__ float red_mx[4], red_sum[4];
-    int K;
-    load_tables<D, kThreads>(L, B.tables, K);
-    const int ti = find_task(B.wg_begin, B.ntasks);
-    const StepTask& T = B.t[ti];
+// (more than 8192 elements, P > 1 only): one workgroup per row, the second sweep re-reads g and idx.
+// Bound by the latency of its loads: few rows, each a serial chain of vectors per
+// lane.  So four 16-byte vectors per lane are in flight at a time, at any alignment;
+// the elements after the row's last whole vector (fewer than W) go one per lane, as
+// the second sweep may not read what another lane has written.  tabs: 512 floats,
+// the row's tables as in step_unit; red: 8 floats.
+// 32M bf16 elements in rows of 33000: 164 us with one element per lane and load, 77 now.
+template <typename D, typename S, bool FINE>
+__device__ __forceinline__ void step_long_row(const StepTask& T, const LdsTables<FINE>& L, float* tabs, float* red, int K,
+                                              int max_probe, int64_t row) {
     constexpr bool QROUND = sizeof(D) == sizeof(S);
-    const int64_t row = blockIdx.x - B.wg_begin[ti];
-    if (row >= T.nrows) return;
-    D* __restrict__ p = static_cast<D*>(T.p);
-    const D* __restrict__ g = static_cast<const D*>(T.g);
-    uint8_t* __restrict__ idx = T.idx;
+    constexpr int W = sizeof(D) == 2 ? 8 : 4, U = 4;
+    static_assert(kThreads == 256, "one thread per codeword, four waves");
+    float* ctab = tabs;
+    float* utab = tabs + 256;
+    const int64_t base = row * T.rowlen;
+    D* __restrict__ p = static_cast<D*>(T.p) + base;
+    const D* __restrict__ g = static_cast<const D*>(T.g) + base;
+    uint8_t* __restrict__ idx = T.idx + base;
     S* __restrict__ mag = static_cast<S*>(T.mag);
     S* __restrict__ vm = static_cast<S*>(T.vmean);
-    const int64_t base = row * T.rowlen;
+    const int64_t nfull = T.rowlen / W, tail = nfull * W;
     const float mold = to_f32(mag[row]);
+    const float vold = T.mode == kStepsizeGiven ? T.stepsize[row] : to_f32(vm[row]);
+    ctab[threadIdx.x] = L.cbd[threadIdx.x] * mold;
+    __syncthreads();  // also: every thread has read mag[row] and vm[row]
     float mx = 0.0f, sumsq = 0.0f;
-    for (int64_t j = threadIdx.x; j < T.rowlen; j += kThreads) {
-        const float gf = to_f32(g[base + j]);
-        const float cur = L.cbd[idx[base + j]] * mold;
+    auto first = [&](float gf, uint8_t i, bool in) {
+        const float cur = ctab[i];
         const float u = __builtin_fmaf(T.b1c, gf - cur, cur);
-        mx = nanmax(mx, fabsf(u));
-        const float sq = gf * gf;
-        sumsq = sumsq + sq;
+        mx = nanmax(mx, in ? fabsf(u) : 0.0f);
+        return gf * gf;
+    };
+    for (int64_t v0 = threadIdx.x; v0 < nfull; v0 += U * kThreads) {
+        Vec<D, W> gv[U];
+        Vec<uint8_t, W> iv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t e = min(v0 + u * kThreads, nfull - 1) * W;
+            gv[u] = sload<D, W, true>(g + e, 0);
+            iv[u] = sload<uint8_t, W, true>(idx + e, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool in = v0 + u * kThreads < nfull;
+            float s = 0.0f;
+#pragma unroll
+            for (int w = 0; w < W; ++w) s = s + first(to_f32(gv[u].v[w]), iv[u].v[w], in);
+            sumsq = sumsq + (in ? s : 0.0f);
+        }
     }
+    if (tail + threadIdx.x < T.rowlen)
+        sumsq = sumsq + first(to_f32(g[tail + threadIdx.x]), idx[tail + threadIdx.x], true);
     mx = group_max(mx, 64);
     sumsq = group_sum(sumsq, 64);
     const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) { red_mx[wave] = mx; red_sum[wave] = sumsq; }
+    if ((threadIdx.x & 63) == 0) { red[wave] = mx; red[4 + wave] = sumsq; }
     __syncthreads();
-    mx = nanmax(nanmax(red_mx[0], red_mx[1]), nanmax(red_mx[2], red_mx[3]));
-    const float tot = (red_sum[0] + red_sum[1]) + (red_sum[2] + red_sum[3]);
-    float ss;
+    mx = nanmax(nanmax(red[0], red[1]), nanmax(red[2], red[3]));
+    float ss = vold;
     if (T.mode == kVmeanUpdate) {
-        const float ms = mean_of(tot, T.period);
-        const float prev = to_f32(vm[row]) * T.b2;
-        const S vnew = from_f32<S>(__builtin_fmaf(ms, T.omb2, prev));
+        const float tot = (red[4] + red[5]) + (red[6] + red[7]);
+        const S vnew = from_f32<S>(__builtin_fmaf(mean_of(tot, T.period), T.omb2, vold * T.b2));
         ss = stepsize_of(to_f32(vnew), T);
-        __syncthreads();  // every thread has read vm[row] before it is replaced
         if (threadIdx.x == 0) vm[row] = vnew;
     } else if (T.mode == kVmeanGiven) {
-        ss = stepsize_of(to_f32(vm[row]), T);
-    } else {
-        ss = T.stepsize[row];
+        ss = stepsize_of(vold, T);
     }
     const S mag_s = from_f32<S>(mx);
     const float mn = to_f32(mag_s);
-    __syncthreads();  // every thread has read mag[row] (mold) before it is replaced
     if (threadIdx.x == 0) mag[row] = mag_s;
-    for (int64_t j = threadIdx.x; j < T.rowlen; j += kThreads) {
-        const float gf = to_f32(g[base + j]);
-        const float cur = L.cbd[idx[base + j]] * mold;
+    float q = L.cbd[threadIdx.x] * mn;
+    if (QROUND) q = round_to<D>(q);
+    utab[threadIdx.x] = (q * ss) * T.lr;
+    __syncthreads();
+    const bool plain = (mn > 0.0f) && (mn < __builtin_inff());
+    const double rb = plain ? 1.0 / (double)mn : 0.0;
+    const bool fast = plain && max_probe <= 2;
+    auto second = [&](float gf, uint8_t& i, D& pe) {
+        const float cur = ctab[i];
         const float u = __builtin_fmaf(T.b1c, gf - cur, cur);
-        const float x = (mn > 0.0f) ? u / mn : 0.0f;
-        const int k = nearest_fast<false>(x, L.thr, L.bucket, K);
-        idx[base + j] = (uint8_t)k;
-        float q = L.cbd[k] * mn;
-        if (QROUND) q = round_to<D>(q);
-        const float uu = (q * ss) * T.lr;
-        float pf = to_f32(p[base + j]);
+        int k;
+        if (fast) {
+            k = nearest_two_probe<FINE>(div_by_block(u, rb), L.thr, L.bucket);
+        } else {
+            const float x = plain ? div_by_block(u, rb) : ((mn > 0.0f) ? u / mn : 0.0f);
+            k = nearest_fast<FINE>(x, L.thr, L.bucket, K);
+        }
+        i = (uint8_t)k;
+        float pf = to_f32(pe);
         if (T.do_wd) pf = round_to<D>(pf * T.wdf);
-        p[base + j] = from_f32<D>(pf - uu);
+        pe = from_f32<D>(pf - utab[k]);
+    };
+    for (int64_t v0 = threadIdx.x; v0 < nfull; v0 += U * kThreads) {
+        Vec<D, W> gv[U], pv[U];
+        Vec<uint8_t, W> iv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t e = min(v0 + u * kThreads, nfull - 1) * W;
+            gv[u] = sload<D, W, true>(g + e, 0);
+            iv[u] = sload<uint8_t, W, true>(idx + e, 0);
+            pv[u] = sload<D, W, true>(p + e, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (v0 + u * kThreads >= nfull) break;
+            const int64_t e = (v0 + u * kThreads) * W;
+#pragma unroll
+            for (int w = 0; w < W; ++w) second(to_f32(gv[u].v[w]), iv[u].v[w], pv[u].v[w]);
+            sstore<uint8_t, W, true>(idx + e, 0, iv[u]);
+            sstore<D, W, true>(p + e, 0, pv[u]);
+        }
     }
+    if (tail + threadIdx.x < T.rowlen) {
+        const int64_t e = tail + threadIdx.x;
+        second(to_f32(g[e]), idx[e], p[e]);
+    }
+}
+
+template <typename D, typename S>
+__global__ __launch_bounds__(kThreads) void k_gefen_step_long(const StepBatch B) {
+    constexpr bool kFine = step_fine<D>();
+    __shared__ LdsTables<kFine> L;
+    __shared__ float tabs[512], red[8];
+    int K;
+    load_tables<D, kThreads>(L, B.tables, K);
+    const int max_probe = kFine ? B.tables->max_probe_fine : B.tables->max_probe;
+    const int ti = find_task(B.wg_begin, B.ntasks);
+    const int64_t row = blockIdx.x - B.wg_begin[ti];
+    if (row >= B.t[ti].nrows) return;
+    step_long_row<D, S>(B.t[ti], L, tabs, red, K, max_probe, row);
+}
+
+// ---------------------------------------------------------------------------
+// Gefen step of many small tensors of all forms in one launch: a launch of a few
+// hundred workgroups or fewer takes as long as one of its rows (5 to 20 us, one after
+// the other), so tensors whose forms would take such launches share this one instead
+// (mark_mixed).  Vectors at any alignment (the aligned kernels' results, bit for bit),
+// one wave-unit per wave, no stepsize tables (their launch costs more than the square
+// roots that they save here).
+// A float32 MLP of 30 small tensors: three launches 15.2 us, one 7.4.  25 float16
+// tensors of odd sizes (11M elements): thirteen launches 108 us, one 45.
+enum StepForm : int16_t { kFormWide1, kFormWide1Tab, kFormWide2, kFormWide4, kFormRow2, kFormRow4, kFormWideP1, kFormWideP2,
+                          kFormHalfP1, kFormHalfP2, kFormOne, kFormOneP1, kFormOneP2, kFormLong };
+
+template <typename D, typename S>
+__global__ __launch_bounds__(kStepThreads) void k_gefen_step_mixed(const StepBatch B) {
+    constexpr bool kFine = step_fine<D>();
+    constexpr int kWide = sizeof(D) == 2 ? 8 : 4;
+    static_assert(kStepThreads == kThreads, "long rows take a workgroup of either kernel");
+    __shared__ LdsTables<kFine> L;
+    __shared__ float row_tab[kStepWaves][2][2][256];
+    __shared__ float red[8];
+    int K;
+    load_tables<D, kStepThreads>(L, B.tables, K);
+    const int max_probe = kFine ? B.tables->max_probe_fine : B.tables->max_probe;
+    const int ti = find_task(B.wg_begin, B.ntasks);
+    const StepTask T = B.t[ti];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t lw = blockIdx.x - B.wg_begin[ti];
+    const int64_t unit = lw * kStepWaves + wave;
+    float* tabs = row_tab[wave][0][0];
+#define GEFEN_FORM(F, W, R, P1, TAB) \
+    case F: step_unit<D, S, W, R, P1, TAB, (W > 1), true>(T, L, tabs, red, nullptr, K, max_probe, unit); break
+    switch (T.form) {
+        GEFEN_FORM(kFormWide1, kWide, 1, false, 0);
+        GEFEN_FORM(kFormWide1Tab, kWide, 1, false, 2);
+        GEFEN_FORM(kFormWide2, kWide, 2, false, 1);
+        GEFEN_FORM(kFormWide4, kWide, 4, false, 1);
+#define GEFEN_ROW_FORM(F, R) \
+    case F: step_unit<D, S, kWide, R, false, 3, true, true>(T, L, row_tab[0][0][0], red, nullptr, K, max_probe, lw); break
+        GEFEN_ROW_FORM(kFormRow2, 2);
+        GEFEN_ROW_FORM(kFormRow4, 4);
+#undef GEFEN_ROW_FORM
+        GEFEN_FORM(kFormWideP1, kWide, 1, true, 0);
+        GEFEN_FORM(kFormWideP2, kWide, 2, true, 0);
+        GEFEN_FORM(kFormHalfP1, 4, 1, true, 0);  // fp32 rows never ask for these two
+        GEFEN_FORM(kFormHalfP2, 4, 2, true, 0);
+        GEFEN_FORM(kFormOne, 1, 1, false, 0);
+        GEFEN_FORM(kFormOneP1, 1, 1, true, 0);
+        GEFEN_FORM(kFormOneP2, 1, 2, true, 0);
+        default: step_long_row<D, S>(T, L, row_tab[0][0][0], red, K, max_probe, lw); break;
+    }
+#undef GEFEN_FORM
 }
 
 // ---------------------------------------------------------------------------
@@ -1220,41 +1360,48 @@ __global__ __launch_bounds__(kThreads) void k_muon_packed(const MuonBatch B) {
 
 // kernel key: dtype pair, W, R (0 = long rows), P1
 struct Key {
-    int d, s, W, R, p1, tab, rag;
+    int d, s, W, R, p1, tab, rag, mixed;
     bool operator==(const Key& o) const {
-        return d == o.d && s == o.s && W == o.W && R == o.R && p1 == o.p1 && tab == o.tab && rag == o.rag;
+        return d == o.d && s == o.s && W == o.W && R == o.R && p1 == o.p1 && tab == o.tab && rag == o.rag &&
+               mixed == o.mixed;
     }
 };
 
 template <typename D, typename S>
 hipError_t launch_step(const Key& k, const StepBatch& b, int grid, hipStream_t st) {
-#define GEFEN_STEP_CASE(WW, RR, RAG)                                                                     \
-    if (k.W == WW && k.R == RR && k.rag == RAG) {                                                       \
-        if (k.p1) { /* ragged period-one rows have at most 256 elements: two vectors per lane */        \
-            if constexpr (!RAG || RR <= 2)                                                              \
-                hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, true, false, RAG>), dim3(grid), dim3(kStepThreads), 0, st, b);  \
-            else return hipErrorInvalidValue;                                                           \
-        } else if constexpr (WW > 1) {                                                                  \
-            if (k.tab) hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, false, true, RAG>), dim3(grid), dim3(kStepThreads), 0, st, b); \
-            else hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, false, false, RAG>), dim3(grid), dim3(kStepThreads), 0, st, b);     \
-        } else {                                                                                        \
-            hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, false, false, RAG>), dim3(grid), dim3(kStepThreads), 0, st, b);     \
-        }                                                                                               \
-        return hipGetLastError();                                                                       \
+#define GEFEN_STEP_CASE(WW, RR, PP, TT, RAG)                                                                            \
+    if (k.W == WW && k.R == RR && k.p1 == PP && k.tab == TT && k.rag == RAG) {                                          \
+        hipLaunchKernelGGL((k_gefen_step<D, S, WW, RR, PP, TT, RAG>), dim3(grid), dim3(kStepThreads), 0, st, b);        \
+        return hipGetLastError();                                                                                       \
+    }
+    if (k.mixed) {
+        hipLaunchKernelGGL((k_gefen_step_mixed<D, S>), dim3(grid), dim3(kStepThreads), 0, st, b);
+        return hipGetLastError();
     }
     if (k.R == 0) {
         hipLaunchKernelGGL((k_gefen_step_long<D, S>), dim3(grid), dim3(kThreads), 0, st, b);
         return hipGetLastError();
     }
     constexpr int kWide = sizeof(D) == 2 ? 8 : 4;
-    GEFEN_STEP_CASE(kWide, 1, false) GEFEN_STEP_CASE(kWide, 2, false)
-    GEFEN_STEP_CASE(kWide, 4, false) GEFEN_STEP_CASE(kWide, 8, false)
+    // rows of two or more vectors per lane own a wave and have tables
+#define GEFEN_STEP_ROWS(RAG)                                                                                            \
+    GEFEN_STEP_CASE(kWide, 1, false, 0, RAG) GEFEN_STEP_CASE(kWide, 1, false, 1, RAG)                                   \
+    GEFEN_STEP_CASE(kWide, 1, false, 2, RAG) GEFEN_STEP_CASE(kWide, 2, false, 1, RAG)                                   \
+    GEFEN_STEP_CASE(kWide, 4, false, 1, RAG)                                                                            \
+    GEFEN_STEP_CASE(kWide, 2, false, 3, RAG) GEFEN_STEP_CASE(kWide, 4, false, 3, RAG)                                   \
+    GEFEN_STEP_CASE(kWide, 1, true, 0, RAG) GEFEN_STEP_CASE(kWide, 2, true, 0, RAG)
+    GEFEN_STEP_ROWS(false) GEFEN_STEP_ROWS(true)
+    if constexpr (sizeof(D) == 4) { GEFEN_STEP_CASE(kWide, 8, false, 3, false) GEFEN_STEP_CASE(kWide, 8, false, 3, true) }
+    // period-one rows of more than 64 vectors (make_step_task bounds the ragged ones)
+    GEFEN_STEP_CASE(kWide, 4, true, 0, false) GEFEN_STEP_CASE(kWide, 8, true, 0, false)
     if constexpr (sizeof(D) == 2) {
-        GEFEN_STEP_CASE(4, 1, false) GEFEN_STEP_CASE(4, 2, false) GEFEN_STEP_CASE(4, 4, false) GEFEN_STEP_CASE(4, 8, false)
+        GEFEN_STEP_CASE(4, 1, true, 0, false) GEFEN_STEP_CASE(4, 2, true, 0, false)
+        GEFEN_STEP_CASE(4, 4, true, 0, false) GEFEN_STEP_CASE(4, 8, true, 0, false)
     }
-    GEFEN_STEP_CASE(kWide, 1, true) GEFEN_STEP_CASE(kWide, 2, true)
-    GEFEN_STEP_CASE(kWide, 4, true) GEFEN_STEP_CASE(kWide, 8, true)
-    GEFEN_STEP_CASE(1, 1, false) GEFEN_STEP_CASE(1, 2, false)  // rows shorter than a vector
+    // rows shorter than a vector
+    GEFEN_STEP_CASE(1, 1, false, 0, false) GEFEN_STEP_CASE(1, 1, true, 0, false)
+    GEFEN_STEP_CASE(1, 2, true, 0, false)
+#undef GEFEN_STEP_ROWS
 #undef GEFEN_STEP_CASE
     return hipErrorInvalidValue;
 }
