@@ -34,16 +34,34 @@ static_assert(offsetof(CodebookTables, bucket_fine) == 6176 && offsetof(Codebook
                   offsetof(CodebookTables, max_probe_fine) == 22592 && offsetof(CodebookTables, nb16) == 22608,
               "codebook table layout");
 
-__global__ __launch_bounds__(256) void k_prepare_codebook(const float* __restrict__ cb, int K,
-                                                          CodebookTables* __restrict__ T) {
+// #{k in [1, K) : thr[k] < x} by bisection, in the same eight steps for every x, so
+// that a thread's searches overlap.
+__device__ __forceinline__ int thresholds_below(const float* thr, int K, float x) {
+    int lo = 1, hi = K;  // first k in [1, K) with thr[k] >= x
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const int mid = (lo + hi) >> 1;  // <= 256
+        const bool open = lo < hi, less = thr[mid] < x;
+        lo = open && less ? mid + 1 : lo;
+        hi = open && !less ? mid : hi;
+    }
+    return lo - 1;
+}
+
+// One workgroup, as max_probe needs all cells.  Bound by the latency of the searches
+// (eight dependent LDS reads each): one after another in 256 threads 42 us; 1024
+// threads with their searches interleaved 11.
+constexpr int kPrepThreads = 1024;
+__global__ __launch_bounds__(kPrepThreads) void k_prepare_codebook(const float* __restrict__ cb, int K,
+                                                                   CodebookTables* __restrict__ T) {
     __shared__ float thr[260];
     __shared__ uint16_t bk[kFineCells + 1];
     __shared__ int probe_max, probe_max_fine;
     const int t = threadIdx.x;
-    T->cb[t] = t < K ? cb[t] : __builtin_inff();
+    if (t < 256) T->cb[t] = t < K ? cb[t] : __builtin_inff();
     if (t == 0) T->K = K;
     // thr[k], k = 1..K-1: largest x in (cb[k-1], cb[k]] where the left entry wins
-    for (int k = t; k < 260; k += 256) {
+    for (int k = t; k < 260; k += kPrepThreads) {
         float v = __builtin_inff();
         if (k >= 1 && k < K) {
             const float a = cb[k - 1], b = cb[k];
@@ -66,14 +84,12 @@ __global__ __launch_bounds__(256) void k_prepare_codebook(const float* __restric
     }
     __syncthreads();
     // bucket_fine[e] = #{k in 1..K-1 : thr[k] < -1 + e/4096}; bucket[e] = bucket8[e] = bucket_fine[2e]
-    for (int e = t; e <= kFineCells; e += 256) {
+#pragma unroll
+    for (int r = 0; r <= kFineCells / kPrepThreads; ++r) {
+        const int e = t + r * kPrepThreads;
         const float edge = -1.0f + (float)e * 0.000244140625f;  // exact: a multiple of 2^-12
-        int lo = 1, hi = K;  // first k in [1, K) with thr[k] >= edge
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (thr[mid] < edge) lo = mid + 1; else hi = mid;
-        }
-        const uint16_t c = (uint16_t)(lo - 1);
+        const uint16_t c = (uint16_t)thresholds_below(thr, K, edge);
+        if (e > kFineCells) continue;
         T->bucket_fine[e] = (uint8_t)c;  // c <= K - 1 <= 255
         if (!(e & 1)) {
             T->bucket[e >> 1] = c;
@@ -81,7 +97,7 @@ __global__ __launch_bounds__(256) void k_prepare_codebook(const float* __restric
         }
         bk[e] = c;
     }
-    for (int e = kFineCells + 1 + t; e < kFineBytes; e += 256) T->bucket_fine[e] = 0;
+    for (int e = kFineCells + 1 + t; e < kFineBytes; e += kPrepThreads) T->bucket_fine[e] = 0;
     if (t < kBucket8Bytes - 4097) T->bucket8[4097 + t] = 0;
     if (t < 3) T->bucket[4097 + t] = 0;
     if (t == 0) probe_max = probe_max_fine = 0;
@@ -89,7 +105,7 @@ __global__ __launch_bounds__(256) void k_prepare_codebook(const float* __restric
     // a search from bucket b (one below x's bucket) meets the thresholds in
     // [edge_b, edge_b+2); past the last edges it meets every finite one left
     int worst = 0, worst_fine = 0;
-    for (int b = t; b <= kFineCells; b += 256) {
+    for (int b = t; b <= kFineCells; b += kPrepThreads) {
         const int hi = (b + 2 <= kFineCells) ? (int)bk[b + 2] : (K - 1);
         const int n = hi - (int)bk[b];
         worst_fine = n > worst_fine ? n : worst_fine;
@@ -99,28 +115,25 @@ __global__ __launch_bounds__(256) void k_prepare_codebook(const float* __restric
             worst = nc > worst ? nc : worst;
         }
     }
-    atomicMax(&probe_max, worst);
-    atomicMax(&probe_max_fine, worst_fine);
+    worst = (int)wave_group_max_u32((uint32_t)worst, 64);  // counts: non-negative where thr is sorted
+    worst_fine = (int)wave_group_max_u32((uint32_t)worst_fine, 64);
+    if ((t & 63) == 0) {
+        atomicMax(&probe_max, worst);
+        atomicMax(&probe_max_fine, worst_fine);
+    }
     __syncthreads();
     if (t == 0) {
         T->max_probe = (bk[0] != 0) ? 1 << 20 : probe_max;
         T->max_probe_fine = (bk[0] != 0) ? 1 << 20 : probe_max_fine;
     }
     // nb16: #{k in 1..K-1 : thr[k] < x} for the bf16 values x of the table
-    for (int i = t; i < kNb16Bytes; i += 256) {
-        uint8_t c = 0;
-        if (i < 2 * (int)kNb16Side) {
-            const uint32_t bits = i >= (int)kNb16Side ? kNb16Lo + (uint32_t)(i - (int)kNb16Side)
-                                                      : 0x8000u | (kNb16Lo + kNb16Side - 1u - (uint32_t)i);
-            const float x = __uint_as_float(bits << 16);
-            int lo = 1, hi = K;  // first k in [1, K) with thr[k] >= x
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (thr[mid] < x) lo = mid + 1; else hi = mid;
-            }
-            c = (uint8_t)(lo - 1);
-        }
-        T->nb16[i] = c;
+#pragma unroll
+    for (int r = 0; r < (kNb16Bytes + kPrepThreads - 1) / kPrepThreads; ++r) {
+        const int i = t + r * kPrepThreads;
+        const uint32_t bits = i >= (int)kNb16Side ? kNb16Lo + (uint32_t)(i - (int)kNb16Side)
+                                                  : 0x8000u | (kNb16Lo + kNb16Side - 1u - (uint32_t)i);
+        const uint8_t c = (uint8_t)thresholds_below(thr, K, __uint_as_float(bits << 16));
+        if (i < kNb16Bytes) T->nb16[i] = i < 2 * (int)kNb16Side ? c : 0;
     }
 }
 
@@ -853,7 +866,7 @@ extern "C" int gefen_prepare_codebook(const float* codebook, int codebook_size, 
     if (!codebook || !tables) return fail_inval("null pointer");
     if (codebook_size <= 0 || codebook_size > 256)
         return fail_inval("Expected codebook to have at most 256 entries, got %d", codebook_size);
-    hipLaunchKernelGGL(k_prepare_codebook, dim3(1), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), codebook,
+    hipLaunchKernelGGL(k_prepare_codebook, dim3(1), dim3(kPrepThreads), 0, reinterpret_cast<hipStream_t>(stream), codebook,
                        codebook_size, static_cast<CodebookTables*>(tables));
     return launch_status("gefen_prepare_codebook");
 }

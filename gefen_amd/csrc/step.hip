@@ -83,24 +83,43 @@ __global__ __launch_bounds__(256) void k_block_stepsize(const V* __restrict__ vm
 }
 
 // ---------------------------------------------------------------------------
-// vmean only (automatic_vmean_update): one lane group per row, streaming.
+// vmean only (automatic_vmean_update): one lane group per row, streaming.  16-byte
+// vectors at any alignment, four in flight per lane; the elements after a row's last
+// whole vector go one per lane.  40000 rows of 768 bf16 (61 MB): 36 us with one element
+// per lane and load, 15.6 now.
 template <typename G, typename S>
 __global__ __launch_bounds__(kThreads) void k_vmean(S* __restrict__ vm, const G* __restrict__ g,
                                                      int64_t nrows, int64_t period, int lpr_log2,
                                                      float b2, float omb2) {
+    constexpr int W = sizeof(G) == 2 ? 8 : 4, U = 4;
     const int lane = threadIdx.x & 63;
     const int lpr = 1 << lpr_log2;
     const int lir = lane & (lpr - 1);
     const int64_t unit = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int64_t row = unit * (64 >> lpr_log2) + (lane >> lpr_log2);
     const bool active = row < nrows;
+    const int64_t nfull = period / W;
     float s = 0.0f;
     if (active) {
-        const int64_t base = row * period;
-        for (int64_t j = lir; j < period; j += lpr) {
-            const float gf = to_f32(g[base + j]);
-            const float sq = gf * gf;
-            s = s + sq;
+        const G* gr = g + row * period;
+        for (int64_t v0 = lir; v0 < nfull; v0 += U * lpr) {
+            Vec<G, W> x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[u] = sload<G, W, true>(gr + min(v0 + u * lpr, nfull - 1) * W, 0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                float sv = 0.0f;
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    const float gf = to_f32(x[u].v[w]);
+                    sv = __builtin_fmaf(gf, gf, sv);
+                }
+                s = s + (v0 + u * lpr < nfull ? sv : 0.0f);
+            }
+        }
+        for (int64_t e = nfull * W + lir; e < period; e += lpr) {
+            const float gf = to_f32(gr[e]);
+            s = __builtin_fmaf(gf, gf, s);
         }
     }
     s = group_sum(s, lpr);
@@ -1382,7 +1401,8 @@ extern "C" int gefen_automatic_vmean_update(void* vmean, int vmean_dtype, const 
     if (num_blocks < 0 || period <= 0) return fail_inval("Expected a positive period, got %lld", (long long)period);
     if (num_blocks == 0) return GEFEN_OK;
     if (!vmean || !grad) return fail_inval("null tensor pointer");
-    const int l2 = lpr_log2_for(period);
+    // a lane per vector, and enough of them for the rest of a short row
+    const int l2 = lpr_log2_for(grad_dtype == GEFEN_F32 ? (period + 3) / 4 : (period + 7) / 8);
     const int64_t rpw = 64 >> l2;
     const int64_t units = (num_blocks + rpw - 1) / rpw;
     const int64_t grid = (units + 3) / 4;

@@ -82,7 +82,8 @@ __device__ __forceinline__ void sstore(T* base, uint32_t elem, const Vec<T, W>& 
 // First element of vector v of a row.  RAG: rows that are no whole number of
 // vectors, or are not aligned for them: the last vector is shifted back to end with
 // the row, so some elements are in two vectors.  Both lanes load the old values
-// before either stores (every load of a row precedes its stores in the wave), form
+// before either stores (every load of a row precedes its stores in the wave, or the
+// barrier before them in the workgroup), form
 // the same results and store the same bytes; only the sum of squares leaves the
 // repeats out.
 template <bool RAG, int W>
