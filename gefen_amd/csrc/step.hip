@@ -284,7 +284,7 @@ constexpr int64_t kMixedElems = 4 << 20;
 
 // The k_gefen_step_mixed form of a task with this key, or -1.
 int mixed_form(const Key& k) {
-    if (k.R == 0) return kFormLong;
+    if (k.R == 0) return k.W == kLongWide ? -1 : kFormLong;
     if (k.W == 1) return !k.p1 ? kFormOne : (k.R == 1 ? kFormOneP1 : kFormOneP2);
     if (k.p1 && k.W != (dtype_size(k.d) == 2 ? 8 : 4)) return k.R == 1 ? kFormHalfP1 : (k.R == 2 ? kFormHalfP2 : -1);
     if (k.p1) return k.R == 1 ? kFormWideP1 : (k.R == 2 ? kFormWideP2 : -1);
@@ -464,7 +464,11 @@ int make_step_task(const gefen_step_task& in, int mode, const float* stepsize, P
         tab = 3;
         R = nvec <= 512 ? 2 : (nvec <= 1024 ? 4 : 8);
     }
-    Key k{in.param_dtype, in.state_dtype, R == 0 ? 1 : W, R, p1 ? 1 : 0, tab, rag && R != 0, 0};
+    // Long rows are few, so one of 65536 elements or more takes 1024 threads: 24M bf16
+    // elements in rows of 66000, 200000 and 2M take 64, 76 and 636 us, with 256 threads
+    // 80, 200 and 1908; in rows of 16384 74 us against 48.
+    const int long_w = rowlen >= 65536 ? kLongWide : 1;
+    Key k{in.param_dtype, in.state_dtype, R == 0 ? long_w : W, R, p1 ? 1 : 0, tab, rag && R != 0, 0};
     out.galign = (rag || R == 0 ? 1 : W) * dsz;
     StepTask& t = out.task;
     memset(&t, 0, sizeof(t));

@@ -609,14 +609,13 @@ __global__ __launch_bounds__(kStepThreads) void k_gefen_step(const StepBatch B) 
 // lane.  So four 16-byte vectors per lane are in flight at a time, at any alignment;
 // the elements after the row's last whole vector (fewer than W) go one per lane, as
 // the second sweep may not read what another lane has written.  tabs: 512 floats,
-// the row's tables as in step_unit; red: 8 floats.
+// the row's tables as in step_unit; red: a maximum and a sum per wave.  NT: threads.
 // 32M bf16 elements in rows of 33000: 164 us with one element per lane and load, 77 now.
-template <typename D, typename S, bool FINE>
+template <typename D, typename S, int NT, bool FINE>
 __device__ __forceinline__ void step_long_row(const StepTask& T, const LdsTables<FINE>& L, float* tabs, float* red, int K,
                                               int max_probe, int64_t row) {
     constexpr bool QROUND = sizeof(D) == sizeof(S);
     constexpr int W = sizeof(D) == 2 ? 8 : 4, U = 4;
-    static_assert(kThreads == 256, "one thread per codeword, four waves");
     float* ctab = tabs;
     float* utab = tabs + 256;
     const int64_t base = row * T.rowlen;
@@ -628,7 +627,7 @@ __device__ __forceinline__ void step_long_row(const StepTask& T, const LdsTables
     const int64_t nfull = T.rowlen / W, tail = nfull * W;
     const float mold = to_f32(mag[row]);
     const float vold = T.mode == kStepsizeGiven ? T.stepsize[row] : to_f32(vm[row]);
-    ctab[threadIdx.x] = L.cbd[threadIdx.x] * mold;
+    if (threadIdx.x < 256) ctab[threadIdx.x] = L.cbd[threadIdx.x] * mold;
     __syncthreads();  // also: every thread has read mag[row] and vm[row]
     float mx = 0.0f, sumsq = 0.0f;
     auto first = [&](float gf, uint8_t i, bool in) {
@@ -637,18 +636,18 @@ __device__ __forceinline__ void step_long_row(const StepTask& T, const LdsTables
         mx = nanmax(mx, in ? fabsf(u) : 0.0f);
         return gf * gf;
     };
-    for (int64_t v0 = threadIdx.x; v0 < nfull; v0 += U * kThreads) {
+    for (int64_t v0 = threadIdx.x; v0 < nfull; v0 += U * NT) {
         Vec<D, W> gv[U];
         Vec<uint8_t, W> iv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int64_t e = min(v0 + u * kThreads, nfull - 1) * W;
+            const int64_t e = min(v0 + u * NT, nfull - 1) * W;
             gv[u] = sload<D, W, true>(g + e, 0);
             iv[u] = sload<uint8_t, W, true>(idx + e, 0);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const bool in = v0 + u * kThreads < nfull;
+            const bool in = v0 + u * NT < nfull;
             float s = 0.0f;
 #pragma unroll
             for (int w = 0; w < W; ++w) s = s + first(to_f32(gv[u].v[w]), iv[u].v[w], in);
@@ -660,12 +659,17 @@ __device__ __forceinline__ void step_long_row(const StepTask& T, const LdsTables
     mx = group_max(mx, 64);
     sumsq = group_sum(sumsq, 64);
     const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) { red[wave] = mx; red[4 + wave] = sumsq; }
+    if ((threadIdx.x & 63) == 0) { red[wave] = mx; red[NT / 64 + wave] = sumsq; }
     __syncthreads();
-    mx = nanmax(nanmax(red[0], red[1]), nanmax(red[2], red[3]));
+    mx = red[0];
+    float tot = red[NT / 64];
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) {
+        mx = nanmax(mx, red[w]);
+        tot = tot + red[NT / 64 + w];
+    }
     float ss = vold;
     if (T.mode == kVmeanUpdate) {
-        const float tot = (red[4] + red[5]) + (red[6] + red[7]);
         const S vnew = from_f32<S>(__builtin_fmaf(mean_of(tot, T.period), T.omb2, vold * T.b2));
         ss = stepsize_of(to_f32(vnew), T);
         if (threadIdx.x == 0) vm[row] = vnew;
@@ -675,9 +679,11 @@ __device__ __forceinline__ void step_long_row(const StepTask& T, const LdsTables
     const S mag_s = from_f32<S>(mx);
     const float mn = to_f32(mag_s);
     if (threadIdx.x == 0) mag[row] = mag_s;
-    float q = L.cbd[threadIdx.x] * mn;
-    if (QROUND) q = round_to<D>(q);
-    utab[threadIdx.x] = (q * ss) * T.lr;
+    if (threadIdx.x < 256) {
+        float q = L.cbd[threadIdx.x] * mn;
+        if (QROUND) q = round_to<D>(q);
+        utab[threadIdx.x] = (q * ss) * T.lr;
+    }
     __syncthreads();
     const bool plain = (mn > 0.0f) && (mn < __builtin_inff());
     const double rb = plain ? 1.0 / (double)mn : 0.0;
@@ -697,20 +703,20 @@ __device__ __forceinline__ void step_long_row(const StepTask& T, const LdsTables
         if (T.do_wd) pf = round_to<D>(pf * T.wdf);
         pe = from_f32<D>(pf - utab[k]);
     };
-    for (int64_t v0 = threadIdx.x; v0 < nfull; v0 += U * kThreads) {
+    for (int64_t v0 = threadIdx.x; v0 < nfull; v0 += U * NT) {
         Vec<D, W> gv[U], pv[U];
         Vec<uint8_t, W> iv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int64_t e = min(v0 + u * kThreads, nfull - 1) * W;
+            const int64_t e = min(v0 + u * NT, nfull - 1) * W;
             gv[u] = sload<D, W, true>(g + e, 0);
             iv[u] = sload<uint8_t, W, true>(idx + e, 0);
             pv[u] = sload<D, W, true>(p + e, 0);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (v0 + u * kThreads >= nfull) break;
-            const int64_t e = (v0 + u * kThreads) * W;
+            if (v0 + u * NT >= nfull) break;
+            const int64_t e = (v0 + u * NT) * W;
 #pragma unroll
             for (int w = 0; w < W; ++w) second(to_f32(gv[u].v[w]), iv[u].v[w], pv[u].v[w]);
             sstore<uint8_t, W, true>(idx + e, 0, iv[u]);
@@ -723,18 +729,18 @@ __device__ __forceinline__ void step_long_row(const StepTask& T, const LdsTables
     }
 }
 
-template <typename D, typename S>
-__global__ __launch_bounds__(kThreads) void k_gefen_step_long(const StepBatch B) {
+template <typename D, typename S, int NT>
+__global__ __launch_bounds__(NT) void k_gefen_step_long(const StepBatch B) {
     constexpr bool kFine = step_fine<D>();
     __shared__ LdsTables<kFine> L;
-    __shared__ float tabs[512], red[8];
+    __shared__ float tabs[512], red[NT / 32];
     int K;
-    load_tables<D, kThreads>(L, B.tables, K);
+    load_tables<D, NT>(L, B.tables, K);
     const int max_probe = kFine ? B.tables->max_probe_fine : B.tables->max_probe;
     const int ti = find_task(B.wg_begin, B.ntasks);
     const int64_t row = blockIdx.x - B.wg_begin[ti];
     if (row >= B.t[ti].nrows) return;
-    step_long_row<D, S>(B.t[ti], L, tabs, red, K, max_probe, row);
+    step_long_row<D, S, NT>(B.t[ti], L, tabs, red, K, max_probe, row);
 }
 
 // ---------------------------------------------------------------------------
@@ -785,7 +791,7 @@ __global__ __launch_bounds__(kStepThreads) void k_gefen_step_mixed(const StepBat
         GEFEN_FORM(kFormOne, 1, 1, false, 0);
         GEFEN_FORM(kFormOneP1, 1, 1, true, 0);
         GEFEN_FORM(kFormOneP2, 1, 2, true, 0);
-        default: step_long_row<D, S>(T, L, row_tab[0][0][0], red, K, max_probe, lw); break;
+        default: step_long_row<D, S, kThreads>(T, L, row_tab[0][0][0], red, K, max_probe, lw); break;
     }
 #undef GEFEN_FORM
 }
@@ -1360,6 +1366,8 @@ __global__ __launch_bounds__(kThreads) void k_muon_packed(const MuonBatch B) {
 // Launch templates (instantiated per dtype pair by GEFEN_STEP_INSTANCES)
 
 // kernel key: dtype pair, W, R (0 = long rows), P1
+constexpr int kLongWide = 1024;  // W of a long row's key (R = 0) that takes 1024 threads
+
 struct Key {
     int d, s, W, R, p1, tab, rag, mixed;
     bool operator==(const Key& o) const {
@@ -1380,7 +1388,8 @@ hipError_t launch_step(const Key& k, const StepBatch& b, int grid, hipStream_t s
         return hipGetLastError();
     }
     if (k.R == 0) {
-        hipLaunchKernelGGL((k_gefen_step_long<D, S>), dim3(grid), dim3(kThreads), 0, st, b);
+        if (k.W == kLongWide) hipLaunchKernelGGL((k_gefen_step_long<D, S, 1024>), dim3(grid), dim3(1024), 0, st, b);
+        else hipLaunchKernelGGL((k_gefen_step_long<D, S, kThreads>), dim3(grid), dim3(kThreads), 0, st, b);
         return hipGetLastError();
     }
     constexpr int kWide = sizeof(D) == 2 ? 8 : 4;
