@@ -510,7 +510,8 @@ __device__ __forceinline__ void step_unit(const StepTask& T, const LdsTables<FIN
             upd[j][w] = u;
             const uint32_t key = abs_key(u);
             mxk = key > mxk ? key : mxk;
-            if (!P1) sj = __builtin_fmaf(gf, RAG && w < skip ? 0.0f : gf, sj);
+            const float gs = RAG && w < skip ? 0.0f : gf;  // both factors: an infinity times 0 is NaN
+            if (!P1) sj = __builtin_fmaf(gs, gs, sj);
         }
         if (!P1) sumsq = sumsq + ((lir + j * lpr < T.nvec) ? sj : 0.0f);
     }

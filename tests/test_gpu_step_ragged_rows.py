@@ -12,6 +12,8 @@ import torch
 
 import gpu_util as gu
 from gefen_amd import _lib
+from gefen_amd import synthetic as syn
+from oracle import oracle as orc
 from test_gpu_step import _codebook, _run_case, _tables
 
 pytestmark = pytest.mark.gpu
@@ -33,6 +35,69 @@ def test_odd_block_rows_match_oracle(dt, sdt):
 @pytest.mark.parametrize("n", [9 * 1009, 251 * 67, 253 * 1013, 17 * 1021, 5 * 1013, 3 * 1019, 1021, 250 * 1009])
 def test_odd_period_one_rows_match_oracle(dt, sdt, n):
     _run_case("rag_p1_{}_{}_{}".format(dt, sdt, n), dt, sdt, n, 1, 0.05)
+
+
+INF = {"bf16": 0x7F80, "f16": 0x7C00, "f32": np.float32(np.inf)}
+NAN = {"bf16": 0x7FC0, "f16": 0x7E00, "f32": np.float32(np.nan)}
+
+
+# lane groups, whole waves of one to four vectors per lane, workgroup rows
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("dt,sdt,length", [(dt, sdt, length) for dt, sdt in
+                                           [("bf16", "bf16"), ("f16", "f16"), ("bf16", "f32"), ("f32", "f32")]
+                                           for length in ([12, 250, 511, 1021, 2047, 4095] if dt != "f32" else
+                                                          [6, 127, 255, 511, 1021, 2045])])
+def test_infinite_gradients_in_repeated_elements(dt, sdt, length, shared):
+    """Elements that the shifted last vector repeats hold +-inf, NaN and values whose
+    square overflows: vmean is inf, NaN and inf, as the oracle's, in the tensor's own
+    kernel and in a shared launch."""
+    wide = 4 if dt == "f32" else 8
+    rows = 9
+    n = rows * length
+    nvec = -(-length // wide)
+    first, last = length - wide, (nvec - 1) * wide - 1  # the repeated elements of a row
+    assert first <= last
+    cb = _codebook()
+    tables = _tables(torch.from_numpy(cb).to("cuda:0"))
+    g = syn.round_to(syn.row_scaled_normal(5, length, rows, length, -9, -4), dt).reshape(-1).copy()
+    g = g.view(np.uint16) if g.dtype == np.float16 else g
+    sign = np.float32(-np.inf) if dt == "f32" else INF[dt] | 0x8000
+    big = np.float32(3e38) if dt == "f32" else INF[dt] - 1  # the largest finite value
+    for row, at, value in ((1, first, INF[dt]), (2, last, sign), (4, first, NAN[dt]), (6, last, big), (8, first, INF[dt])):
+        g[row * length + at] = value
+    p = syn.round_to(syn.normal(syn.make_key(6, length), n) * 0.02, dt)
+    p = p.view(np.uint16) if p.dtype == np.float16 else p
+    ref = {"p": p.copy(), "idx": np.zeros(n, np.uint8), "mag": np.zeros(rows, orc.NP_STORAGE[sdt]),
+           "v": np.zeros(rows, orc.NP_STORAGE[sdt])}
+    dev = {"p": gu.to_dev(p, dt), "g": gu.to_dev(g, dt), "idx": torch.zeros(n, dtype=torch.uint8, device="cuda:0"),
+           "mag": torch.zeros(rows, dtype=gu.TORCH[sdt], device="cuda:0"),
+           "v": torch.zeros(rows, dtype=gu.TORCH[sdt], device="cuda:0")}
+    # a tensor of one-element rows asks for another kernel, so that the two share a launch
+    other = {"p": torch.zeros(96, dtype=gu.TORCH[dt], device="cuda:0"), "g": torch.ones(96, dtype=gu.TORCH[dt], device="cuda:0"),
+             "idx": torch.zeros(96, dtype=torch.uint8, device="cuda:0"),
+             "mag": torch.zeros(32, dtype=gu.TORCH[sdt], device="cuda:0"),
+             "v": torch.zeros(32, dtype=gu.TORCH[sdt], device="cuda:0")}
+    tasks = np.zeros(1 + shared, dtype=_lib.STEP_TASK)
+    for t, d, size, period in zip(tasks, (dev, other), (n, 96), (length, 3)):
+        t["p"], t["grad"], t["m_codebook"] = d["p"].data_ptr(), d["g"].data_ptr(), d["idx"].data_ptr()
+        t["m_magnitude"], t["vmean"] = d["mag"].data_ptr(), d["v"].data_ptr()
+        t["numel"], t["period"] = size, period
+        t["param_dtype"], t["state_dtype"] = gu.CODE[dt], gu.CODE[sdt]
+        t["beta1"], t["beta2"], t["lr"], t["eps"] = 0.9, 0.999, 1e-3, 1e-8
+        t["bias_correction_1"], t["bias_correction_2"] = 0.1, 1 - 0.999
+    _lib.check(_lib.load().gefen_step_tasks(tasks.ctypes.data, len(tasks), tables.data_ptr(), gu.stream()))
+    rc = orc.lib().orc_gefen_step(gu.CODE[dt], gu.CODE[sdt], orc._ptr(ref["p"]), orc._ptr(np.ascontiguousarray(g)),
+                                  orc._ptr(ref["idx"]), orc._ptr(ref["mag"]), orc._ptr(ref["v"]), n, length, 0,
+                                  orc._ptr(cb), cb.size, 0.9, 0.999, 1e-3, 1e-8, 0.0, 0.1, 1 - 0.999, 1)
+    assert rc == 0
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(gu.to_np(dev["idx"]), ref["idx"])
+    np.testing.assert_array_equal(orc.to_f32(gu.to_np(dev["mag"]), sdt), orc.to_f32(ref["mag"], sdt))
+    v, w = orc.to_f32(gu.to_np(dev["v"]), sdt), orc.to_f32(ref["v"], sdt)
+    assert np.isinf(w[[1, 2, 8]]).all() and np.isnan(w[4]), w
+    np.testing.assert_array_equal(np.isnan(v), np.isnan(w))
+    np.testing.assert_array_equal(np.isinf(v), np.isinf(w))
+    np.testing.assert_array_equal(np.isnan(orc.to_f32(gu.to_np(dev["p"]), dt)), np.isnan(orc.to_f32(ref["p"], dt)))
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
