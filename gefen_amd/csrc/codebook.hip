@@ -337,7 +337,7 @@ __global__ void k_accumulate_counts(float* __restrict__ acc, const int64_t* __re
 // ---------------------------------------------------------------------------
 // exact DP workspace:
 //   header  int32[64]      : [0] N active bins, [1] status (0 ok, 1 padded done, 2 empty),
-//                            [2..3] kDpSlack * sum(w) as a double
+//                            [2..3] the cut's slack as a double (dp_slack)
 //   pw, pwx, pwx2          : double[bins + 1] each (prefix sums, sequential order)
 //   dp                     : double[(K + 1) * (bins + 1)], level-major
 //   bt                     : int32[(K + 1) * (bins + 1)]
@@ -363,7 +363,23 @@ struct DpLayout {
 
 constexpr int kDpMaxBins = 4096;
 constexpr int kDpInitThreads = 256;
-constexpr double kDpSlack = 0x1p-28;  // see k_dp_level
+
+// How much a segment's cost alone may exceed the best candidate before longer segments
+// are left out (k_dp_level), for counts of this sum W and smallest value m; infinite,
+// which leaves nothing out, where no such bound holds.  In exact arithmetic a segment's
+// cost never falls when it grows, and dp >= 0.  In float64 a prefix sum of up to 4096
+// counts is within 2^-41 W of the exact one (|x| < 1), so a segment's sums sw, swx and
+// swx2 are within h = 2^-40 W of theirs.  The error of swx^2 / sw is then at most
+// h (3 sw + h) / (sw - h), 4 h where sw >= m >= 5 h, a cost's 5 h < 2^-37 W and a dp
+// value's (up to 256 costs) 2^-29 W: 2^-28 W covers both with room, and is far below the
+// costs it is compared with (5e-6 W for 256 even levels).  Where m < 5 h the divisor can
+// cancel, and a cost be off by any amount: counts that span about 15 decades and more gave
+// another codebook than the full search.  2^37 below is 2^40 / 5 rounded down; an
+// optimizer's counts, whole numbers, exceed it only past 1.4e11 elements.  256 codewords
+// of 4096 full bins: 1.7 ms with the bound, 6.5 without.
+__device__ __forceinline__ double dp_slack(double W, double m) {
+    return W <= 0x1p37 * m ? 0x1p-28 * W : __builtin_inf();
+}
 
 // The first `n` values of v (LDS, n <= kDpMaxK) in ascending order, equal ones as
 // they stood (an insertion sort; in parallel it is only checked, since codewords
@@ -400,6 +416,7 @@ __global__ __launch_bounds__(kDpInitThreads) void k_dp_init(const float* __restr
     constexpr int kPer = kDpMaxBins / kDpInitThreads;  // bins per thread
     __shared__ __attribute__((aligned(16))) double sums[3][kDpMaxBins];
     __shared__ int wave_total[kDpInitThreads / 64];
+    __shared__ float wave_least[kDpInitThreads / 64];
     __shared__ float sorted[kDpMaxK];
     __shared__ int unsorted;
     int32_t* hdr = reinterpret_cast<int32_t*>(ws);
@@ -410,13 +427,16 @@ __global__ __launch_bounds__(kDpInitThreads) void k_dp_init(const float* __restr
     float* cw = reinterpret_cast<float*>(ws + L.cw);
     const int t = threadIdx.x, lane = t & 63;
     const int b0 = t * kPer;  // this thread's bins b0 .. b0 + kPer - 1 (in order)
-    float mine[kPer];
+    float mine[kPer], least = __builtin_inff();
     int cnt = 0;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
         mine[k] = b0 + k < bins ? counts[b0 + k] : 0.0f;
         cnt += mine[k] > 0.0f ? 1 : 0;
+        if (mine[k] > 0.0f) least = fminf(least, mine[k]);
     }
+    for (int off = 32; off > 0; off >>= 1) least = fminf(least, __shfl_xor(least, off, 64));
+    if (lane == 0) wave_least[t >> 6] = least;
     int incl = cnt;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -492,7 +512,8 @@ __global__ __launch_bounds__(kDpInitThreads) void k_dp_init(const float* __restr
     if (t == 0) {
         hdr[0] = N;
         hdr[1] = N == 0 ? 2 : (K > N ? 1 : 0);
-        *reinterpret_cast<double*>(hdr + 2) = N ? kDpSlack * sums[0][N - 1] : 0.0;
+        for (int w = 1; w < kDpInitThreads / 64; ++w) least = fminf(least, wave_least[w]);
+        *reinterpret_cast<double*>(hdr + 2) = N ? dp_slack(sums[0][N - 1], (double)least) : 0.0;
     }
 }
 static_assert(kDpMaxBins % kDpInitThreads == 0, "whole bins per thread");
@@ -505,15 +526,8 @@ static_assert(kDpInitThreads >= kDpMaxK && kDpInitThreads / 64 >= 3, "one codewo
 // minimum.
 //
 // A wave takes one end and looks at the starts from the nearest one down, 128 at
-// a time, until the cost of the segment alone exceeds the best candidate by
-// kDpSlack * sum(w).  In exact arithmetic a segment's cost never falls when it
-// grows and dp >= 0, so no start further down can be as good.  In float64 each of
-// the three prefix sums is within 4096 * 2^-53 * sum(w) of the exact sum (|x| < 1,
-// the terms themselves are exact), which moves a cost by less than 2^-38 sum(w) and a
-// dp value of up to 256 costs by less than 2^-30 sum(w); 2^-28 covers both with
-// room, and is still far below the costs it is compared with (5e-6 sum(w) for 256
-// even levels).  A count that is not finite gives an infinite or NaN slack, and
-// then nothing is cut.
+// a time, until the cost of the segment alone exceeds the best candidate by the
+// slack: then no start further down can be as good (dp_slack).
 //
 // The optimal segment spans about N / c points, and the bound cuts at N / c^(2/3),
 // so most levels are one or two passes per end, bound by the launch and one trip to

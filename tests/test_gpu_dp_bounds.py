@@ -51,3 +51,20 @@ def test_codebook_equals_the_oracle(kind, bins, k, force):
     got = exact_dp_from_counts(torch.from_numpy(counts).to("cuda:0"), k, force).cpu().numpy()
     ref = orc.exact_dp(counts, k, force)
     np.testing.assert_array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("decades", [9, 14, 15, 17, 25])
+@pytest.mark.parametrize("bins,k", [(1024, 4), (1024, 16), (512, 64), (512, 200)])
+def test_counts_over_many_decades(bins, k, decades):
+    """Log-uniform counts.  Over 9 decades starts are left out; from 14 on none are, and from
+    about 15 on none may be: the rounding of the prefix sums exceeds the smallest counts, so
+    that a segment's computed cost no longer grows with the segment."""
+    from gefen_amd.quantization import exact_dp_from_counts
+
+    for seed in range(4):
+        rng = np.random.default_rng(seed * 1000 + k + bins)
+        counts = (10.0 ** (rng.random(bins) * decades - decades / 2)).astype(np.float32)
+        got = exact_dp_from_counts(torch.from_numpy(counts).to("cuda:0"), k, True).cpu().numpy()
+        ref = orc.exact_dp(counts, k, True)
+        # codewords of segments whose weights cancel are infinite or NaN, in an order of their own
+        np.testing.assert_array_equal(np.sort(got), np.sort(ref), err_msg="seed {}".format(seed))
