@@ -169,7 +169,7 @@ class GefenMuon(Gefen):
         # buffer: the momentum kernel writes each one's Nesterov blend into its
         # slice and Newton-Schulz runs on the whole stack.  Sides that fill no tile run
         # zero-padded (one call per stack, its update included).
-        from gefen_amd.newton_schulz import batched_shape_ok, padded_shape_ok
+        from gefen_amd.newton_schulz import batched_shape_ok, padded_chunk, padded_shape_ok
 
         stacks = {}
         padded = {}
@@ -280,9 +280,12 @@ class GefenMuon(Gefen):
             t["weight_decay"] = wd
             t["adjusted_lr"] = adjusted
         pruns = []
+        chunks = {key: padded_chunk(len(idx), key[0], key[1]) for key, idx in padded.items()}
+        # the stacks run one after the other and share a workspace
+        work = torch.empty(max((nbytes for _, nbytes in chunks.values()), default=0), dtype=torch.uint8, device=dev)
         for key, idx in padded.items():
             _check_ns_args(key[3], key[4])
-            pruns.append(_PaddedStack(key, idx, bufs[key], sum_index[key]))
+            pruns.append(_PaddedStack(key, idx, bufs[key], sum_index[key], chunks[key][0], work))
             pruns[-1].run(apply, sumsq)
         rest = np.ascontiguousarray(apply[[i for i in range(len(items)) if i not in in_padded]])
         with torch.cuda.device(dev):
@@ -318,24 +321,24 @@ class GefenMuon(Gefen):
 
 class _PaddedStack:
     """A stack of matrices whose sides fill no tile: Newton-Schulz on zero-padded
-    copies and the parameters' updates, one library call per step
-    (gefen_newton_schulz_apply)."""
+    copies and the parameters' updates (gefen_newton_schulz_apply), `chunk` matrices
+    per library call, which share the workspace `work`."""
 
-    def __init__(self, key, idx, buf, index):
+    def __init__(self, key, idx, buf, index, chunk, work):
         (self.rows, self.cols, _, self.coeffs, self.steps, self.eps, _) = key
-        self.idx, self.buf, self.index = idx, buf, index
-        nbytes = int(_lib.load().gefen_newton_schulz_workspace_size(len(idx), self.rows, self.cols))
-        self.work = torch.empty(nbytes, dtype=torch.uint8, device=buf.device)
+        self.idx, self.buf, self.index, self.chunk, self.work = idx, buf, index, chunk, work
 
     def run(self, apply, sumsq):
         tasks = np.ascontiguousarray(apply[self.idx])
         a, b, c = self.coeffs
         with torch.cuda.device(self.buf.device):
-            rc = _lib.load().gefen_newton_schulz_apply(
-                self.buf.data_ptr(), len(self.idx), self.rows, self.cols, a, b, c, self.steps, float(self.eps),
-                sumsq.data_ptr(), self.index.data_ptr(), self.work.data_ptr(), tasks.ctypes.data,
-                torch.cuda.current_stream(self.buf.device).cuda_stream)
-        _lib.check(rc, "gefen_newton_schulz_apply")
+            stream = torch.cuda.current_stream(self.buf.device).cuda_stream
+            for i in range(0, len(self.idx), self.chunk):
+                part = tasks[i:i + self.chunk]
+                rc = _lib.load().gefen_newton_schulz_apply(
+                    self.buf[i].data_ptr(), len(part), self.rows, self.cols, a, b, c, self.steps, float(self.eps),
+                    sumsq.data_ptr(), self.index.data_ptr() + 4 * i, self.work.data_ptr(), part.ctypes.data, stream)
+                _lib.check(rc, "gefen_newton_schulz_apply")
 
 
 class _MuonPlan:

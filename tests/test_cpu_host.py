@@ -449,3 +449,28 @@ def test_step_entry_calls_hooks_and_profiler_range_as_torch_does():
         entry.step()
     assert "Optimizer.step#Entry.step" in [e.name for e in prof.events()]
     assert entry.code_calls == 2
+
+
+@pytest.mark.parametrize("batch,rows,cols", [(1, 1, 30000), (448, 8, 4096), (224, 4096, 16), (64, 14336, 8), (28, 648, 1728),
+                                             (70000, 1, 129), (200, 2000, 6000), (3, 129, 130)])
+def test_padded_stacks_run_through_a_bounded_workspace(batch, rows, cols):
+    from gefen_amd import _lib
+    from gefen_amd import newton_schulz as ns
+
+    size = _lib.load().gefen_newton_schulz_workspace_size
+    chunk, nbytes = ns.padded_chunk(batch, rows, cols)
+    assert 1 <= chunk <= min(batch, 65535)
+    assert nbytes >= int(size(chunk, rows, cols))
+    last = batch % chunk
+    assert not last or nbytes >= int(size(last, rows, cols))
+    m, n = min(rows, cols), max(rows, cols)
+    assert chunk == 1 or nbytes <= max(256 << 20, 4 * 4 * batch * m * (m + n))
+    if rows * cols < 1 << 20:  # whatever the padding that a stack's number of matrices leads to
+        for count in range(1, 700):
+            chunk, nbytes = ns.padded_chunk(count, rows, cols)
+            sizes = {min(chunk, count - i) for i in range(0, count, chunk)}
+            assert nbytes >= max(int(size(k, rows, cols)) for k in sizes)
+    chunk, _ = ns.padded_chunk(batch, rows, cols)
+    # stacks of little padding, and small ones, run in one call
+    if (batch, rows, cols) in ((28, 648, 1728), (200, 2000, 6000), (3, 129, 130)):
+        assert chunk == batch

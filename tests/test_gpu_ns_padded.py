@@ -99,3 +99,41 @@ def test_padded_call_refuses_what_it_cannot_take():
     assert call() == 1
     t[0]["transposed"], t[0]["numel"] = 0, 5
     assert call() == 1
+
+
+def _low_rank_run(bound, monkeypatch):
+    """Two steps of GefenMuon on 64 matrices of 8 x 14336 (29 MB; 256 times their
+    elements where the three products of all of them are padded at once) and 3 of 30 x 9000; parameters
+    and the device memory that the optimizer holds."""
+    from gefen_amd import GefenMuon, newton_schulz
+
+    if bound is not None:
+        monkeypatch.setattr(newton_schulz, "_PADDED_WORKSPACE", bound)
+        monkeypatch.setattr(newton_schulz, "_PADDED_MAX_WASTE", 0)
+    gen = torch.Generator(device="cuda:0").manual_seed(4)
+    shapes = [(8, 14336)] * 64 + [(30, 9000)] * 3
+    ps = [torch.nn.Parameter(torch.randn(s, generator=gen, device="cuda:0") * 0.02) for s in shapes]
+    for p in ps:
+        p.grad = torch.randn(p.shape, generator=gen, device="cuda:0") * 1e-3
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    opt = GefenMuon([("p{}".format(i), p) for i, p in enumerate(ps)], lr=0.02)
+    for _ in range(2):
+        opt.step()
+    torch.cuda.synchronize()
+    held, peak = torch.cuda.memory_allocated() - before, torch.cuda.max_memory_allocated() - before
+    return [p.detach().clone() for p in ps], held, peak
+
+
+def test_padded_workspace_is_bounded():
+    """Matrices that padding would grow many times over run through one bounded
+    workspace, and the bound does not change a bit of the result."""
+    with pytest.MonkeyPatch.context() as patch:
+        want, held, peak = _low_rank_run(None, patch)
+    assert peak < (256 << 20) + 6 * 30e6, (held, peak)
+    with pytest.MonkeyPatch.context() as patch:
+        got, held, _ = _low_rank_run(20 << 20, patch)
+    assert held < (20 << 20) + 4 * 30e6, held
+    for a, b in zip(want, got):
+        assert torch.equal(a, b)
