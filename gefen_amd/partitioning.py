@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import functools
 import math
-from typing import List, Optional, Sequence, Tuple
+from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
@@ -112,10 +112,10 @@ def _finalize_period_results(list_periods_and_scores: Sequence[Tuple[int, float]
 
 
 class PeriodScorer:
-    """Scores the candidate divisors of many gradients with one host sync.
+    """Scores the candidate divisors of many gradients with one host sync per device.
 
-    add() takes one flat gradient; finish() scores them all in one library call,
-    copies the scores to the host once and returns the chosen period of each."""
+    add() takes one flat gradient; finish() scores those of a device in one library
+    call, copies their scores to the host once and returns the chosen period of each."""
 
     def __init__(self, mode: int = 1, epsilon: float = 1e-12, min_num_blocks: int = DMNB):
         self.mode = mode
@@ -135,8 +135,14 @@ class PeriodScorer:
         work = [(i, f.detach().reshape(-1).contiguous(), d) for i, (f, d, _) in enumerate(self.items) if d]
         results: List[Optional[int]] = [None if d else 1 for (_, d, _) in self.items]
         if work:
-            scores = period_scores_tasks([(f, d) for _, f, d in work], self.mode, self.epsilon)
-            for (i, f, d), s in zip(work, scores):
+            devices: Dict[torch.device, List[int]] = {}
+            for k, (_, f, _) in enumerate(work):
+                devices.setdefault(f.device, []).append(k)
+            scores = {}
+            for ks in devices.values():
+                scores.update(zip(ks, period_scores_tasks([work[k][1:] for k in ks], self.mode, self.epsilon)))
+            for k, (i, f, d) in enumerate(work):
+                s = scores[k]
                 if s[-1] > 0:
                     raise ValueError("Expected values plus epsilon to be positive before log transform.")
                 results[i] = _finalize_period_results(list(zip(d, s)), self.items[i][2], f.numel(), 0.25)

@@ -474,3 +474,27 @@ def test_padded_stacks_run_through_a_bounded_workspace(batch, rows, cols):
     # stacks of little padding, and small ones, run in one call
     if (batch, rows, cols) in ((28, 648, 1728), (200, 2000, 6000), (3, 129, 130)):
         assert chunk == batch
+
+
+def test_period_scorer_scores_each_device_s_gradients_there(monkeypatch):
+    """Gradients on several devices: one library call per device, the periods in the
+    order of add()."""
+    from gefen_amd import partitioning
+    from gefen_amd.kernels import period_variance
+
+    calls = []
+
+    def scores(items, mode, epsilon):
+        devs = {v.device for v, _ in items}
+        if len(devs) != 1:
+            raise ValueError("Expected contiguous tensors on one device.")
+        calls.append((devs.pop().type, [v.numel() for v, _ in items]))
+        # a peak at the divisor 12 of the 96-element gradients, at 16 of the others
+        return [[2.0 if p == (12 if v.numel() == 96 else 16) else 1.0 for p in divs] + [0.0] for v, divs in items]
+
+    monkeypatch.setattr(period_variance, "period_scores_tasks", scores)
+    scorer = partitioning.PeriodScorer()
+    for n, dev in ((96, "meta"), (128, "cpu"), (1, "cpu"), (128, "meta"), (96, "cpu")):
+        scorer.add(torch.empty(n, device=dev))
+    assert scorer.finish() == [12, 16, 1, 16, 12]
+    assert sorted(calls) == [("cpu", [128, 96]), ("meta", [96, 128])]
