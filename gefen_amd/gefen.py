@@ -210,7 +210,7 @@ def learn_gefen_exact_codebook_from_grad_periods(*, grad_periods, codebook_devic
     for _, flat, period, _ in grad_periods:
         if flat.device.type != "cuda":
             raise ValueError("gefen_amd learns the codebook from HIP device gradients, got {}".format(flat.device))
-        items.append((flat if not items else flat.to(items[0][0].device), period))
+        items.append((flat, period))
         total += flat.numel()
     if total == 0:
         return None

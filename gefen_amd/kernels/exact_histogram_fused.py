@@ -41,25 +41,36 @@ def gefen_exact_histogram_cuda(grad_flat: torch.Tensor, period: int, bin_counts:
     check(rc, "gefen_exact_histogram_cuda")
 
 
+# Gradients of one library call: their own counts take 32 KB each at 4096 bins, 16 MB
+# together.  A call of 512 is several launches of hundreds of workgroups anyway.
+_CALL_GRADIENTS = 512
+
+
 def accumulate_histograms(items, acc: torch.Tensor) -> None:
     """acc (float32, one entry per bin) += float32(histogram) of each (flat gradient,
-    period) of items in order (gefen.py:331-366), in a few launches; the gradients are
-    on acc's device."""
+    period) of items in order (gefen.py:331-366), in a few launches; gradients on
+    another device are moved to acc's."""
     lib = load_extension()
-    tasks = np.zeros(len(items), dtype=_lib.HISTOGRAM_TASK)
-    keep = []
-    for t, (flat, period) in zip(tasks, items):
-        if flat.dim() != 1:
-            raise ValueError("Expected grad_flat to be 1D, got dim={}".format(flat.dim()))
-        if period <= 0:
-            raise ValueError("Expected period to be positive, got {}".format(period))
-        if flat.numel() % period != 0:
-            raise ValueError("Expected grad_flat.numel()={} to be divisible by period={}.".format(flat.numel(), period))
-        g = flat.contiguous()
-        keep.append(g)
-        t["grad"], t["numel"], t["period"], t["dtype"] = g.data_ptr(), g.numel(), int(period), dtype_code(g.dtype)
-    counts = torch.empty(len(items) * acc.numel(), dtype=torch.int64, device=acc.device)
-    with device_guard(acc):
-        rc = lib.gefen_exact_histogram_tasks(tasks.ctypes.data, len(tasks), acc.data_ptr(), acc.numel(),
-                                             counts.data_ptr(), stream_of(acc))
-    check(rc, "gefen_exact_histogram_tasks")
+    dev = acc.device
+    counts = torch.empty(min(len(items), _CALL_GRADIENTS) * acc.numel(), dtype=torch.int64, device=dev)
+    for first in range(0, len(items), _CALL_GRADIENTS):
+        part = items[first:first + _CALL_GRADIENTS]
+        tasks = np.zeros(len(part), dtype=_lib.HISTOGRAM_TASK)
+        keep = []
+        for t, (flat, period) in zip(tasks, part):
+            if flat.device != dev:
+                flat = flat.to(dev)
+            if flat.dim() != 1:
+                raise ValueError("Expected grad_flat to be 1D, got dim={}".format(flat.dim()))
+            if period <= 0:
+                raise ValueError("Expected period to be positive, got {}".format(period))
+            if flat.numel() % period != 0:
+                raise ValueError("Expected grad_flat.numel()={} to be divisible by period={}.".format(flat.numel(),
+                                                                                                    period))
+            g = flat.contiguous()
+            keep.append(g)
+            t["grad"], t["numel"], t["period"], t["dtype"] = g.data_ptr(), g.numel(), int(period), dtype_code(g.dtype)
+        with device_guard(acc):
+            rc = lib.gefen_exact_histogram_tasks(tasks.ctypes.data, len(tasks), acc.data_ptr(), acc.numel(),
+                                                 counts.data_ptr(), stream_of(acc))
+        check(rc, "gefen_exact_histogram_tasks")

@@ -498,3 +498,38 @@ def test_period_scorer_scores_each_device_s_gradients_there(monkeypatch):
         scorer.add(torch.empty(n, device=dev))
     assert scorer.finish() == [12, 16, 1, 16, 12]
     assert sorted(calls) == [("cpu", [128, 96]), ("meta", [96, 128])]
+
+
+def test_histograms_of_gradients_elsewhere_are_formed_on_the_sum_s_device(monkeypatch):
+    """accumulate_histograms moves a gradient of another device over, and hands the
+    library tensors of the sum's device alone."""
+    import contextlib
+    import ctypes
+
+    from gefen_amd import _lib
+    from gefen_amd.kernels import exact_histogram_fused as fused
+
+    class Elsewhere:  # a gradient on a device that this machine does not have
+        device = "hip:1"
+
+        def __init__(self, tensor):
+            self.tensor = tensor
+
+        def to(self, device):
+            assert device == torch.device("cpu")
+            return self.tensor
+
+    seen = []
+
+    class Library:
+        def gefen_exact_histogram_tasks(self, tasks, ntasks, acc, bins, counts, stream):
+            rows = (ctypes.c_char * (ntasks * _lib.HISTOGRAM_TASK.itemsize)).from_address(tasks)
+            seen.append([int(t["grad"]) for t in np.frombuffer(rows, dtype=_lib.HISTOGRAM_TASK)])
+            return 0
+
+    monkeypatch.setattr(fused, "load_extension", Library)
+    monkeypatch.setattr(fused, "device_guard", lambda t: contextlib.nullcontext())
+    monkeypatch.setattr(fused, "stream_of", lambda t: 0)
+    here = [torch.zeros(8) for _ in range(3)]
+    fused.accumulate_histograms([(here[0], 4), (Elsewhere(here[1]), 2), (here[2], 8)], torch.zeros(16))
+    assert seen == [[t.data_ptr() for t in here]]

@@ -84,3 +84,22 @@ def test_many_tensors_sum_in_order():
         want = want + _ref(v, 48 + (i % 3) * 200, "f32", 4096).astype(np.float32)
     accumulate_histograms(items, acc)
     np.testing.assert_array_equal(acc.cpu().numpy(), want)
+
+
+def test_counts_of_many_tensors_stay_small():
+    """The tensors' own counts (32 KB each) are formed a bounded number of tensors at a time."""
+    from gefen_amd.kernels.exact_histogram_fused import accumulate_histograms
+
+    v = torch.randn(3000 * 64, generator=torch.Generator().manual_seed(5)).cuda()
+    items = [(v[i * 64:(i + 1) * 64], 16) for i in range(3000)]
+    acc = torch.zeros(4096, dtype=torch.float32, device="cuda:0")
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    accumulate_histograms(items, acc)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - before <= 40 << 20
+    want = np.zeros(4096, dtype=np.float32)
+    for i in range(3000):
+        want += _ref(v[i * 64:(i + 1) * 64], 16, "f32", 4096).astype(np.float32)
+    np.testing.assert_array_equal(acc.cpu().numpy(), want)
