@@ -43,6 +43,8 @@ SIGNATURES = {
     "gefen_step_tasks_noalloc": (I32, [P, I32, P, P]),
     "gefen_step_plan_create": (I32, [P, I32, P, P]),
     "gefen_step_plan_run": (I32, [P, P, I32, P]),
+    "gefen_step_plan_kept_runs": (I64, [P]),
+    "gefen_step_tasks_summary": (I32, [P, I32, P]),
     "gefen_step_plan_time_runs": (I32, [P, I32]),
     "gefen_step_plan_last_ms": (I32, [P, P]),
     "gefen_step_plan_destroy": (None, [P]),
@@ -69,6 +71,7 @@ SIGNATURES = {
     "gefen_lloyd_accumulate": (I32, [P, I32, I64, I64, P, I32, P, P, P]),
     "gefen_lloyd_mse": (I32, [P, I32, I64, I64, P, P, I32, P, P, P]),
     "gefen_gemm_bf16": (I32, [P, I64, P, I64, I32, P, I64, P, I64, I32, I32, I32, DBL, DBL, P]),
+    "gefen_gemm_bf16_nt_batched_tile": (I32, [I32, I32, I32, I32, I32]),
     "gefen_gemm_bf16_nt_batched": (I32, [P, I64, I64, P, I64, I64, P, I64, I64, P, I64, I64, P, I64, I64, I32, I32,
                                          I32, I32, I32, DBL, DBL, I32, P]),
     "gefen_gram_bf16_batched": (I32, [P, I64, I64, P, I64, I64, I32, I32, I32, DBL, P]),
@@ -100,6 +103,7 @@ PERIOD_TASK = np.dtype([
 HISTOGRAM_TASK = np.dtype([
     ("grad", np.uint64), ("numel", np.int64), ("period", np.int64), ("dtype", np.int32), ("pad", np.int32),
 ])
+STEP_SUMMARY = np.dtype([("launches", np.int32), ("shared", np.int32), ("small", np.int32), ("tables", np.int32)])
 assert PERIOD_TASK.itemsize == 40 and HISTOGRAM_TASK.itemsize == 32
 assert STEP_TASK.itemsize == 128 and MUON_TASK.itemsize == 72 and MUON_APPLY_TASK.itemsize == 56
 

@@ -855,6 +855,12 @@ extern "C" int gefen_gemm_bf16_nt_batched(const void* a, int64_t lda, int64_t st
     return ns::launch_product(g, batch, false, reinterpret_cast<hipStream_t>(stream), "gefen_gemm_bf16_nt_batched");
 }
 
+extern "C" int gefen_gemm_bf16_nt_batched_tile(int batch, int m, int n, int k, int symmetric) {
+    bool small;
+    ns::product_us(m, n, k, symmetric != 0, batch, &small);
+    return small ? ns::Small::T : ns::Big::T;
+}
+
 extern "C" int gefen_gram_bf16_batched(const void* xt, int64_t ldxt, int64_t stride_xt, void* c, int64_t ldc,
                                        int64_t stride_c, int batch, int m, int k, double alpha,
                                        gefen_stream_t stream) {

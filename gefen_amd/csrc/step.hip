@@ -733,10 +733,8 @@ int check_codebook(const float* cb, int K) {
     return GEFEN_OK;
 }
 
-// gefen_step_tasks: check and plan every row, then run them with the pooled
-// stepsize tables.
-int step_tasks_general(const gefen_step_task* tasks, int ntasks, const CodebookTables* tables, hipStream_t st) {
-    std::vector<PendingStep> pend;
+// Check and plan every row of a call.
+int pending_steps(const gefen_step_task* tasks, int ntasks, std::vector<PendingStep>& pend) {
     pend.reserve(ntasks);
     for (int i = 0; i < ntasks; ++i) {
         int rc = check_step_task(tasks[i]);
@@ -747,6 +745,14 @@ int step_tasks_general(const gefen_step_task* tasks, int ntasks, const CodebookT
         if (rc) return rc;
         pend.push_back(ps);
     }
+    return GEFEN_OK;
+}
+
+// gefen_step_tasks: plan every row, then run them with the pooled stepsize tables.
+int step_tasks_general(const gefen_step_task* tasks, int ntasks, const CodebookTables* tables, hipStream_t st) {
+    std::vector<PendingStep> pend;
+    const int rc = pending_steps(tasks, ntasks, pend);
+    if (rc) return rc;
     mark_mixed(pend);
     return run_steps_pooled(pend, tables, st);
 }
@@ -846,6 +852,7 @@ struct gefen_step_plan {
     LutPlan lp;                          // stepsize tables of the current run
     std::vector<int> launch_key;         // stepsize-table key of each launch in the current run
     SideStream* side = nullptr;
+    int64_t kept_runs = 0;
     bool timing = false, timed = false;
     hipEvent_t t0 = nullptr, t1 = nullptr;
 };
@@ -861,8 +868,6 @@ bool same_tensors(const gefen_step_task& a, const gefen_step_task& b) {
            a.state_dtype == b.state_dtype;
 }
 
-// The plan's fast path: a GEFEN_* status, or -1 when the rows do not fit the
-// plan (then nothing was launched).
 // The hyperparameters and bias corrections of a task row, as compared between rows.
 bool same_scalars(const gefen_step_task& a, const gefen_step_task& b) {
     return a.beta1 == b.beta1 && a.beta2 == b.beta2 && a.lr == b.lr && a.eps == b.eps &&
@@ -870,6 +875,20 @@ bool same_scalars(const gefen_step_task& a, const gefen_step_task& b) {
            a.bias_correction_2 == b.bias_correction_2;
 }
 
+// The launches of the pending tasks as gefen_step_tasks would make them, before any
+// stepsize table has an address: the tables' keys stand in for it.
+void group_planned(std::vector<PendingStep>& pend, LutPlan& lp, const CodebookTables* tables,
+                   std::vector<StepLaunch>& launches, std::vector<int>& slot) {
+    mark_mixed(pend);
+    plan_luts(pend, lp);
+    for (size_t i = 0; i < pend.size(); ++i)
+        pend[i].task.lut = lp.which[i] >= 0 ? reinterpret_cast<const float*>((uintptr_t)(lp.which[i] + 1) * 256) : nullptr;
+    group_launches(pend, tables, launches, &slot);
+    for (PendingStep& ps : pend) ps.task.lut = nullptr;
+}
+
+// The plan's fast path: a GEFEN_* status, or -1 when the rows do not fit the
+// plan (then nothing was launched).
 int plan_run_fast(gefen_step_plan& P, const gefen_step_task* tasks, hipStream_t st) {
     // rows of one group share their scalars: the float forms are computed once per run of equal rows
     const gefen_step_task* prev = nullptr;
@@ -1017,14 +1036,7 @@ extern "C" int gefen_step_plan_create(const gefen_step_task* tasks, int ntasks, 
             return rc;
         }
     }
-    // group as gefen_step_tasks would, with the creation rows' stepsize-table keys
-    mark_mixed(P->pend);
-    plan_luts(P->pend, P->lp);
-    for (size_t i = 0; i < P->pend.size(); ++i)
-        P->pend[i].task.lut = P->lp.which[i] >= 0 ? reinterpret_cast<const float*>((uintptr_t)(P->lp.which[i] + 1) * 256)
-                                                  : nullptr;
-    group_launches(P->pend, P->tables, P->launches, &P->slot);
-    for (PendingStep& ps : P->pend) ps.task.lut = nullptr;
+    group_planned(P->pend, P->lp, P->tables, P->launches, P->slot);
     P->side = side_stream_of(dev);
     *out = P;
     return GEFEN_OK;
@@ -1041,6 +1053,7 @@ extern "C" int gefen_step_plan_run(gefen_step_plan* plan, const gefen_step_task*
     if (ntasks == plan->ntasks && dev == plan->dev) {
         DeviceScope scope(dev);
         rc = plan_run_fast(*plan, tasks, st);
+        if (rc == GEFEN_OK) ++plan->kept_runs;
         if (rc != -1) return rc;
     }
     DeviceScope scope(dev);
@@ -1053,6 +1066,28 @@ extern "C" int gefen_step_plan_run(gefen_step_plan* plan, const gefen_step_task*
         plan->timed = e == hipSuccess;
     }
     return rc;
+}
+
+extern "C" int64_t gefen_step_plan_kept_runs(const gefen_step_plan* plan) { return plan ? plan->kept_runs : -1; }
+
+extern "C" int gefen_step_tasks_summary(const gefen_step_task* tasks, int ntasks, gefen_step_summary* out) {
+    if (!out) return fail_inval("null summary pointer");
+    if (ntasks < 0 || (ntasks > 0 && !tasks)) return fail_inval("invalid task array");
+    std::vector<PendingStep> pend;
+    int rc = pending_steps(tasks, ntasks, pend);
+    if (rc) return rc;
+    LutPlan lp;
+    std::vector<StepLaunch> launches;
+    std::vector<int> slot;
+    group_planned(pend, lp, nullptr, launches, slot);
+    memset(out, 0, sizeof(*out));
+    out->launches = (int32_t)launches.size();
+    out->tables = (int32_t)lp.keys.size();
+    for (const StepLaunch& L : launches) {
+        out->shared += L.key.mixed;
+        out->small += L.elems < kSmallLaunchElems;
+    }
+    return GEFEN_OK;
 }
 
 extern "C" int gefen_step_plan_time_runs(gefen_step_plan* plan, int enable) {

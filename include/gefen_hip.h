@@ -153,6 +153,14 @@ int gefen_step_tasks(const gefen_step_task* tasks, int ntasks, const void* table
 int gefen_step_tasks_noalloc(const gefen_step_task* tasks, int ntasks, const void* tables,
                              gefen_stream_t stream);
 
+/* How gefen_step_tasks would run this call (a diagnostic; nothing is launched): its
+ * launches, those that hold tensors of several row forms, those of small tensors (which
+ * take the second stream where the call has others too), and its stepsize tables. */
+typedef struct gefen_step_summary {
+    int32_t launches, shared, small, tables;
+} gefen_step_summary;
+int gefen_step_tasks_summary(const gefen_step_task* tasks, int ntasks, gefen_step_summary* out);
+
 /* A prepared step: gefen_step_tasks for a task table whose tensors stay the
  * same from step to step (the optimizer's cached plan).  No single counterpart
  * in the reference: it replaces the per-parameter loop of Gefen.step
@@ -169,6 +177,7 @@ int gefen_step_tasks_noalloc(const gefen_step_task* tasks, int ntasks, const voi
  * gradients lose the alignment their kernels were chosen for, or a stream of
  * another device takes the gefen_step_tasks path.  One plan must not be run
  * from two threads at once.
+ * gefen_step_plan_kept_runs: how many runs used the kept launches (a diagnostic).
  * gefen_step_plan_time_runs: enable != 0 makes each later run record two
  * timing events on its stream, right before its first launch and after its
  * last; gefen_step_plan_last_ms waits for the last timed run to finish and
@@ -176,6 +185,7 @@ int gefen_step_tasks_noalloc(const gefen_step_task* tasks, int ntasks, const voi
 typedef struct gefen_step_plan gefen_step_plan;
 int gefen_step_plan_create(const gefen_step_task* tasks, int ntasks, const void* tables, gefen_step_plan** plan);
 int gefen_step_plan_run(gefen_step_plan* plan, const gefen_step_task* tasks, int ntasks, gefen_stream_t stream);
+int64_t gefen_step_plan_kept_runs(const gefen_step_plan* plan);
 int gefen_step_plan_time_runs(gefen_step_plan* plan, int enable);
 int gefen_step_plan_last_ms(gefen_step_plan* plan, float* ms);
 void gefen_step_plan_destroy(gefen_step_plan* plan);
@@ -270,6 +280,10 @@ int gefen_gemm_bf16_nt_batched_apply(const void* a, int64_t lda, int64_t stride_
                                      int64_t stride_b, const void* d_t, int64_t ldd, int64_t stride_d, int batch,
                                      int m, int n, int k, double alpha, double beta,
                                      const gefen_muon_apply_task* tasks, gefen_stream_t stream);
+
+/* Side (128 or 256) of the output tiles that a batched product of this size takes (a
+ * diagnostic; symmetric as in gefen_gemm_bf16_nt_batched, 1 for the Gram product). */
+int gefen_gemm_bf16_nt_batched_tile(int batch, int m, int n, int k, int symmetric);
 
 /* Newton-Schulz of a stack and GefenMuon's update of its parameters in one call,
  * for matrices of any size (gefen_muon.py:16-51, 325-329): x holds `batch` bf16
