@@ -296,17 +296,25 @@ def test_many_tasks_in_one_call():
         np.testing.assert_array_equal(gu.to_np(d["mag"]), o["mag"])
 
 
-def test_small_launches_on_the_side_stream_match_the_oracle():
+# Groups of 4M elements keep launches of their own; two or more smaller ones of a dtype
+# pair share one.  The first call has small launches of single groups, one of them
+# reading the large launch's stepsize table; the second a small shared one.
+@pytest.mark.parametrize("specs,summary", [
+    ([("bf16", 2048 * 2100, 2048), ("bf16", 256 * 16800, 1), ("bf16", 250 * 64, 1), ("f32", 96 * 8, 96),
+      ("f32", 1024 * 4100, 1024)], {"launches": 5, "shared": 0, "small": 2, "tables": 1}),
+    ([("bf16", 2048 * 2100, 2048), ("bf16", 256 * 16800, 1), ("bf16", 250 * 64, 1), ("bf16", 768 * 5, 768),
+      ("f32", 96 * 8, 96), ("bf16", 2304, 18), ("f32", 1024 * 1100, 1024)],
+     {"launches": 4, "shared": 2, "small": 1, "tables": 1}),
+])
+def test_small_launches_on_the_side_stream_match_the_oracle(specs, summary):
     """A call mixing large launches (at least 2^20 elements) with small ones: the
     small launches run on the library's second stream, forked from and joined back
     to the caller's stream.  Every tensor matches the oracle, including period-one
-    tensors on both streams (each reading the shared stepsize table) and a read of
-    the results right after the call on the caller's stream."""
+    tensors on both streams (each reading the shared stepsize table, or in a shared
+    launch) and a read of the results right after the call on the caller's stream."""
     cb = _codebook()
     cb_dev = torch.from_numpy(cb).to("cuda:0")
     tables = _tables(cb_dev)
-    specs = [("bf16", 2048 * 600, 2048), ("bf16", 256 * 4200, 1), ("bf16", 256 * 12, 1), ("bf16", 768 * 5, 768),
-             ("f32", 96 * 8, 96), ("bf16", 2304, 18), ("f32", 1024 * 1100, 1024)]
     tasks = np.zeros(len(specs), dtype=_lib.STEP_TASK)
     devs, oracle = [], []
     for i, (dt, n, period) in enumerate(specs):
@@ -328,6 +336,9 @@ def test_small_launches_on_the_side_stream_match_the_oracle():
         t["param_dtype"] = t["state_dtype"] = gu.CODE[dt]
         t["beta1"], t["beta2"], t["lr"], t["eps"] = 0.9, 0.999, 1e-3, 1e-8
         t["bias_correction_1"], t["bias_correction_2"] = 0.1, 1 - 0.999
+    out = np.zeros(1, dtype=_lib.STEP_SUMMARY)
+    _lib.check(_lib.load().gefen_step_tasks_summary(tasks.ctypes.data, len(specs), out.ctypes.data))
+    assert {key: int(out[0][key]) for key in out.dtype.names} == summary
     _lib.check(_lib.load().gefen_step_tasks(tasks.ctypes.data, len(specs), tables.data_ptr(), gu.stream()))
     # read on the caller's stream without a device-wide synchronisation first
     got = [{k: d[k].clone() for k in ("p", "idx", "mag", "v")} for d in devs]

@@ -22,10 +22,11 @@ pytestmark = pytest.mark.gpu
 DT = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
 
 # (dtype, numel, period): period-one bf16 and f16 states (stepsize tables), block
-# rows of several kernel shapes, a long row (two-sweep kernel), fp32, and enough
-# small tensors of one shape that the plan has several launches of one key, some
-# on the side stream beside the large ones
-SPECS = ([("bf16", 1 << 21, 1), ("bf16", 96 * 2048, 2048), ("f32", 48 * 768, 768), ("f16", 3 * 4096, 1),
+# rows of several kernel shapes, fp32, and enough small tensors of the first one's
+# shape that the plan has two launches of that key (of 4M elements together: fewer
+# would join the shared launch, which reads no tables), the others in shared launches,
+# some of them on the side stream
+SPECS = ([("bf16", 1 << 22, 1), ("bf16", 96 * 2048, 2048), ("f32", 48 * 768, 768), ("f16", 3 * 4096, 1),
           ("bf16", 5000 * 6, 5000), ("f32", 4096, 1), ("bf16", 64 * 300, 64)]
          + [("bf16", 2048, 1)] * 34 + [("f32", 768, 768)] * 3)
 
@@ -120,6 +121,8 @@ def test_step_plan_runs_equal_step_tasks():
                 n, what = n - 3, "a shorter table"
             print("step", step, what, flush=True)
             _lib.check(lib.gefen_step_plan_run(plan, ta.ctypes.data, n, gu.stream()), "gefen_step_plan_run")
+            # steps 1, 2 and 4 use the kept launches; from step 6 on a row names another tensor
+            assert lib.gefen_step_plan_kept_runs(plan) == {1: 1, 2: 2, 3: 2}.get(step, 3), (step, what)
             ms = ctypes.c_float()
             _lib.check(lib.gefen_step_plan_last_ms(plan, ctypes.byref(ms)))
             assert ms.value > 0.0

@@ -139,18 +139,27 @@ def test_unaligned_tensors_step_as_aligned_ones(dt):
             t["bias_correction_1"], t["bias_correction_2"] = 1 - 0.9 ** 3, 1 - 0.999 ** 3
         return rows, tasks
 
-    (ra, ta), (rb, tb), (rc, tc) = build(0), build(1), build(1)
+    # aligned and shifted tensors one per call (their own kernels), and the shifted ones
+    # together, in a shared launch and in a plan of it
+    (ra, ta), (rb, tb), (rc, tc), (rd, td) = build(0), build(1), build(1), build(1)
+    out = np.zeros(1, dtype=_lib.STEP_SUMMARY)
+    for tasks, shared in [(t[i:i + 1], 0) for t in (ta, tb) for i in range(len(t))] + [(tc, 1)]:
+        _lib.check(lib.gefen_step_tasks_summary(tasks.ctypes.data, len(tasks), out.ctypes.data))
+        assert (out[0]["launches"], out[0]["shared"]) == (1, shared)
     plan = ctypes.c_void_p()
     _lib.check(lib.gefen_step_plan_create(tc.ctypes.data, len(tc), tables.data_ptr(), ctypes.byref(plan)))
     for _ in range(2):
-        _lib.check(lib.gefen_step_tasks(ta.ctypes.data, len(ta), tables.data_ptr(), gu.stream()))
-        _lib.check(lib.gefen_step_tasks(tb.ctypes.data, len(tb), tables.data_ptr(), gu.stream()))
+        for t in (ta, tb):
+            for i in range(len(t)):
+                _lib.check(lib.gefen_step_tasks(t[i:i + 1].ctypes.data, 1, tables.data_ptr(), gu.stream()))
         _lib.check(lib.gefen_step_plan_run(plan, tc.ctypes.data, len(tc), gu.stream()))
+        _lib.check(lib.gefen_step_tasks(td.ctypes.data, len(td), tables.data_ptr(), gu.stream()))
     torch.cuda.synchronize()
     lib.gefen_step_plan_destroy(plan)
-    for i, (a, b, c) in enumerate(zip(ra, rb, rc)):
-        for key, x, y, z in zip(("p", "g", "idx", "mag", "vmean"), a, b, c):
+    for i, (a, b, c, d) in enumerate(zip(ra, rb, rc, rd)):
+        for key, x, y, z, w in zip(("p", "g", "idx", "mag", "vmean"), a, b, c, d):
             assert torch.equal(x[0].view(torch.uint8), y[0].contiguous().view(torch.uint8)), (shapes[i], key)
             assert torch.equal(x[0].view(torch.uint8), z[0].contiguous().view(torch.uint8)), (shapes[i], key)
+            assert torch.equal(x[0].view(torch.uint8), w[0].contiguous().view(torch.uint8)), (shapes[i], key)
             shift = y[0].storage_offset()
             assert not y[1][:shift].any() and not y[1][shift + y[0].numel():].any(), (shapes[i], key)  # nothing beside it

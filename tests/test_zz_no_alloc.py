@@ -76,13 +76,37 @@ def _run(entry, specs, steps):
     return [gu.to_np(p) for p in ps], [{k: gu.to_np(v) for k, v in st.items()} for st in states]
 
 
+def _table_count(specs):
+    """Stepsize tables of a step of these tensors (from the host, whatever their addresses)."""
+    fake = torch.empty(1, dtype=torch.uint8)
+    ones = [fake.data_ptr() // 256 * 256] * len(specs)
+
+    class At:
+        def __init__(self, address):
+            self.address = address
+
+        def data_ptr(self):
+            return self.address
+
+    at = [At(a) for a in ones]
+    t = _tasks(specs, at, at, [{"idx": a, "mag": a, "vmean": a} for a in at], 1)
+    out = np.zeros(1, dtype=_lib.STEP_SUMMARY)
+    _lib.check(_lib.load().gefen_step_tasks_summary(t.ctypes.data, len(t), out.ctypes.data))
+    return int(out[0]["tables"])
+
+
 def test_noalloc_step_equals_step_tasks_on_two_calls():
-    big = [("bf16", 1 << 20, 1), ("f16", 3 * 4096, 1), ("bf16", 96 * 2048, 2048), ("f32", 48 * 768, 768),
-           ("f16", 1000, 1), ("bf16", 5 * 300, 1)]
+    # the tables of a large bf16 group and of the only small f16 group; then fewer and
+    # smaller ones; then all tensors of a dtype in shared launches, which read none
+    big = [("bf16", 1 << 22, 1), ("f16", 3 * 4096, 1), ("bf16", 96 * 2048, 2048), ("f32", 48 * 768, 768)]
     small = [("bf16", 4096, 1), ("f16", 512, 1), ("bf16", 2 * 2048, 2048)]
-    for label, shapes, steps in (("first call", big, 3), ("second, smaller call", small, 2)):
+    shared = [("bf16", 1 << 20, 1), ("f16", 3 * 4096, 1), ("bf16", 96 * 2048, 2048), ("f32", 48 * 768, 768),
+              ("f16", 1000, 1), ("bf16", 5 * 300, 1)]
+    for label, shapes, steps, tables in (("first call", big, 3, 2), ("second, smaller call", small, 2, 1),
+                                         ("shared launches", shared, 3, 0)):
         print("noalloc", label, flush=True)
-        specs = _tensor_set(11 if label == "first call" else 12, shapes)
+        specs = _tensor_set(11 + steps, shapes)
+        assert _table_count(specs) == tables
         ref_p, ref_s = _run("gefen_step_tasks", specs, steps)
         got_p, got_s = _run("gefen_step_tasks_noalloc", specs, steps)
         for i in range(len(specs)):
@@ -120,7 +144,8 @@ from gefen_amd import _lib
 lib = _lib.load()
 tables = t._tables(lib)
 before = lib.gefen_device_allocations()
-specs = t._tensor_set(14, [("bf16", 1 << 16, 1), ("f16", 4096, 1), ("bf16", 8 * 2048, 2048)])
+specs = t._tensor_set(14, [("bf16", 1 << 16, 1), ("f16", 4096, 1), ("f32", 8 * 2048, 2048)])
+assert t._table_count(specs) == 2
 ps = [t.gu.to_dev(s[4], s[0]) for s in specs]
 gs = [t.gu.to_dev(s[5], s[0]) for s in specs]
 states = [t._state(*s[:4]) for s in specs]
