@@ -5,7 +5,7 @@ times:  A = X X^T;  B = b A + c A A;  X = a X + B X.  Each product rounds
 alpha*AB + beta*D to bf16 once, as torch.addmm does.
 
 newton_schulz_batched runs a stack of same-shaped matrices at once with the
-large-tile batched GEMM, keeping only X^T between iterations: X X^T comes from
+tiled batched GEMM, keeping only X^T between iterations: X X^T comes from
 X^T through transposing LDS reads (gefen_gram_bf16_batched), b A + c A A is an
 A B^T product of the symmetric A, and B X = (X^T B)^T is written as X'^T (the
 last iteration writes the orientation it returns).  gefen_newton_schulz_apply does

@@ -80,7 +80,7 @@ def _nt_batched(a, b, out, out_t=None, d=None, alpha=1.0, beta=0.0, symmetric=Fa
     (2, 512, 512, 1024, 2.0315, -4.775, True, True),
 ])
 def test_batched_gemm_equals_one_matrix_gemm(g, m, n, k, alpha, beta, sym, dt):
-    """The batched large-tile GEMM accumulates K in the same MFMA order as the
+    """The batched tiled GEMM (128 x 128 tiles at these sizes) accumulates K in the same MFMA order as the
     one-matrix kernel: results are bit-identical, C^T is C transposed, and a
     symmetric product's mirrored tiles equal the computed ones."""
     from gefen_amd.newton_schulz import gemm

@@ -4,8 +4,8 @@ The one-matrix kernel (gefen_gemm_bf16: C = alpha A op(B) + beta D, one bf16
 rounding) over 40 random (m, n, k) from 1 to 700, both operand layouts, with
 and without D: every element within one bf16 ulp of the float64 result plus the
 float32 accumulation bound (k + 2) 2^-24 sum|terms| (half a bf16 ulp is at most
-2^-8 of the value).  The batched tile kernel over random stacks of 256-multiple
-shapes (symmetric or not, with D or D^T, with and without the transposed copy
+2^-8 of the value).  The batched tile kernel (its 128 x 128 tiles at these sizes)
+over random stacks of 256-multiple shapes (symmetric or not, with D or D^T, with and without the transposed copy
 of a non-symmetric product): bit-identical to the one-matrix kernel on every
 matrix (both use the same MFMA K order)."""
 
