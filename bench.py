@@ -205,8 +205,10 @@ def bench_kernels(args, dev):
                             nact, K, cands),
                         "note": "compute-bound in float64 on the vector ALU, not MFMA: the peak is MI355X's fp64 "
                                 "figure (78.6 TFLOP/s, vector and matrix alike); a division counts as one "
-                                "operation though the IEEE float64 quotient takes about 11 instructions; the "
-                                "operands sit in LDS, so HBM traffic is negligible",
+                                "operation though the IEEE float64 quotient takes about 11 instructions.  The "
+                                "flops are the recurrence's, every start of every end; k_dp_level leaves out those "
+                                "that a bound on the cost rules out, and its dependent launches are bound by their "
+                                "latency; the operands sit in L2, so HBM traffic is negligible",
                         "algorithmic_flops": dp_flops}}
     if not args.no_cpu_baseline:
         out["cpu_baseline"] = cpu_baseline_kernels(g.cpu().numpy(), divs)

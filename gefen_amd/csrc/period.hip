@@ -40,7 +40,10 @@ __device__ __forceinline__ double transform(T raw, int mode) {
 }
 
 // Natural logarithm of a positive, finite, normal y by an accurate table (S. Gal,
-// "Computing elementary functions", 1986): y = z 2^e with z in [0.6875, 1.375), c
+// "Computing elementary functions", 1986), arranged as the log of Arm's Optimized
+// Routines is (an interval's index from the bits below an offset that is subtracted, a
+// two-part ln 2); the entries are this file's own and the polynomial is the plain
+// series.  y = z 2^e with z in [0.6875, 1.375), c
 // the table's reciprocal of z's interval, log y = (e ln 2 - log c) + log1p(z c - 1).
 // The entries are chosen so that -log c is a multiple of 2^-42 to within 2^-64, and
 // ln 2 is split at the same bit, so the bracket is exact; the intervals beside 1
@@ -285,8 +288,9 @@ __global__ __launch_bounds__(kScoreThreads, 4) void k_score_pass(const ScorePass
 static_assert(kScoreThreads == 256 && kScoreThreads * kScorePer == kScoreChunk, "four waves, a chunk in registers");
 
 // out[j] = sum of log(x + eps) over block j of p elements, from the values: for
-// divisors that share too little with a pass (multiples of a prime above kPassMax).  A wave per block; each lane sums its strided items in order,
-// then a butterfly.  `bad`: where blocks count x + eps <= 0, or null.
+// divisors that share too little with a pass (multiples of a prime above kPassMax).
+// A wave per block; each lane sums its strided items in order, then a butterfly.
+// `bad`: where blocks count x + eps <= 0, or null.
 template <typename T>
 __global__ __launch_bounds__(256) void k_log_block_sums(const T* __restrict__ src, int64_t nblocks, int64_t p, int mode,
                                                         double eps, double* __restrict__ out, double* __restrict__ bad) {

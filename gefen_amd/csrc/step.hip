@@ -164,7 +164,7 @@ int r_bucket(int64_t nvec, int lpr_log2) {
     if (r <= 2) return 2;
     if (r <= 4) return 4;
     if (r <= 8) return 8;
-    return 0;  // two-sweep path
+    return 0;  // more than the register kernels hold
 }
 
 

@@ -11,8 +11,9 @@
 // of LPR lanes (LPR = power of two <= 64, so a wave64 holds 64/LPR rows); each
 // lane keeps up to R vectors of W elements in registers, so the row is read
 // once, reduced with xor-butterflies inside the lane group (absmax for the
-// magnitude, sum of squares for vmean) and written once.  Rows longer than
-// 64*R*W elements take a two-sweep workgroup-per-row kernel.
+// magnitude, sum of squares for vmean) and written once.  Rows of more than 256
+// vectors belong to a whole workgroup: up to 8192 elements in its registers, longer
+// ones swept twice.  GefenMuon's rows past 64*R*W elements are swept twice too.
 //
 // The arithmetic is the reference's CPU path (gefen.py:116-119, 1153-1206,
 // 1280-1281, 1326-1333; gefen_muon.py:132-171, 302-316), op by op.
@@ -54,7 +55,7 @@ namespace gefen {
 #ifndef GEFEN_STEP_WAVES
 #define GEFEN_STEP_WAVES 4
 #endif
-constexpr int kThreads = 256;  // 4 waves: two-sweep, GefenMuon and vmean kernels
+constexpr int kThreads = 256;  // 4 waves: long rows, GefenMuon and vmean kernels
 constexpr int kMuonIter = GEFEN_MUON_ITER;  // wave-units per wave in one GefenMuon workgroup
 // wave-units per wave in one step workgroup: block rows, period-one rows
 constexpr int kIterRows = GEFEN_STEP_ITER_ROWS;
