@@ -135,14 +135,18 @@ class PeriodScorer:
         work = [(i, f.detach().reshape(-1).contiguous(), d) for i, (f, d, _) in enumerate(self.items) if d]
         results: List[Optional[int]] = [None if d else 1 for (_, d, _) in self.items]
         if work:
-            devices: Dict[torch.device, List[int]] = {}
-            for k, (_, f, _) in enumerate(work):
-                devices.setdefault(f.device, []).append(k)
-            scores = {}
-            for ks in devices.values():
-                scores.update(zip(ks, period_scores_tasks([work[k][1:] for k in ks], self.mode, self.epsilon)))
-            for k, (i, f, d) in enumerate(work):
-                s = scores[k]
+            dev = work[0][1].device
+            if all(f.device == dev for _, f, _ in work):
+                scores = period_scores_tasks([(f, d) for _, f, d in work], self.mode, self.epsilon)
+            else:
+                scores = [[]] * len(work)
+                devices: Dict[torch.device, List[int]] = {}
+                for k, (_, f, _) in enumerate(work):
+                    devices.setdefault(f.device, []).append(k)
+                for ks in devices.values():
+                    for k, s in zip(ks, period_scores_tasks([work[k][1:] for k in ks], self.mode, self.epsilon)):
+                        scores[k] = s
+            for (i, f, d), s in zip(work, scores):
                 if s[-1] > 0:
                     raise ValueError("Expected values plus epsilon to be positive before log transform.")
                 results[i] = _finalize_period_results(list(zip(d, s)), self.items[i][2], f.numel(), 0.25)
